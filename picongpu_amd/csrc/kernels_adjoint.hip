@@ -291,13 +291,7 @@ __global__ __launch_bounds__(256) void kDiffPush(DiffArgs a, DiffParticles P) {
         Vec3 const b{gatherGlobalCIC(a.B[0], a.g, cx, cy, cz, pos, 0.0f, 0.5f, 0.5f),
                      gatherGlobalCIC(a.B[1], a.g, cx, cy, cz, pos, 0.5f, 0.0f, 0.5f),
                      gatherGlobalCIC(a.B[2], a.g, cx, cy, cz, pos, 0.5f, 0.5f, 0.0f)};
-        PushConsts pk;
-        for (int d = 0; d < 3; ++d) pk.cell[d] = a.cell[d];
-        pk.dt = a.dt;
-        pk.c2 = a.c2;
-        pk.rc2 = a.rc2;
-        pk.c = a.c;
-        pushBoris(e, b, mom, vel, mass, charge, pk);
+        pushBoris(e, b, mom, vel, mass, charge, weightTerms<PIC_PUSHER_BORIS>(mass, charge));
         p[0] = pos.x;
         p[1] = pos.y;
         p[2] = pos.z;

@@ -25,31 +25,52 @@ __device__ __forceinline__ int wrapIdx(int v, int n) {
 constexpr int kPushThreads = kPushThreadsPerBlock;
 constexpr int kPushWaves = kPushThreads / 64;
 
-// LDS bytes of one supercell's work: the E/B tile (or the epilogue's
-// scratch), then the int64 J tile
+// t / D for 0 <= t < N by one 24-bit multiplication; the compiler's form for
+// a general int needs the high half of a 32-bit product, a quarter-rate
+// instruction
+template <int D, int N>
+constexpr bool divSmallExact() {
+    for (int t = 0; t < N; ++t)
+        if (((t * ((65536 + D - 1) / D)) >> 16) != t / D) return false;
+    return true;
+}
+template <int D, int N>
+__device__ __forceinline__ int divSmall(int t) {
+    static_assert(divSmallExact<D, N>(), "the reciprocal is too short for this range");
+    return (int)(__umul24((unsigned)t, (65536 + D - 1) / D) >> 16);
+}
+
+// element t of a box of X x Y x Z elements (x fastest) as coordinates
+template <int X, int Y, int Z>
+__device__ __forceinline__ void boxCoords(int t, int& x, int& y, int& z) {
+    constexpr int N = ((X * Y * Z + kPushThreads - 1) / kPushThreads) * kPushThreads;
+    int const row = divSmall<X, N>(t);
+    x = t - row * X;
+    z = divSmall<Y, N>(row);
+    y = row - z * Y;
+}
+
 // A particle whose move changes its shifted cell on some axis needs the
 // general Esirkepov form (up to (SUPP+1)^2*SUPP cells per component); the rest
 // need SUPP^2*(SUPP-1). The push deposits the latter at once and queues the
 // former per wave: lane l holds queued item l in A (items 64..127 in B), and
-// a full A is deposited by all 64 lanes together. An item carries what the
-// deposit reads: the tile cell, the position after the move, the move in
-// cells (vel * dt / cell) and the charge, so the contribution is the one the
-// particle would have made in place.
-struct SlowItem {
-    int cell;  // tile cell x | y << 8 | z << 16
-    float x, y, z, dx, dy, dz, q;
-};
-
-__device__ __forceinline__ int permuteLane(int dstLane, int v) { return __builtin_amdgcn_ds_permute(dstLane << 2, v); }
-__device__ __forceinline__ float permuteLane(int dstLane, float v) {
-    return __int_as_float(__builtin_amdgcn_ds_permute(dstLane << 2, __float_as_int(v)));
+// a full A is deposited by all 64 lanes together. An item is one word: the
+// particle's slot, its tile cell and its species in the launch. The deposit
+// reads the particle's new state back (its lines were written a few
+// iterations ago) and forms its velocity and move from it, the values the
+// push formed: the unfused deposit does the same. Keeping the state in the
+// queue instead took 16 registers of every wave for the whole loop, and with
+// them the kernel spilled.
+__device__ __forceinline__ uint32_t slowItem(int slot, int cx, int cy, int cz, int species) {
+    return (uint32_t)slot | ((uint32_t)cx << 16) | ((uint32_t)cy << 20) | ((uint32_t)cz << 24) |
+           ((uint32_t)species << 28);
 }
 
 // Append the items of the lanes with `slow` set after the P queued ones
 // (wave-uniform P). Every lane of the wave calls it: the ds_permute moves
 // slow lanes to queue positions P.. and the other lanes to the free ones, a
 // permutation of the 64 lanes.
-__device__ __forceinline__ void queueSlow(bool slow, const SlowItem& mine, SlowItem& A, SlowItem& B, int& P) {
+__device__ __forceinline__ void queueSlow(bool slow, uint32_t mine, uint32_t& A, uint32_t& B, int& P) {
     unsigned long long const m = __ballot(slow);
     int const k = __popcll(m);
     if (k == 0) return;
@@ -57,49 +78,189 @@ __device__ __forceinline__ void queueSlow(bool slow, const SlowItem& mine, SlowI
     int const below = __popcll(m & laneMaskLt());
     int const dst = (P + (slow ? below : k + (lane - below))) & 63;
     int const off = (lane - P) & 63;
-    bool const toA = off < k && lane >= P;
-    bool const toB = off < k && lane < P;
-#define PIC_QUEUE_MOVE(f)                          \
-    {                                              \
-        auto const r = permuteLane(dst, mine.f);   \
-        if (toA) A.f = r;                          \
-        if (toB) B.f = r;                          \
-    }
-    PIC_QUEUE_MOVE(cell)
-    PIC_QUEUE_MOVE(x)
-    PIC_QUEUE_MOVE(y)
-    PIC_QUEUE_MOVE(z)
-    PIC_QUEUE_MOVE(dx)
-    PIC_QUEUE_MOVE(dy)
-    PIC_QUEUE_MOVE(dz)
-    PIC_QUEUE_MOVE(q)
-#undef PIC_QUEUE_MOVE
+    uint32_t const r = (uint32_t)__builtin_amdgcn_ds_permute(dst << 2, (int)mine);
+    if (off < k && lane >= P) A = r;
+    if (off < k && lane < P) B = r;
     P += k;
 }
 
+// the deposit of the queued particle `item` of supercell sc
 template <int SUPP, class TG>
-__device__ __forceinline__ void depositQueued(unsigned long long* __restrict__ sJ, const SlowItem& t,
-                                              const DepositConsts& dk) {
-    float const dp[3] = {t.dx, t.dy, t.dz};
-    Esirkepov<SUPP>::template depositGeometry<TG, true>(sJ, t.cell & 255, (t.cell >> 8) & 255, t.cell >> 16,
-                                                        Esirkepov<SUPP>::geometryDp(Vec3{t.x, t.y, t.z}, dp), t.q, dk);
+__device__ __forceinline__ void depositQueued(unsigned long long* __restrict__ sJ, const PushArgs& a, int sc,
+                                              uint32_t item, const DepositConsts& dk) {
+    static_assert(SCX + Esirkepov<SUPP>::lowerMargin < 16 && PIC_MAX_SPECIES <= 4, "fields of an item");
+    Vec3 pos{0.0f, 0.0f, 0.0f}, mom{0.0f, 0.0f, 0.0f};
+    float mass = 0.0f, charge = 0.0f;
+    int const species = (int)(item >> 28);
+    for (int s = 0; s < a.nsp; ++s) {  // uniform; a lane loads in its species' round
+        const SpeciesDev& S = a.sp[s];
+        if (species != s) continue;
+        size_t const gidx = slotBase(S, sc) + (item & 0xffffu);
+        pos = Vec3{S.pos[0][gidx], S.pos[1][gidx], S.pos[2][gidx]};
+        mom = Vec3{S.mom[0][gidx], S.mom[1][gidx], S.mom[2][gidx]};
+        float const w = S.w[gidx];
+        mass = S.mass * w;
+        charge = S.charge * w;
+    }
+    Vec3 const vel = velocityOf(mom, mass);
+    Esirkepov<SUPP>::template depositGeometry<TG, true>(sJ, (item >> 16) & 15, (item >> 20) & 15, (item >> 24) & 15,
+                                                        Esirkepov<SUPP>::geometry(pos, vel, dk), charge, dk);
 }
 
+// leavers of one species the epilogue keeps in LDS (slot and exchange code);
+// a supercell with more takes the lists in global memory
+constexpr int kLeaverListLds = 2048;
+
+// LDS bytes of one supercell's work: the E/B tile (or the epilogue's
+// scratch), then the int64 J tile
 template <int SUPP, int MODE>
 struct PushLds {
-    static constexpr int GLO = SUPP / 2;
-    static constexpr int GUP = (SUPP + 1) / 2;
-    static constexpr int GV = (SCX + GLO + GUP) * (SCY + GLO + GUP) * (SCZ + GLO + GUP);
     using TG = JTileGeom<Esirkepov<SUPP>::lowerMargin, Esirkepov<SUPP>::upperMargin>;
-    static constexpr int EB_ELEMS = MODE == 2 ? 1 : 6 * GV;
+    static constexpr int EB_ELEMS = MODE == 2 ? 1 : EBTile<SUPP>::total();
     static constexpr int J_ELEMS = MODE == 0 ? 1 : TG::total();
     static constexpr int EB_BYTES = ((EB_ELEMS * 4 + 15) / 16) * 16;
     static constexpr int EPI_BYTES =
-        (kPushMaxIters * kPushWaves + 1) * 4 + kPushWaves * kNumDirs * 4 + (int)sizeof(GroupScratch);
+        MODE == 2 ? 0
+                  : (kPushMaxIters * kPushWaves + 1) * 4 + kPushWaves * kNumDirs * 4 + (int)sizeof(GroupScratch) +
+                        kLeaverListLds * 4;
     // 16-byte multiple: the int64 J tile that follows needs 8-byte aligned LDS addresses
     static constexpr int LO_BYTES = (((EB_BYTES > EPI_BYTES ? EB_BYTES : EPI_BYTES) + 15) / 16) * 16;
     static constexpr int BYTES = LO_BYTES + J_ELEMS * 8;
 };
+
+// J += the tile's component C. A thread's J values are loaded together, then
+// added and stored; an element that adds nothing (zero, or beyond an open
+// border) loads J's first cell instead and stores nothing. inside: the tile
+// lies in the box on every axis (uniform).
+template <class TG, int C, int DLO>
+__device__ __forceinline__ void flushComponent(const PushArgs& a, const unsigned long long* sJ, int ox, int oy, int oz,
+                                               bool inside) {
+    constexpr int VOL = TG::vol(C);
+    constexpr int NU = (VOL + kPushThreads - 1) / kPushThreads;
+    float* const J = a.J[C];
+    float add[NU], old[NU];
+    size_t gi[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+        int const t = threadIdx.x + u * kPushThreads;
+        long long const acc = fixedTileValue(sJ[TG::off(C) + (t < VOL ? t : 0)]);
+        int tx, ty, tz;
+        boxCoords<TG::ext(C, 0), TG::ext(C, 1), TG::ext(C, 2)>(t, tx, ty, tz);
+        int gx = ox - DLO + tx, gy = oy - DLO + ty, gz = oz - DLO + tz;
+        bool adds = t < VOL && acc != 0;
+        if (!inside) {
+            adds = adds && !(a.g.open && outsideOpen(a.g, gx, gy, gz));
+            gx = wrapIdx(gx, a.g.nx);
+            gy = wrapIdx(gy, a.g.ny);
+            gz = wrapIdx(gz, a.g.nz);
+        }
+        size_t const at = (size_t)gx + (size_t)a.g.nx * ((size_t)gy + (size_t)a.g.ny * gz);
+        gi[u] = adds ? at : 0;
+        add[u] = adds ? (float)((double)acc * a.jinv) : 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < NU; ++u) old[u] = J[gi[u]];
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+        if (add[u] != 0.0f) J[gi[u]] = old[u] + add[u];
+}
+
+// The shift's staging of one species from its leaver bits, with the leaver
+// list in LDS (L <= kLeaverListLds entries): the records of the leavers go to
+// the outbox grouped by exchange code (ascending slot inside a code), the
+// offset table to outOff, and the supercell is compacted as stageSC does.
+// `pre`: per (iteration, wave) entry the number of leavers before it. The
+// same orders as groupLeavers and stageSC; the list never leaves the CU, so
+// a supercell waits for three memory round trips (the codes, the records,
+// the moved particles) instead of ten.
+__device__ void stageFromBits(const SpeciesDev& S, int sc, int n, int iters, uint32_t bits, int L, const uint32_t* pre,
+                              GroupScratch& g, uint32_t* sWaveCnt, uint32_t* sList) {
+    int const tid = threadIdx.x;
+    int const lane = tid & 63;
+    int const wave = tid >> 6;
+    size_t const base = slotBase(S, sc);
+    uint32_t* const off = S.outOff + (size_t)sc * kOffStride;
+    if (L == 0) {  // uniform
+        if (tid < kOffStride) off[tid] = 0u;
+        return;
+    }
+    if (tid < kNumDirs) g.cnt[tid] = 0u;
+    for (int it = 0; it < iters; ++it) {
+        bool const left = (bits >> it) & 1u;
+        unsigned long long const m = __ballot(left);
+        if (left) sList[pre[it * kPushWaves + wave] + (uint32_t)__popcll(m & laneMaskLt())] = it * kPushThreads + tid;
+    }
+    __syncthreads();
+    for (int k = tid; k < L; k += kPushThreads) {
+        uint32_t const slot = sList[k];
+        uint32_t const code = (uint32_t)S.mask[base + slot] - 1u;
+        sList[k] = slot | (code << 16);
+        atomicAdd(&g.cnt[code], 1u);
+    }
+    __syncthreads();
+    if (wave == 0) {  // offsets of the codes 1..26, [27] = L
+        uint32_t const c = lane >= 1 && lane < kNumDirs ? g.cnt[lane] : 0u;
+        uint32_t const before = waveInclusiveScan(c) - c;
+        if (lane < kNumDirs) g.run[lane] = before;
+        if (lane < kOffStride) off[lane] = before;
+    }
+    for (int c0 = 0; c0 < L; c0 += kPushThreads) {
+        int const k = c0 + tid;
+        uint32_t const e = k < L ? sList[k] : 0u;
+        int const code = (int)(e >> 16);
+        size_t const from = base + (e & 0xffffu);
+        float4 r0, r1;
+        if (code != 0) {
+            r0 = make_float4(S.pos[0][from], S.pos[1][from], S.pos[2][from], S.mom[0][from]);
+            r1 = make_float4(S.mom[1][from], S.mom[2][from], S.w[from], __int_as_float((int)S.cell[from]));
+        }
+        for (int j = tid; j < kNumDirs * kPushWaves; j += kPushThreads) sWaveCnt[j] = 0u;
+        __syncthreads();
+        int myRank = 0;
+        unsigned long long pending = __ballot(code != 0);
+        while (pending) {
+            int const leader = __ffsll((long long)pending) - 1;
+            int const kc = __shfl(code, leader);
+            unsigned long long const same = __ballot(code == kc);
+            if (code == kc) myRank = __popcll(same & laneMaskLt());
+            if (lane == 0) sWaveCnt[wave * kNumDirs + kc] = (uint32_t)__popcll(same);
+            pending &= ~same;
+        }
+        __syncthreads();
+        if (code != 0) {
+            uint32_t r = g.run[code] + (uint32_t)myRank;
+            for (int w = 0; w < wave; ++w) r += sWaveCnt[w * kNumDirs + code];
+            S.outbox[2 * (base + r)] = r0;
+            S.outbox[2 * (base + r) + 1] = r1;
+        }
+        if (c0 + kPushThreads < L) {
+            __syncthreads();
+            if (tid > 0 && tid < kNumDirs) {
+                uint32_t add = 0;
+                for (int w = 0; w < kPushWaves; ++w) add += sWaveCnt[w * kNumDirs + tid];
+                g.run[tid] += add;
+            }
+            __syncthreads();
+        }
+    }
+    __syncthreads();  // every leaver record has been read before its slot is overwritten
+    int const nn = n - L;
+    int run = 0;
+    for (int it = nn / kPushThreads; it < iters; ++it) {
+        int const i = it * kPushThreads + tid;
+        bool const stays = i >= nn && i < n && !((bits >> it) & 1u);
+        int total;
+        int const r = blockRank<kPushWaves>(stays, sWaveCnt, &total);
+        if (stays) {
+            size_t const dst = base + (sList[run + r] & 0xffffu);
+            copyParticle(S, dst, base + i);
+            S.mask[dst] = 1;
+        }
+        run += total;
+    }
+    for (int i = nn + tid; i < n; i += kPushThreads) S.mask[base + i] = 0;
+    if (tid == 0) S.count[sc] = (uint32_t)nn;
+}
 
 // The work of one supercell `sc` of the simulation described by `a`; every
 // thread of the workgroup calls it.
@@ -116,8 +277,9 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
     // path starts inside the old cell and moves less than one cell per axis
     // (the host requires float(c*dt)/cell < 1).
     constexpr int DLO = Esirkepov<SUPP>::lowerMargin;
-    using TG = JTileGeom<DLO, Esirkepov<SUPP>::upperMargin>;
-    constexpr int EB_ELEMS = MODE == 2 ? 1 : 6 * GV;
+    constexpr int UPM = Esirkepov<SUPP>::upperMargin;
+    using TG = JTileGeom<DLO, UPM>;
+    constexpr int EB_ELEMS = MODE == 2 ? 1 : EBTile<SUPP>::total();
     constexpr int J_ELEMS = MODE == 0 ? 1 : TG::total();
 
     // One LDS buffer: the E/B tile, then the J tile. After the particle loop
@@ -130,69 +292,101 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
     uint32_t* const sPre = reinterpret_cast<uint32_t*>(smem);
     uint32_t* const sWaveCnt = sPre + kPushMaxIters * kPushWaves + 1;
     GroupScratch& sGroup = *reinterpret_cast<GroupScratch*>(sWaveCnt + kPushWaves * kNumDirs);
+    uint32_t* const sList = reinterpret_cast<uint32_t*>(&sGroup + 1);
 
     if (halted(a.g)) return;  // uniform: a later step of an overflowed simulation
     int const sx = sc % a.g.nscx;
     int const sy = (sc / a.g.nscx) % a.g.nscy;
     int const sz = sc / (a.g.nscx * a.g.nscy);
     int const ox = sx * SCX, oy = sy * SCY, oz = sz * SCZ;
-    int const tid = threadIdx.x;
+    // opaque, so that a persistent workgroup's loop over supercells does not
+    // keep the staging's node offsets in registers (they spilled)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    __builtin_assume(tid >= 0 && tid < kPushThreads);
 
     int total = 0;
     for (int s = 0; s < a.nsp; ++s) total += (int)a.sp[s].count[sc];
     if (total == 0) {  // uniform across the workgroup
         if (MODE != 2 && tid < kOffStride) {
-            for (int s = 0; s < a.nsp; ++s)
-                if (a.sp[s].lists) a.sp[s].outOff[(size_t)sc * kOffStride + tid] = 0u;
+            for (int s = 0; s < a.nsp; ++s) a.sp[s].outOff[(size_t)sc * kOffStride + tid] = 0u;
         }
         if (MODE == 1 && a.tileOut)  // an empty tile for the gather flush
             for (int t = tid; t < J_ELEMS; t += blockDim.x) a.tileOut[(size_t)sc * J_ELEMS + t] = 0.0f;
         return;
     }
 
-    // the open-border checks are compiled only into the loop a box with open
-    // borders runs (the branch is uniform)
-    auto stageEB = [&](auto openBorders) {
-        for (int t = tid; t < 6 * GV; t += blockDim.x) {
-            int const c = t / GV;
-            int const r = t - c * GV;
-            int const tx = r % GX;
-            int const ty = (r / GX) % GY;
-            int const tz = r / (GX * GY);
-            int const gx = wrapIdx(ox - GLO + tx, a.g.nx);
-            int const gy = wrapIdx(oy - GLO + ty, a.g.ny);
-            int const gz = wrapIdx(oz - GLO + tz, a.g.nz);
-            size_t const gi = (size_t)gx + (size_t)a.g.nx * ((size_t)gy + (size_t)a.g.ny * gz);
-            const float* src = c < 3 ? a.E[c] : a.B[c - 3];
-            // fields beyond an open border read zero
-            bool const out = decltype(openBorders)::value && outsideOpen(a.g, ox - GLO + tx, oy - GLO + ty, oz - GLO + tz);
-            sEB[t] = out ? 0.0f : src[gi];
-        }
-    };
+    // The E/B tile: a thread's node offsets are formed once for the six
+    // components, and all its loads are in flight before the first LDS write
+    // (a loop of load and write costs a memory latency per round, which a
+    // supercell of few particles does not hide). Supercells whose tile lies
+    // inside the box skip the wrap.
     if (MODE != 2) {
-        if (a.g.open)
-            stageEB(std::true_type{});
-        else
-            stageEB(std::false_type{});
+        using T = EBTile<SUPP>;
+        constexpr int NU = (GV + kPushThreads - 1) / kPushThreads;
+        bool const inside = ox >= GLO && ox + SCX + GUP <= a.g.nx && oy >= GLO && oy + SCY + GUP <= a.g.ny &&
+                            oz >= GLO && oz + SCZ + GUP <= a.g.nz;
+        size_t gi[NU];
+        bool out[NU];
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            int tx, ty, tz;
+            boxCoords<GX, GY, GZ>(tid + u * kPushThreads, tx, ty, tz);
+            int gx = ox - GLO + tx, gy = oy - GLO + ty, gz = oz - GLO + tz;
+            out[u] = false;
+            if (!inside) {  // uniform
+                out[u] = a.g.open && outsideOpen(a.g, gx, gy, gz);  // fields beyond an open border read zero
+                gx = wrapIdx(gx, a.g.nx);
+                gy = wrapIdx(gy, a.g.ny);
+                gz = wrapIdx(gz, a.g.nz);
+            }
+            gi[u] = (size_t)gx + (size_t)a.g.nx * ((size_t)gy + (size_t)a.g.ny * gz);
+            if (tid + u * kPushThreads >= GV) gi[u] = 0;
+        }
+        float v[6][NU];
+#pragma unroll
+        for (int c = 0; c < 6; ++c) {
+            const float* const src = c < 3 ? a.E[c] : a.B[c - 3];
+#pragma unroll
+            for (int u = 0; u < NU; ++u) v[c][u] = src[gi[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            int tx, ty, tz;
+            boxCoords<GX, GY, GZ>(tid + u * kPushThreads, tx, ty, tz);
+#pragma unroll
+            for (int c = 0; c < 6; ++c) {
+                // the component's box of nodes within the common one
+                int const x = tx - (GLO - T::lo(c, 0)), y = ty - (GLO - T::lo(c, 1)), z = tz - (GLO - T::lo(c, 2));
+                if ((unsigned)x >= (unsigned)T::ext(c, 0) || (unsigned)y >= (unsigned)T::ext(c, 1) ||
+                    (unsigned)z >= (unsigned)T::ext(c, 2))
+                    continue;
+                float const f = out[u] ? 0.0f : v[c][u];
+                float* const row = sEB + T::off(c) + (z * T::ext(c, 1) + y) * T::pitch(c);
+                if (T::ODD) {
+                    row[x] = f;
+                    if (T::ext(c, 0) % 2 == 1 && x == T::ext(c, 0) - 1) row[x + 1] = 0.0f;  // the pad
+                } else {  // node x in the pairs (x, x+1) and (x-1, x)
+                    if (x < T::ext(c, 0) - 1) row[2 * x] = f;
+                    if (x > 0) row[2 * x - 1] = f;
+                }
+            }
+        }
     }
     if (MODE != 0) {
-        for (int t = tid; t < J_ELEMS; t += blockDim.x) sJ[t] = 0ull;
+        static_assert(MODE == 0 || J_ELEMS % 2 == 0, "two tile elements per store");
+        for (int t = tid; t < J_ELEMS / 2; t += kPushThreads) reinterpret_cast<ulonglong2*>(sJ)[t] = make_ulonglong2(0ull, 0ull);
     }
     __syncthreads();
 
-    PushConsts pk;
-    pk.cell[0] = a.cell[0];
-    pk.cell[1] = a.cell[1];
-    pk.cell[2] = a.cell[2];
-    pk.dt = a.dt;
-    pk.c2 = a.c2;
-    pk.rc2 = a.rc2;
-    pk.c = a.c;
     DepositConsts dk;
     dk.cell[0] = a.cell[0];
     dk.cell[1] = a.cell[1];
     dk.cell[2] = a.cell[2];
-    dk.dt = a.dt;
+    dk.rcell[0] = a.rcell[0];
+    dk.rcell[1] = a.rcell[1];
+    dk.rcell[2] = a.rcell[2];
+    dk.rvol = a.rvol;
     dk.inv_vdt = a.inv_vdt;
     dk.jscale = a.jscale;
 
@@ -207,20 +401,21 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
                 dampSC = dampSC || org[d] - 1 < a.damp.lo[d] || org[d] + ext[d] >= a.damp.hi[d];
     }
 
-    SlowItem qA{}, qB{};
+    uint32_t qA = 0u, qB = 0u;
     int queued = 0;  // wave-uniform
+    uint32_t leaveBits = 0u;
     for (int s = 0; s < a.nsp; ++s) {
         const SpeciesDev& S = a.sp[s];
         int const n = (int)S.count[sc];
         size_t const base = slotBase(S, sc);
-        uint32_t leaveBits = 0u;  // bit `it`: the particle of iteration `it` left the supercell
-        int const iters = (n + (int)blockDim.x - 1) / (int)blockDim.x;  // uniform across the workgroup
+        leaveBits = 0u;  // bit `it`: the particle of iteration `it` left the supercell (it < kPushMaxIters)
+        int const iters = (n + kPushThreads - 1) / kPushThreads;  // uniform across the workgroup
         // the last species runs one iteration more, without particles, that drains the queue
         bool const lastSpecies = s == a.nsp - 1;
         for (int it = 0; it < iters + (MODE == 1 && !EMZ && lastSpecies ? 1 : 0); ++it) {
-            int const i = it * (int)blockDim.x + tid;
+            int const i = it * kPushThreads + tid;
             bool slow = false;
-            SlowItem mine{};
+            uint32_t mine = 0u;
             if (i < n) {
                 size_t const gidx = base + i;
                 Vec3 const pos{S.pos[0][gidx], S.pos[1][gidx], S.pos[2][gidx]};
@@ -231,19 +426,21 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
                 float const mass = S.mass * w;     // attribute::getMass (GetMass.hpp:40-44)
                 float charge = S.charge * w;       // attribute::getCharge (GetCharge.hpp:45-66)
                 if (MODE != 2) {
-                    Vec3 const e = gatherE<SUPP, GX, GY, GV>(sEB, lx + GLO, ly + GLO, lz + GLO, pos);
-                    Vec3 const b = gatherB<SUPP, GX, GY, GV>(sEB + 3 * GV, lx + GLO, ly + GLO, lz + GLO, pos);
+                    WeightTerms const terms = weightTerms<PUSHER>(mass, charge);
+                    GatherWeights<SUPP> const gw(pos, lx, ly, lz);
+                    Vec3 const e{gather1<SUPP, 0>(sEB, gw), gather1<SUPP, 1>(sEB, gw), gather1<SUPP, 2>(sEB, gw)};
+                    Vec3 const b{gather1<SUPP, 3>(sEB, gw), gather1<SUPP, 4>(sEB, gw), gather1<SUPP, 5>(sEB, gw)};
                     Vec3 vel;
                     if (PUSHER == PIC_PUSHER_VAY)
-                        pushVay(e, b, mom, vel, mass, charge, pk);
+                        pushVay(e, b, mom, vel, mass, charge, terms);
                     else if (PUSHER == PIC_PUSHER_HIGUERA_CARY)
-                        pushHigueraCary(e, b, mom, vel, mass, charge, pk);
+                        pushHigueraCary(e, b, mom, vel, mass, charge, terms);
                     else
-                        pushBoris(e, b, mom, vel, mass, charge, pk);
+                        pushBoris(e, b, mom, vel, mass, charge, terms);
                     float p[3] = {pos.x, pos.y, pos.z};
                     // the move in cells; Esirkepov forms the same quotients (Esirkepov.hpp:82)
-                    float dp[3] = {(vel.x * pk.dt) / pk.cell[0], (vel.y * pk.dt) / pk.cell[1],
-                                   (vel.z * pk.dt) / pk.cell[2]};
+                    float dp[3] = {divExact(vel.x, dk.rcell[0]), divExact(vel.y, dk.rcell[1]),
+                                   divExact(vel.z, dk.rcell[2])};
                     p[0] += dp[0];
                     p[1] += dp[1];
                     p[2] += dp[2];
@@ -272,18 +469,18 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
                                 bool const inArea = (e & 1) == 0 ? cn >= a.damp.hi[d] : cn < a.damp.lo[d];
                                 if (!inArea) continue;
                                 float const pd = d == 0 ? p[0] : (d == 1 ? p[1] : p[2]);
-                                float const cs = d == 0 ? pk.cell[0] : (d == 1 ? pk.cell[1] : pk.cell[2]);
-                                pmlDamp(a.damp, d, cn, pd, S.mass, pk.rc2, pk.dt, cs, mom, w);
+                                float const cs = d == 0 ? a.cell[0] : (d == 1 ? a.cell[1] : a.cell[2]);
+                                pmlDamp(a.damp, d, cn, pd, S.mass, cs, mom, w);
                                 any = true;
                             }
                         }
                         if (any) {
                             S.w[gidx] = w;
                             charge = S.charge * w;
-                            vel = velocityOf(mom, S.mass * w, pk.rc2);
-                            dp[0] = (vel.x * pk.dt) / pk.cell[0];
-                            dp[1] = (vel.y * pk.dt) / pk.cell[1];
-                            dp[2] = (vel.z * pk.dt) / pk.cell[2];
+                            vel = velocityOf(mom, S.mass * w);
+                            dp[0] = divExact(vel.x, dk.rcell[0]);
+                            dp[1] = divExact(vel.y, dk.rcell[1]);
+                            dp[2] = divExact(vel.z, dk.rcell[2]);
                         }
                     }
                     S.pos[0][gidx] = p[0];
@@ -294,7 +491,7 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
                     S.mom[2][gidx] = mom.z;
                     if ((dir[0] | dir[1] | dir[2]) != 0) S.cell[gidx] = (uint16_t)newIdx;
                     if (newMask >= 2) S.mask[gidx] = (uint8_t)newMask;
-                    leaveBits |= (newMask >= 2 ? 1u : 0u) << (i / kPushThreads);
+                    leaveBits |= (newMask >= 2 ? 1u : 0u) << (it & (kPushMaxIters - 1));
                     // a particle leaving through an open border is absorbed by the
                     // boundary before the reference's deposit stage sees it
                     if (MODE == 1 && !(a.g.open && outsideOpen(a.g, ox + lx + dir[0], oy + ly + dir[1], oz + lz + dir[2]))) {
@@ -303,17 +500,17 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
                         if (EMZ) {
                             EmZ<SUPP>::template depositDp<TG>(sJ, cx, cy, cz, np, dp, charge, dk);
                         } else {
-                            auto const G = Esirkepov<SUPP>::geometryDp(np, dp);
-                            if (Esirkepov<SUPP>::changesCell(G)) {
-                                slow = true;
-                                mine = SlowItem{cx | (cy << 8) | (cz << 16), np.x, np.y, np.z, dp[0], dp[1], dp[2], charge};
-                            } else {
+                            typename Esirkepov<SUPP>::Geometry G;
+                            if (Esirkepov<SUPP>::stayGeometry(np, dp, G)) {
                                 Esirkepov<SUPP>::template depositStay<TG>(sJ, cx, cy, cz, G, charge, dk);
+                            } else {
+                                slow = true;
+                                mine = slowItem(i, cx, cy, cz, s);
                             }
                         }
                     }
                 } else {
-                    Vec3 const vel = velocityOf(mom, mass, a.rc2);
+                    Vec3 const vel = velocityOf(mom, mass);
                     if (EMZ)
                         EmZ<SUPP>::template deposit<TG>(sJ, lx + DLO, ly + DLO, lz + DLO, pos, vel, charge, dk);
                     else
@@ -324,89 +521,97 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
             if (MODE == 1 && !EMZ) {
                 queueSlow(slow, mine, qA, qB, queued);
                 if (queued >= 64 || (it == iters && queued > 0)) {
-                    if ((int)(tid & 63) < queued) depositQueued<SUPP, TG>(sJ, qA, dk);
+                    // the queued particles' stores by other lanes of this wave come first
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    if ((int)(tid & 63) < queued) depositQueued<SUPP, TG>(sJ, a, sc, qA, dk);
                     qA = qB;
                     queued = queued > 64 ? queued - 64 : 0;
                 }
             }
         }
-        if (MODE != 2 && S.lists) S.leaveBits[(size_t)sc * kPushThreads + tid] = leaveBits;
+        // (the last species' bits stay in the register)
+        if (MODE != 2 && !lastSpecies) S.leaveBits[(size_t)sc * kPushThreads + tid] = leaveBits;
     }
     __syncthreads();
 
-    auto flushJ = [&](auto openBorders) {
-        for (int t = tid; t < J_ELEMS; t += blockDim.x) {
-            long long const acc = fixedTileValue(sJ[t]);
-            if (acc == 0) continue;
-            int const c = t < TG::off(1) ? 0 : (t < TG::off(2) ? 1 : 2);
-            int const r = t - (c == 0 ? 0 : TG::off(c));
-            int const ex = c == 0 ? TG::ext(0, 0) : (c == 1 ? TG::ext(1, 0) : TG::ext(2, 0));
-            int const ey = c == 0 ? TG::ext(0, 1) : (c == 1 ? TG::ext(1, 1) : TG::ext(2, 1));
-            int const tx = r % ex;
-            int const ty = (r / ex) % ey;
-            int const tz = r / (ex * ey);
-            if (decltype(openBorders)::value && outsideOpen(a.g, ox - DLO + tx, oy - DLO + ty, oz - DLO + tz))
-                continue;  // dropped beyond the border
-            int const gx = wrapIdx(ox - DLO + tx, a.g.nx);
-            int const gy = wrapIdx(oy - DLO + ty, a.g.ny);
-            int const gz = wrapIdx(oz - DLO + tz, a.g.nz);
-            size_t const gi = (size_t)gx + (size_t)a.g.nx * ((size_t)gy + (size_t)a.g.ny * gz);
-            float const v = (float)((double)acc * a.jinv);
-            a.J[c][gi] += v;
-        }
-    };
     if (MODE == 1 && a.tileOut) {
         // one launch for every supercell: the tile is left for the gather
         // flush as the floats the flush would add, zero where it adds
         // nothing (adding a zero would change nothing either: J never holds
         // -0, its sums start at +0 and round to nearest)
-        for (int t = tid; t < J_ELEMS; t += blockDim.x) {
+        for (int t = tid; t < J_ELEMS; t += kPushThreads) {
             long long const acc = fixedTileValue(sJ[t]);
             a.tileOut[(size_t)sc * J_ELEMS + t] = acc == 0 ? 0.0f : (float)((double)acc * a.jinv);
         }
     } else if (MODE != 0) {
-        if (a.g.open)
-            flushJ(std::true_type{});
-        else
-            flushJ(std::false_type{});
+        bool const inside = ox >= DLO && ox + SCX + UPM <= a.g.nx && oy >= DLO && oy + SCY + UPM <= a.g.ny &&
+                            oz >= DLO && oz + SCZ + UPM <= a.g.nz;
+        flushComponent<TG, 0, DLO>(a, sJ, ox, oy, oz, inside);
+        flushComponent<TG, 1, DLO>(a, sJ, ox, oy, oz, inside);
+        flushComponent<TG, 2, DLO>(a, sJ, ox, oy, oz, inside);
     }
 
-    // Epilogue: slot-ordered leaver list from the ballots, then grouped by
-    // exchange code (the input of the supercell shift); in a full step also
-    // the staging of the shift (outbox records, compaction of the supercell).
+    // Epilogue: the leavers from the per-thread bits, in slot order; in a full
+    // step staged for the shift (outbox records, compaction of the supercell),
+    // else as the leaver lists of the stage calls.
     if (MODE != 2) {
         for (int s = 0; s < a.nsp; ++s) {
             const SpeciesDev& S = a.sp[s];
-            if (!S.lists) continue;
             int const n = (int)S.count[sc];
             int const iters = (n + kPushThreads - 1) / kPushThreads;
             int const wave = tid >> 6;
-            uint32_t const bits = S.leaveBits[(size_t)sc * kPushThreads + tid];
-            __syncthreads();
-            // leavers per (iteration, wave) entry, entries in slot order
-            for (int it = 0; it < iters; ++it) {
-                unsigned long long const m = __ballot((bits >> it) & 1u);
-                if ((tid & 63) == 0) sPre[it * kPushWaves + wave] = (uint32_t)__popcll(m);
-            }
-            __syncthreads();
-            if (tid == 0) {
-                uint32_t acc = 0;
-                for (int e = 0; e < iters * kPushWaves; ++e) {
-                    uint32_t const c = sPre[e];
-                    sPre[e] = acc;
-                    acc += c;
-                }
-                sPre[kPushMaxIters * kPushWaves] = acc;
-            }
-            __syncthreads();
-            int const L = (int)sPre[kPushMaxIters * kPushWaves];
             size_t const base = slotBase(S, sc);
-            for (int it = 0; it < iters; ++it) {
-                bool const left = (bits >> it) & 1u;
-                unsigned long long const m = __ballot(left);
-                if (left)
-                    S.scratch[base + sPre[it * kPushWaves + wave] + (uint32_t)__popcll(m & laneMaskLt())] =
-                        it * kPushThreads + tid;
+            int L = 0;
+            __syncthreads();
+            if (iters <= kPushMaxIters) {
+                uint32_t const bits =
+                    s == a.nsp - 1 ? leaveBits : S.leaveBits[(size_t)sc * kPushThreads + tid];
+                // leavers per (iteration, wave) entry, entries in slot order
+                for (int it = 0; it < iters; ++it) {
+                    unsigned long long const m = __ballot((bits >> it) & 1u);
+                    if ((tid & 63) == 0) sPre[it * kPushWaves + wave] = (uint32_t)__popcll(m);
+                }
+                __syncthreads();
+                if (wave == 0) {  // exclusive prefix, four entries per lane
+                    constexpr int PER = kPushMaxIters * kPushWaves / 64;
+                    int const entries = iters * kPushWaves;
+                    uint32_t c[PER], sum = 0;
+#pragma unroll
+                    for (int e = 0; e < PER; ++e) {
+                        c[e] = tid * PER + e < entries ? sPre[tid * PER + e] : 0u;
+                        sum += c[e];
+                    }
+                    uint32_t const incl = waveInclusiveScan(sum);
+                    uint32_t acc = incl - sum;
+#pragma unroll
+                    for (int e = 0; e < PER; ++e) {
+                        if (tid * PER + e < entries) sPre[tid * PER + e] = acc;
+                        acc += c[e];
+                    }
+                    if (tid == 63) sPre[kPushMaxIters * kPushWaves] = incl;
+                }
+                __syncthreads();
+                L = (int)sPre[kPushMaxIters * kPushWaves];
+                if (a.stageShift && L <= kLeaverListLds) {
+                    stageFromBits(S, sc, n, iters, bits, L, sPre, sGroup, sWaveCnt, sList);
+                    continue;
+                }
+                for (int it = 0; it < iters; ++it) {
+                    bool const left = (bits >> it) & 1u;
+                    unsigned long long const m = __ballot(left);
+                    if (left)
+                        S.scratch[base + sPre[it * kPushWaves + wave] + (uint32_t)__popcll(m & laneMaskLt())] =
+                            it * kPushThreads + tid;
+                }
+            } else {  // more particles than bits: the leavers from their multiMask
+                for (int c0 = 0; c0 < n; c0 += kPushThreads) {
+                    int const i = c0 + tid;
+                    bool const left = i < n && S.mask[base + i] >= 2;
+                    int total;
+                    int const r = blockRank<kPushWaves>(left, sWaveCnt, &total);
+                    if (left) S.scratch[base + L + r] = i;
+                    L += total;
+                }
             }
             __syncthreads();
             groupLeavers<kPushWaves>(S, sc, L, sGroup, sWaveCnt);
@@ -415,13 +620,19 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
     }
 }
 
-// Waves per SIMD the register budget must allow: PQS at most 128 VGPRs, so
-// two workgroups share a CU (their LDS fits); TSC at most 80, so three do
-// (3 x 53.6 KB of LDS fit the CU's 160 KB): the compiler spills a few values
-// and the launch is faster, the LDS bank conflicts of the gather and the
-// deposit being hidden better by the extra waves
+// What bounds the kernel (TSC, Boris, 33.5M particles a launch): the LDS, whose
+// bank conflicts follow from 64 lanes at unrelated cells, and the vector
+// issue, both near 80 % of the launch. Before the aligned reads of the E/B
+// tile and the one-word queue the LDS was busy 86 % of it and the vector
+// units 73 %; on the 256^3 two-species shear flow a pass of five steps went
+// from 150.1 to 125.5 ms.
+// Waves per SIMD the register budget must allow. TSC and PQS: at most 128
+// VGPRs, two workgroups per CU. TSC at 80 VGPRs has room for three, but the
+// loop then spills (126 ms a pass against 133 to 142 with 80 VGPRs), and
+// workgroups of 320 to 768 threads measured 12 to 28 % slower than 512. CIC
+// needs 80 VGPRs, three workgroups.
 template <int SUPP, int PUSHER, int MODE, bool EMZ = false>
-__global__ __launch_bounds__(kPushThreads, SUPP == 4 ? 4 : (SUPP == 3 ? 6 : 1)) void kPushDeposit(PushArgs a) {
+__global__ __launch_bounds__(kPushThreads, SUPP == 2 ? 6 : 4) void kPushDeposit(PushArgs a) {
     __shared__ __align__(16) unsigned char smem[PushLds<SUPP, MODE>::BYTES];
     pushDepositSC<SUPP, PUSHER, MODE, EMZ>(a, a.scList[blockIdx.x], smem);
 }
@@ -430,7 +641,7 @@ __global__ __launch_bounds__(kPushThreads, SUPP == 4 ? 4 : (SUPP == 3 ? 6 : 1)) 
 // its own: the FP64 pow and exp of the damping would raise the register
 // pressure of every launch)
 template <int SUPP, int PUSHER, int MODE, bool EMZ = false>
-__global__ __launch_bounds__(kPushThreads, SUPP == 4 ? 4 : (SUPP == 3 ? 6 : 1)) void kPushDepositPml(PushArgs a) {
+__global__ __launch_bounds__(kPushThreads, SUPP == 2 ? 6 : 4) void kPushDepositPml(PushArgs a) {
     __shared__ __align__(16) unsigned char smem[PushLds<SUPP, MODE>::BYTES];
     pushDepositSC<SUPP, PUSHER, MODE, EMZ, true>(a, a.scList[blockIdx.x], smem);
 }
@@ -438,14 +649,21 @@ __global__ __launch_bounds__(kPushThreads, SUPP == 4 ? 4 : (SUPP == 3 ? 6 : 1)) 
 // Batched form for ensembles: work items (simulation, supercell) of one
 // checkerboard phase of every simulation in one launch; a workgroup takes
 // items blockIdx.x, blockIdx.x + gridDim.x, ... so a grid smaller than the
-// item count runs persistently.
+// item count runs persistently. The member's arguments are read as constant
+// memory (the table does not change while the kernel runs) at a uniform
+// index, so they come by scalar loads as a kernel's own arguments do; as
+// ordinary memory that stores might change they were held in vector
+// registers (240 bytes per lane spilled, one workgroup less per CU).
 template <int SUPP, int PUSHER, int MODE, bool EMZ = false>
-__global__ __launch_bounds__(kPushThreads) void kPushDepositBatch(const PushArgs* __restrict__ table,
+__global__ __launch_bounds__(kPushThreads, SUPP == 2 ? 6 : 4) void kPushDepositBatch(const PushArgs* __restrict__ table,
                                                                   const int2* __restrict__ work, int nwork) {
     __shared__ __align__(16) unsigned char smem[PushLds<SUPP, MODE>::BYTES];
     for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
         int2 const it = work[w];
-        pushDepositSC<SUPP, PUSHER, MODE>(table[it.x], it.y, smem);
+        uintptr_t at = reinterpret_cast<uintptr_t>(table + __builtin_amdgcn_readfirstlane(it.x));
+        asm volatile("" : "+s"(at));  // hides where the address comes from, so the cast below stays
+        auto const entry = (const __attribute__((address_space(4))) PushArgs*)at;
+        pushDepositSC<SUPP, PUSHER, MODE>(*(const PushArgs*)entry, __builtin_amdgcn_readfirstlane(it.y), smem);
         __syncthreads();  // the next item reuses the LDS
     }
 }

@@ -61,17 +61,6 @@ __global__ __launch_bounds__(kThreads) void kStage(SpeciesDev S, GridDev grid) {
 // One wave per destination supercell, four supercells per workgroup.
 constexpr int kScPerBlock = kThreads / 64;
 
-// inclusive prefix sum over the 64 lanes of a wave
-__device__ __forceinline__ uint32_t waveInclusiveScan(uint32_t v) {
-    int const lane = threadIdx.x & 63;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        uint32_t const t = __shfl_up(v, o);
-        if (lane >= o) v += t;
-    }
-    return v;
-}
-
 // insert for destination supercell d; called by one whole wave. A record
 // whose slot lies beyond the capacity is left in the sender's outbox, the
 // count still grows by every incoming record and the overflow flag is set;

@@ -1010,11 +1010,10 @@ pic::PushArgs makePushArgs(pic_ctx* c) {
         a.B[d] = c->B[d];
         a.J[d] = c->J[d];
         a.cell[d] = c->k.cell[d];
+        a.rcell[d] = 1.0 / static_cast<double>(c->k.cell[d]);
     }
-    a.dt = c->k.dt;
-    a.c = c->k.c;
-    a.c2 = c->k.c * c->k.c;
-    a.rc2 = c->k.mue0_eps0;
+    float const volume = c->k.cell[0] * c->k.cell[1] * c->k.cell[2];
+    a.rvol = 1.0 / static_cast<double>(volume);
     a.inv_vdt = c->k.inv_cell_volume_dt;
     a.jscale = std::ldexp(1.0, c->jexp);
     a.jinv = std::ldexp(1.0, -c->jexp);
@@ -1092,7 +1091,7 @@ int runPush(pic_ctx* c, int32_t species, int mode, bool stageShift = false) {
         for (size_t i = 0; i < grp.size(); ++i) a.sp[i] = c->sp[grp[i]].dev;
         a.stageShift = stageShift ? 1 : 0;
         if (mode != 2)
-            for (int s : grp) c->sp[s].shiftReady = c->sp[s].dev.lists != 0 ? (stageShift ? 2 : 1) : 0;
+            for (int s : grp) c->sp[s].shiftReady = stageShift ? 2 : 1;
         if (mode == 0) {
             a.scList = c->dAll;
             TimerScope ts(c, PIC_TIMER_PUSH);
@@ -1278,11 +1277,6 @@ int growSpecies(pic_ctx* c, int s, const std::vector<uint32_t>& caps) {
         m.desc.frames_per_sc = m.cap / pic::kSCV;
         c->cfg.species[s].frames_per_sc = m.desc.frames_per_sc;
         d.cap = m.cap;
-        int const lists = m.cap <= pic::kListMaxSlots ? 1 : 0;
-        if (lists != d.lists) {  // captured steps hold the old flag
-            d.lists = lists;
-            dropGraphs(c);
-        }
         return uploadRuns(c, m);
     }
     // repack into fresh arrays with a quarter more slots
@@ -1322,7 +1316,6 @@ int growSpecies(pic_ctx* c, int s, const std::vector<uint32_t>& caps) {
     devFree(c, d.outIdx);
     devFree(c, d.scratch);
     n.cap = m.cap;
-    n.lists = m.cap <= pic::kListMaxSlots ? 1 : 0;
     d = n;
     m.desc.frames_per_sc = m.cap / pic::kSCV;
     c->cfg.species[s].frames_per_sc = m.desc.frames_per_sc;
@@ -1589,7 +1582,6 @@ int pic_create(const pic_config* cfg, pic_ctx** out) {
         d.base = m.dBase;
         d.capOf = m.dCap;
         d.cap = m.cap;
-        d.lists = m.cap <= pic::kListMaxSlots ? 1 : 0;
         d.reflect = 0;
         for (int a = 0; a < 3; ++a)
             if (cfg->species[s].particle_boundary[a] == PIC_PARTICLE_REFLECTING) d.reflect |= 1 << a;
@@ -2857,6 +2849,9 @@ int pic_adjoint_backward(pic_ctx* c, const double* dE, const double* dB, double*
 // ---------------------------------------------------------------------------
 // batched ensembles of independent simulations
 // ---------------------------------------------------------------------------
+// frames per supercell an ensemble's members are bound to
+constexpr int kEnsembleMaxFrames = 64;
+
 struct pic_ensemble {
     std::vector<pic_ctx*> sims;
     int device = 0;
@@ -3078,14 +3073,14 @@ int ensFinish(pic_ensemble* e) {
         int skipped = 0;
         uint32_t const raised = c->hostFlags;
         c->hostFlags = 0;
-        int r = recoverCapacity(c, &skipped, pic::kListMaxSlots / pic::kSCV);
+        int r = recoverCapacity(c, &skipped, kEnsembleMaxFrames);
         if (c->hostFlags & PIC_FLAG_CAPACITY_GREW) moved = true;
         c->hostFlags |= raised;
         if (r != PIC_OK) return r;
         while (skipped > 0) {
             for (int i = 0; i < skipped; ++i)
                 if ((r = oneStep(c)) != PIC_OK) return r;
-            if ((r = recoverCapacity(c, &skipped, pic::kListMaxSlots / pic::kSCV)) != PIC_OK) return r;
+            if ((r = recoverCapacity(c, &skipped, kEnsembleMaxFrames)) != PIC_OK) return r;
         }
     }
     if (moved) return ensUploadTables(e);
@@ -3124,7 +3119,7 @@ int pic_ensemble_create(const pic_config* cfgs, int32_t n, pic_ensemble** out) {
                 return bail(fail(PIC_E_INVALID, "ensemble species use the Esirkepov current solver"));
             supp = sp;
             pusher = c.species[s].pusher;
-            if (c.species[s].frames_per_sc * pic::kSCV > pic::kListMaxSlots)
+            if (c.species[s].frames_per_sc > kEnsembleMaxFrames)
                 return bail(fail(PIC_E_INVALID, "ensemble species need at most 64 frames per supercell"));
         }
         if (i == 0) {

@@ -49,6 +49,47 @@ __device__ __forceinline__ float esirkepovWeight(float s0i, float dsi, float s0j
     return mad((1.0f / 3.0f) * dsj, dsi, half);
 }
 
+// RN(1 / s) for the root s of a float: the hardware reciprocal (within an ulp)
+// and one Newton step in multiply-adds. The residual 1 - s r is exact; the
+// step's rounding is the correct one for every float of [1, 4), which with
+// the exact scaling by powers of 2 is every s whose reciprocal is normal
+// (a root lies in [2^-75, 2^64]); div_fixup gives 1/0, 1/inf and 1/NaN. Four
+// instructions instead of the eleven of the full division, whose scaling of
+// denormal operands a root never needs.
+__device__ __forceinline__ float recipOfRoot(float s) {
+    float r = __builtin_amdgcn_rcpf(s);
+    r = __builtin_fmaf(__builtin_fmaf(-s, r, 1.0f), r, r);
+    return __builtin_amdgcn_div_fixupf(r, s, 1.0f);
+}
+
+// the same for x >= 1 (or NaN); the full division above 2^126
+__device__ __forceinline__ float recipAbove1(float x) {
+    float r = __builtin_amdgcn_rcpf(x);
+    r = __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+    if (!(x <= 8.5070592e37f)) r = 1.0f / x;
+    return r;
+}
+
+// RN(sqrt(x)) for x >= 1 (or NaN): the hardware root (within an ulp) and its
+// two neighbours tested by the signs of exact residuals. The general sqrtf
+// scales arguments below 2^-96 besides.
+__device__ __forceinline__ float sqrtAbove1(float x) {
+    float const s = __builtin_amdgcn_sqrtf(x);
+    float const down = __int_as_float(__float_as_int(s) - 1);
+    float const up = __int_as_float(__float_as_int(s) + 1);
+    float const rd = __builtin_fmaf(-down, s, x);
+    float const ru = __builtin_fmaf(-up, s, x);
+    float const t = rd <= 0.0f ? down : s;
+    return ru > 0.0f ? up : t;
+}
+
+// RN(x / c) from rc = RN64(1 / c): the FP64 product is within 2^-52 of x / c
+// relatively, and no quotient of two floats lies closer than 2^-49 to the
+// midpoint of two neighbouring normal floats (|x - m c| is at least one unit
+// of a 49-bit product, and never 0 for a 25-bit m), so rounding the product
+// rounds the quotient. Three instructions instead of eleven.
+__device__ __forceinline__ float divExact(float x, double rc) { return (float)((double)x * rc); }
+
 // cross product (pmacc/math/vector/Vector.tpp:71-76)
 __device__ __forceinline__ Vec3 cross(Vec3 a, Vec3 b) {
     return Vec3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
@@ -197,69 +238,139 @@ __device__ __forceinline__ void cachedShape(float pos, bool outOfRange, float* s
 // Field gather: FieldToParticleInterpolation<Shape, AssignedTrilinearInterpolation>
 // (algorithms/FieldToParticleInterpolation.hpp:43-131,
 // ShiftCoordinateSystem.hpp:36-80, AssignedTrilinearInterpolation.hpp:53-86).
-// `tile` is one field component staged as [z][y][x] with row pitch TX and
-// plane pitch TX*TY; (cx,cy,cz) is the particle's cell in tile coordinates.
+// Components 0..2 are E, at (1/2,0,0),(0,1/2,0),(0,0,1/2); 3..5 are B, at
+// (0,1/2,1/2),(1/2,0,1/2),(1/2,1/2,0) (fields/YeeCell.hpp:69-123).
 // ---------------------------------------------------------------------------
-template <int SUPP, int TX, int TY>
-__device__ __forceinline__ float gather1(const float* __restrict__ tile, int cx, int cy, int cz, Vec3 pos,
-                                         float fx, float fy, float fz) {
-    constexpr bool isEven = (SUPP % 2) == 0;
-    constexpr int begin = -SUPP / 2 + (SUPP + 1) % 2;
-    float p[3] = {pos.x, pos.y, pos.z};
-    float const f[3] = {fx, fy, fz};
-    int ishift[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        float const v_pos = p[d] - f[d] - 0.5f;
-        int s;
-        if (isEven)
-            s = v_pos >= -0.5f ? 0 : -1;
-        else
-            s = v_pos >= 0.0f ? 1 : 0;
-        ishift[d] = s;
-        p[d] = v_pos - (float)s + 0.5f;
+
+// component c sits half a cell off along axis a
+__host__ __device__ constexpr bool yeeHalf(int c, int a) { return c < 3 ? a == c : a != c - 3; }
+
+// The E/B tile in LDS: one box per component, holding the nodes the particles
+// of a supercell reach. Along an axis the stencil's first node lies at a fixed
+// distance from the particle's cell or at one of two (ShiftCoordinateSystem:
+// an odd support shifts on the integer positions, an even one on the half
+// positions, for in-cell positions in [0,1)).
+// The lanes of a wave read rows at unrelated addresses, so the bank conflicts
+// set the cost of a read: measured on random rows, cycles per CU and wave
+// instruction, ds_read_b32 7.0, ds_read2_b32 13.7, an aligned ds_read_b64 6.6
+// (unaligned 65, ds_read2_b64 24), an aligned ds_read_b128 11.4 (ds_read_b96
+// 20). Hence aligned pairs, each an instruction of its own:
+//  - even support (CIC, PQS): every node x is stored as the pair (x, x+1), so
+//    a row of 2 or 4 nodes is one read or two (6.6 and 13.2 cycles instead of
+//    13.7 and 27.4);
+//  - odd support (TSC): rows have an even pitch, and a row of 3 nodes is read
+//    as the two aligned pairs that hold it, its weights shifted by one place
+//    and padded with a zero when it starts on an odd node: 13.2 cycles
+//    instead of 20.7 for one multiply-add more. Storing every start (quads or
+//    pairs) spares the multiply-add and measured 2 to 7 % slower.
+template <int SUPP>
+struct EBTile {
+    static constexpr bool ODD = SUPP % 2 == 1;
+    static constexpr int begin = -SUPP / 2 + (SUPP + 1) % 2;
+    __host__ __device__ static constexpr bool shifts(int c, int a) { return yeeHalf(c, a) != ODD; }
+    // nodes below and above the particle's cell
+    __host__ __device__ static constexpr int lo(int c, int a) { return -begin + (!ODD && shifts(c, a) ? 1 : 0); }
+    __host__ __device__ static constexpr int hi(int c, int a) { return begin + SUPP - 1 + (ODD && shifts(c, a) ? 1 : 0); }
+    __host__ __device__ static constexpr int ext(int c, int a) {
+        return (a == 0 ? SCX : (a == 1 ? SCY : SCZ)) + lo(c, a) + hi(c, a);
     }
-    float sx[SUPP], sy[SUPP], sz[SUPP];
-    Shape<SUPP>::onSupport(p[0], sx);
-    Shape<SUPP>::onSupport(p[1], sy);
-    Shape<SUPP>::onSupport(p[2], sz);
-    int const bx = cx + ishift[0] + begin;
-    int const by = cy + ishift[1] + begin;
-    int const bz = cz + ishift[2] + begin;
-    // each partial sum starts at its first term; the reference adds that term
-    // to 0.0, which differs only in the sign of an all-zero sum (a zero field
-    // value adds nothing to a momentum, whatever its sign). Every further
-    // term is a multiply-add.
+    // floats per row
+    __host__ __device__ static constexpr int pitch(int c) { return ODD ? (ext(c, 0) + 1) / 2 * 2 : 2 * (ext(c, 0) - 1); }
+    __host__ __device__ static constexpr int plane(int c) { return pitch(c) * ext(c, 1); }
+    // first float of a component (even)
+    __host__ __device__ static constexpr int after(int at, int c) { return at + plane(c) * ext(c, 2); }
+    static constexpr int O1 = after(0, 0), O2 = after(O1, 1), O3 = after(O2, 2), O4 = after(O3, 3), O5 = after(O4, 4);
+    __host__ __device__ static constexpr int off(int c) {
+        return c == 0 ? 0 : (c == 1 ? O1 : (c == 2 ? O2 : (c == 3 ? O3 : (c == 4 ? O4 : O5))));
+    }
+    static constexpr int total() { return after(O5, 5); }
+};
+// Two floats of the tile. Volatile, because the compiler would join two pairs
+// of a row into one ds_read2_b64, which takes nearly twice their time.
+typedef float PairLds __attribute__((ext_vector_type(2)));
+typedef const volatile __attribute__((address_space(3))) PairLds* PairLdsPtr;
+
+// Shape values of one axis for the integer (HALF = false) or half positions;
+// returns the stencil's shift. A fixed stencil's shift is 0.
+template <int SUPP, bool HALF>
+__device__ __forceinline__ int nodeWeights(float pos, float* w) {
+    constexpr bool isEven = (SUPP % 2) == 0;
+    float const v = HALF ? pos - 0.5f - 0.5f : pos - 0.5f;
+    int shift = 0;
+    float p;
+    if (HALF == isEven) {
+        shift = isEven ? (v >= -0.5f ? 0 : -1) : (v >= 0.0f ? 1 : 0);
+        p = v - (float)shift + 0.5f;
+    } else {
+        p = v + 0.5f;
+    }
+    Shape<SUPP>::onSupport(p, w);
+    return shift;
+}
+
+// The six (axis, position) weight sets of a particle, for all components.
+template <int SUPP>
+struct GatherWeights {
+    float w[3][2][SUPP];  // axis, half
+    float wx[2][4];       // odd support: the x weights on the row's two aligned pairs
+    int first[3][2];      // cell + shift per axis and half
+    __device__ __forceinline__ GatherWeights(Vec3 pos, int lx, int ly, int lz) {
+        first[0][0] = lx + nodeWeights<SUPP, false>(pos.x, w[0][0]);
+        first[0][1] = lx + nodeWeights<SUPP, true>(pos.x, w[0][1]);
+        first[1][0] = ly + nodeWeights<SUPP, false>(pos.y, w[1][0]);
+        first[1][1] = ly + nodeWeights<SUPP, true>(pos.y, w[1][1]);
+        first[2][0] = lz + nodeWeights<SUPP, false>(pos.z, w[2][0]);
+        first[2][1] = lz + nodeWeights<SUPP, true>(pos.z, w[2][1]);
+        if (SUPP == 3) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                bool const odd = first[0][h] & 1;  // the row starts at node `first`
+                wx[h][0] = odd ? 0.0f : w[0][h][0];
+                wx[h][1] = odd ? w[0][h][0] : w[0][h][1];
+                wx[h][2] = odd ? w[0][h][1] : w[0][h][SUPP - 1];
+                wx[h][3] = odd ? w[0][h][SUPP - 1] : 0.0f;
+            }
+        }
+    }
+};
+
+// Component C at the particle. Each partial sum starts at its first term; the
+// reference adds that term to 0.0, which differs only in the sign of an
+// all-zero sum (a zero field value adds nothing to a momentum, whatever its
+// sign), as does the term of a padded zero weight. Every further term is a
+// multiply-add. One address for the stencil's first node: the others are
+// constant offsets from it, which the LDS reads take as immediates.
+template <int SUPP, int C>
+__device__ __forceinline__ float gather1(const float* __restrict__ tile, const GatherWeights<SUPP>& g) {
+    using T = EBTile<SUPP>;
+    constexpr int hx = yeeHalf(C, 0), hy = yeeHalf(C, 1), hz = yeeHalf(C, 2);
+    int const bx = g.first[0][hx] + (T::begin + T::lo(C, 0));
+    int const by = g.first[1][hy] + (T::begin + T::lo(C, 1));
+    int const bz = g.first[2][hz] + (T::begin + T::lo(C, 2));
+    constexpr int PP = T::pitch(C) / 2;  // in pairs
+    PairLdsPtr const corner =
+        (PairLdsPtr)(tile + T::off(C)) + ((bz * T::ext(C, 1) + by) * PP + (T::ODD ? bx >> 1 : bx));
     float result_z = 0.0f;
 #pragma unroll
     for (int z = 0; z < SUPP; ++z) {
         float result_y = 0.0f;
 #pragma unroll
         for (int y = 0; y < SUPP; ++y) {
-            const float* row = tile + ((bz + z) * TY + (by + y)) * TX + bx;
-            float result_x = row[0] * sx[0];
-#pragma unroll
-            for (int x = 1; x < SUPP; ++x) result_x = mad(row[x], sx[x], result_x);
-            result_y = y == 0 ? result_x * sy[0] : mad(result_x, sy[y], result_y);
+            PairLdsPtr const row = corner + (z * T::ext(C, 1) + y) * PP;
+            PairLds const p = row[0];
+            const float* const w = SUPP == 3 ? g.wx[hx] : g.w[0][hx];
+            float result_x = p.x * w[0];
+            result_x = mad(p.y, w[1], result_x);
+            if (SUPP > 2) {
+                PairLds const q = row[SUPP == 3 ? 1 : 2];
+                result_x = mad(q.x, w[2], result_x);
+                result_x = mad(q.y, w[3], result_x);
+            }
+            result_y = y == 0 ? result_x * g.w[1][hy][0] : mad(result_x, g.w[1][hy][y], result_y);
         }
-        result_z = z == 0 ? result_y * sz[0] : mad(result_y, sz[z], result_z);
+        result_z = z == 0 ? result_y * g.w[2][hz][0] : mad(result_y, g.w[2][hz][z], result_z);
     }
     return result_z;
-}
-
-// E components sit at (1/2,0,0),(0,1/2,0),(0,0,1/2); B at (0,1/2,1/2),
-// (1/2,0,1/2),(1/2,1/2,0) (fields/YeeCell.hpp:69-123).
-template <int SUPP, int TX, int TY, int TV>
-__device__ __forceinline__ Vec3 gatherE(const float* __restrict__ t, int cx, int cy, int cz, Vec3 pos) {
-    return Vec3{gather1<SUPP, TX, TY>(t, cx, cy, cz, pos, 0.5f, 0.0f, 0.0f),
-                gather1<SUPP, TX, TY>(t + TV, cx, cy, cz, pos, 0.0f, 0.5f, 0.0f),
-                gather1<SUPP, TX, TY>(t + 2 * TV, cx, cy, cz, pos, 0.0f, 0.0f, 0.5f)};
-}
-template <int SUPP, int TX, int TY, int TV>
-__device__ __forceinline__ Vec3 gatherB(const float* __restrict__ t, int cx, int cy, int cz, Vec3 pos) {
-    return Vec3{gather1<SUPP, TX, TY>(t, cx, cy, cz, pos, 0.0f, 0.5f, 0.5f),
-                gather1<SUPP, TX, TY>(t + TV, cx, cy, cz, pos, 0.5f, 0.0f, 0.5f),
-                gather1<SUPP, TX, TY>(t + 2 * TV, cx, cy, cz, pos, 0.5f, 0.5f, 0.0f)};
 }
 
 // ---------------------------------------------------------------------------
@@ -267,16 +378,15 @@ __device__ __forceinline__ Vec3 gatherB(const float* __restrict__ t, int cx, int
 // Velocity uses 1/sqrt like the reference CPU build
 // (thirdParty/alpaka/include/alpaka/math/Traits.hpp:729-734), not rsqrtf.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ float gammaOf(Vec3 mom, float mass, float c2) {
+__device__ __forceinline__ float gammaOf(Vec3 mom, float reciM2) {
     float const fMom2 = l2norm2(mom);
-    float const m2_c2_reci = 1.0f / (mass * mass * c2);
-    return sqrtf(1.0f + fMom2 * m2_c2_reci);
+    return sqrtAbove1(1.0f + fMom2 * reciM2);
 }
 
-__device__ __forceinline__ Vec3 velocityOf(Vec3 mom, float mass, float rc2) {
+__device__ __forceinline__ Vec3 velocityOf(Vec3 mom, float mass) {
     float const m0_2 = mass * mass;
     float const fMom2 = l2norm2(mom);
-    float const t = 1.0f / sqrtf(m0_2 + fMom2 * rc2);
+    float const t = recipOfRoot(sqrtf(m0_2 + fMom2));
     return Vec3{t * mom.x, t * mom.y, t * mom.z};
 }
 
@@ -399,8 +509,9 @@ __device__ __forceinline__ float pmlSigmaIntegral(const PmlDampArgs& p, int d, f
 // weighting and momentum scaled by exp(-integral), the weighting kept at
 // MIN_WEIGHTING or above
 __device__ __forceinline__ void pmlDamp(const PmlDampArgs& p, int d, int cell, float pos, float massPerWeight,
-                                        float rc2, float dt, float cellSize, Vec3& mom, float& w) {
-    Vec3 const vel = velocityOf(mom, massPerWeight * w, rc2);
+                                        float cellSize, Vec3& mom, float& w) {
+    constexpr float dt = 1.0f;
+    Vec3 const vel = velocityOf(mom, massPerWeight * w);
     float const v = d == 0 ? vel.x : (d == 1 ? vel.y : vel.z);
     float const current = static_cast<float>(cell) + pos;
     float const previous = current - v * dt / cellSize;
@@ -415,52 +526,65 @@ __device__ __forceinline__ void pmlDamp(const PmlDampArgs& p, int d, int cell, f
     w = damped;
 }
 
-struct PushConsts {
-    float cell[3];
-    float dt;
-    float c2;         // speedOfLight^2
-    float rc2;        // mue0*eps0
-    float c;          // speedOfLight
+// The units of time and speed are dt and c (simulation.unitless:428-479), so
+// the reference's factors dt, c, c^2 and mue0 eps0 are exactly 1 and are left
+// out below; a product with 1 rounds nothing.
+
+// The terms of a pusher that depend on the particle's mass and charge alone.
+struct WeightTerms {
+    float qom;      // charge / mass (Boris), factor / mass (Vay)
+    float reciM2;   // 1 / mass^2 (Gamma.hpp:28-38)
 };
 
 // Boris (particles/pusher/particlePusherBoris.hpp:41-90). Returns new momentum
-// and velocity; pos is advanced in place.
+// and velocity.
 __device__ __forceinline__ void pushBoris(Vec3 e, Vec3 b, Vec3& mom, Vec3& vel, float mass, float charge,
-                                          const PushConsts& k) {
-    float const QoM = charge / mass;
-    float const deltaT = k.dt;
+                                          const WeightTerms& k) {
     float const hq = 0.5f * charge;
-    Vec3 const mom_minus{mom.x + hq * e.x * deltaT, mom.y + hq * e.y * deltaT, mom.z + hq * e.z * deltaT};
-    float const gamma_reci = 1.0f / gammaOf(mom_minus, mass, k.c2);
-    float const hqm = 0.5f * QoM;
-    Vec3 const t{hqm * b.x * gamma_reci * deltaT, hqm * b.y * gamma_reci * deltaT, hqm * b.z * gamma_reci * deltaT};
-    float const sfac = 1.0f / (1.0f + l2norm2(t));
+    Vec3 const de{hq * e.x, hq * e.y, hq * e.z};
+    Vec3 const mom_minus{mom.x + de.x, mom.y + de.y, mom.z + de.z};
+    float const gamma_reci = recipOfRoot(gammaOf(mom_minus, k.reciM2));
+    float const hqm = 0.5f * k.qom;
+    Vec3 const t{hqm * b.x * gamma_reci, hqm * b.y * gamma_reci, hqm * b.z * gamma_reci};
+    float const sfac = recipAbove1(1.0f + l2norm2(t));
     Vec3 const s{2.0f * t.x * sfac, 2.0f * t.y * sfac, 2.0f * t.z * sfac};
     Vec3 const cp = cross(mom_minus, t);
     Vec3 const mom_prime{mom_minus.x + cp.x, mom_minus.y + cp.y, mom_minus.z + cp.z};
     Vec3 const cs = cross(mom_prime, s);
     Vec3 const mom_plus{mom_minus.x + cs.x, mom_minus.y + cs.y, mom_minus.z + cs.z};
-    mom = Vec3{mom_plus.x + hq * e.x * deltaT, mom_plus.y + hq * e.y * deltaT, mom_plus.z + hq * e.z * deltaT};
-    vel = velocityOf(mom, mass, k.rc2);
+    mom = Vec3{mom_plus.x + de.x, mom_plus.y + de.y, mom_plus.z + de.z};
+    vel = velocityOf(mom, mass);
+}
+
+// Vay's factor 0.5 charge dt (particlePusherVay.hpp:54)
+__device__ __forceinline__ float vayFactor(float charge) { return (float)(0.5 * (double)charge); }
+
+template <int PUSHER>
+__device__ __forceinline__ WeightTerms weightTerms(float mass, float charge) {
+    WeightTerms t;
+    t.reciM2 = 1.0f / (mass * mass);
+    t.qom = 0.0f;
+    if (PUSHER == PIC_PUSHER_BORIS) t.qom = charge / mass;
+    if (PUSHER == PIC_PUSHER_VAY) t.qom = vayFactor(charge) / mass;
+    return t;
 }
 
 // Vay (particles/pusher/particlePusherVay.hpp:42-111); the gamma root section
 // in FP64 as param/pusher.param:62 selects (sqrt_Vay = precision64Bit).
 __device__ __forceinline__ void pushVay(Vec3 e, Vec3 b, Vec3& mom, Vec3& vel, float mass, float charge,
-                                        const PushConsts& k) {
-    float const deltaT = k.dt;
-    float const factor = (float)(0.5 * (double)charge * (double)deltaT);
-    Vec3 const v_mh = velocityOf(mom, mass, k.rc2);
+                                        const WeightTerms& k) {
+    float const factor = vayFactor(charge);
+    Vec3 const v_mh = velocityOf(mom, mass);
     Vec3 const cvb = cross(v_mh, b);
     Vec3 const mom0{mom.x + factor * (e.x + cvb.x), mom.y + factor * (e.y + cvb.y), mom.z + factor * (e.z + cvb.z)};
     Vec3 const mp{mom0.x + factor * e.x, mom0.y + factor * e.y, mom0.z + factor * e.z};
-    float const gamma_prime = gammaOf(mp, mass, k.c2);
-    float const fm = factor / mass;
+    float const gamma_prime = gammaOf(mp, k.reciM2);
+    float const fm = k.qom;
     double const tx = (double)(fm * b.x), ty = (double)(fm * b.y), tz = (double)(fm * b.z);
     double dotp = (double)mp.x * tx;
     dotp += (double)mp.y * ty;
     dotp += (double)mp.z * tz;
-    double const u_star = dotp / (double)(k.c * mass);
+    double const u_star = dotp / (double)mass;
     double tau2 = tx * tx;
     tau2 += ty * ty;
     tau2 += tz * tz;
@@ -468,13 +592,13 @@ __device__ __forceinline__ void pushVay(Vec3 e, Vec3 b, Vec3& mom, Vec3& vel, fl
     double const gamma_ph = sqrt(0.5 * (sigma + sqrt(sigma * sigma + 4.0 * (tau2 + u_star * u_star))));
     double const rg = 1.0 / gamma_ph;
     Vec3 const t{(float)(tx * rg), (float)(ty * rg), (float)(tz * rg)};
-    float const s = 1.0f / (1.0f + l2norm2(t));
+    float const s = recipAbove1(1.0f + l2norm2(t));
     float dpt = mp.x * t.x;
     dpt += mp.y * t.y;
     dpt += mp.z * t.z;
     Vec3 const cpt = cross(mp, t);
     mom = Vec3{s * (mp.x + dpt * t.x + cpt.x), s * (mp.y + dpt * t.y + cpt.y), s * (mp.z + dpt * t.z + cpt.z)};
-    vel = velocityOf(mom, mass, k.rc2);
+    vel = velocityOf(mom, mass);
 }
 
 // ---------------------------------------------------------------------------
@@ -484,16 +608,15 @@ __device__ __forceinline__ void pushVay(Vec3 e, Vec3 b, Vec3& mom, Vec3& vel, fl
 // precision64Bit); Gamma<> stays FP32 (Gamma.def:31, Gamma.hpp:28-38).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void pushHigueraCary(Vec3 e, Vec3 b, Vec3& mom, Vec3& vel, float mass, float charge,
-                                                const PushConsts& k) {
-    float const deltaT = k.dt;
+                                                const WeightTerms& k) {
     float const hq = 0.5f * charge;
-    Vec3 const de{hq * e.x * deltaT, hq * e.y * deltaT, hq * e.z * deltaT};
+    Vec3 const de{hq * e.x, hq * e.y, hq * e.z};
     Vec3 const mmf{mom.x + de.x, mom.y + de.y, mom.z + de.z};
     double const mx = mmf.x, my = mmf.y, mz = mmf.z;
-    double const gamma_minus = (double)gammaOf(mmf, mass, k.c2);
-    double const tx = (double)(0.5f * b.x * charge * deltaT / mass);
-    double const ty = (double)(0.5f * b.y * charge * deltaT / mass);
-    double const tz = (double)(0.5f * b.z * charge * deltaT / mass);
+    double const gamma_minus = (double)gammaOf(mmf, k.reciM2);
+    double const tx = (double)(0.5f * b.x * charge / mass);
+    double const ty = (double)(0.5f * b.y * charge / mass);
+    double const tz = (double)(0.5f * b.z * charge / mass);
     double tau2 = tx * tx;
     tau2 += ty * ty;
     tau2 += tz * tz;
@@ -501,7 +624,7 @@ __device__ __forceinline__ void pushHigueraCary(Vec3 e, Vec3 b, Vec3& mom, Vec3&
     double dmt = mx * tx;
     dmt += my * ty;
     dmt += mz * tz;
-    double const u_star = dmt / (double)(mass * k.c);
+    double const u_star = dmt / (double)mass;
     double const gamma_plus = sqrt(0.5 * (sigma + sqrt(sigma * sigma + 4.0 * (tau2 + u_star * u_star))));
     double const t0 = tx / gamma_plus, t1 = ty / gamma_plus, t2 = tz / gamma_plus;
     double tt = t0 * t0;
@@ -516,7 +639,7 @@ __device__ __forceinline__ void pushHigueraCary(Vec3 e, Vec3 b, Vec3& mom, Vec3&
     double const pz = s * (mz + dm * t2 + (mx * t1 - my * t0));
     Vec3 const d2{(float)(py * t2 - pz * t1), (float)(pz * t0 - px * t2), (float)(px * t1 - py * t0)};
     mom = Vec3{(float)px + (de.x + d2.x), (float)py + (de.y + d2.y), (float)pz + (de.z + d2.z)};
-    vel = velocityOf(mom, mass, k.rc2);
+    vel = velocityOf(mom, mass);
 }
 
 // ---------------------------------------------------------------------------
@@ -545,27 +668,24 @@ __device__ __forceinline__ void moveAxes(float* pos, int* dir) {
 
 // the cell part of moveParticle: local cell index after the steps dir
 // (wrapped into the destination supercell) and the multiMask towards it
+// (MoveParticle.hpp:139-157: per axis the digit 0 stays, 1 up, 2 down of a
+// base-3 number, plus 1). The supercell's extents are powers of two: the bits
+// above an axis' coordinate are the supercell step (-1, 0 or 1), its low bits
+// the wrapped cell. Branch-free (about 25 integer instructions): nearly every
+// wave holds a particle that changes its cell, so a branch around the work
+// is taken anyway.
 __device__ __forceinline__ void cellAfterMove(int localIdx, const int* dir, int& newIdx, int& newMask) {
-    const int sc[3] = {SCX, SCY, SCZ};
-    newIdx = localIdx;
-    newMask = 1;
-    if ((dir[0] | dir[1] | dir[2]) != 0) {
-        int lc[3] = {localIdx % SCX, (localIdx / SCX) % SCY, localIdx / (SCX * SCY)};
-        int ex[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            lc[i] += dir[i];
-            ex[i] = (unsigned)lc[i] >= (unsigned)sc[i] ? dir[i] : 0;
-            lc[i] -= ex[i] * sc[i];
-        }
-        newIdx = lc[0] + SCX * (lc[1] + SCY * lc[2]);
-        int exchangeType = 1;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            newMask += (ex[i] == -1 ? 2 : ex[i]) * exchangeType;
-            exchangeType *= 3;
-        }
-    }
+    static_assert(SCX == 8 && SCY == 8 && SCZ == 4, "shifts and masks of the supercell's extents");
+    int const x = (localIdx & 7) + dir[0];
+    int const y = ((localIdx >> 3) & 7) + dir[1];
+    int const z = (localIdx >> 6) + dir[2];
+    newIdx = (x & 7) | ((y & 7) << 3) | ((z & 3) << 6);
+    // step e in {-1, 0, 1} to its digit: (e & 3) ^ (bit 1 of e)
+    int const ex = x >> 3, ey = y >> 3, ez = z >> 2;
+    int const digitX = (ex & 3) ^ ((ex >> 1) & 1);
+    int const digitY = (ey & 3) ^ ((ey >> 1) & 1);
+    int const digitZ = (ez & 3) ^ ((ez >> 1) & 1);
+    newMask = 1 + digitX + 3 * digitY + 9 * digitZ;
 }
 
 __device__ __forceinline__ void moveParticle(float* pos, int localIdx, int* dir, int& newIdx, int& newMask) {
@@ -628,7 +748,8 @@ __device__ __forceinline__ bool reflectParticle(const int* n, int reflect, int* 
 // ---------------------------------------------------------------------------
 struct DepositConsts {
     float cell[3];
-    float dt;
+    double rcell[3];  // 1 / cell and 1 / float(cell volume), for divExact
+    double rvol;
     float inv_vdt;  // 1 / float(V*dt)
     double jscale;  // 2^e
 };
@@ -769,13 +890,29 @@ struct Esirkepov {
     }
 
     __device__ __forceinline__ static Geometry geometry(Vec3 pos, Vec3 vel, const DepositConsts& k) {
-        float const dp[3] = {vel.x * k.dt / k.cell[0], vel.y * k.dt / k.cell[1], vel.z * k.dt / k.cell[2]};
+        float const dp[3] = {divExact(vel.x, k.rcell[0]), divExact(vel.y, k.rcell[1]), divExact(vel.z, k.rcell[2])};
         return geometryDp(pos, dp);
     }
 
-    // true when the move changes the shifted cell on some axis (the general form is needed)
-    __device__ __forceinline__ static bool changesCell(const Geometry& G) {
-        return ((G.st[0] | G.st[1] | G.st[2]) & 1) != 0;
+    // The geometry of a move that keeps its shifted cell on every axis; false
+    // when it does not. The values of geometryDp, with the cells compared and
+    // subtracted as the floats floor gives.
+    __device__ __forceinline__ static bool stayGeometry(Vec3 pos, const float* dp, Geometry& G) {
+        constexpr bool isEven = (SUPP % 2) == 0;
+        float const np[3] = {pos.x, pos.y, pos.z};
+        bool stays = true;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            float const p0 = np[d] - dp[d], p1 = np[d];
+            float const s = isEven ? floorf(p0) : floorf(p0 + 0.5f);
+            float const e = isEven ? floorf(p1) : floorf(p1 + 0.5f);
+            stays = stays && s == e;
+            G.gs[d] = (int)e;
+            G.st[d] = 6;
+            G.p0[d] = p0 - e;
+            G.p1[d] = p1 - e;
+        }
+        return stays;
     }
 
     // Shape values of one axis for a particle whose start and end lie in the
@@ -831,7 +968,7 @@ struct Esirkepov {
         }
     }
 
-    // Deposit of a particle with changesCell(G) == false: the contributions
+    // Deposit of a particle with stayGeometry: the contributions
     // of depositGeometry<..., false>, bit for bit, with each axis' shape
     // values formed once.
     // tile element of component c for the cell (x, y, z) in tile coordinates
@@ -860,7 +997,7 @@ struct Esirkepov {
     // Deposit one particle. (cx,cy,cz) is the particle's cell in J-tile
     // coordinates, G its move geometry. Tile layout: component-major planes
     // of TV elements, [z][y][x] with pitches TX, TX*TY. GENERAL = false only
-    // for a geometry with changesCell(G) == false.
+    // for a geometry with stayGeometry.
     template <class TG, bool GENERAL>
     __device__ __forceinline__ static void depositGeometry(unsigned long long* __restrict__ jt, int cx, int cy, int cz,
                                                            const Geometry& G, float charge, const DepositConsts& k) {
@@ -951,16 +1088,16 @@ struct EmZ {
             float const q0[3] = {a[1], a[2], a[0]};
             float const q1[3] = {b[1], b[2], b[0]};
             cpt1D<TG::py(0), TG::pz(0), 1>(Esirkepov<SUPP>::template cornerOf<TG>(jt, 0, x, y, z), q0, q1,
-                                           k.cell[0] * chargeDensity / k.dt, k.jscale);
+                                           k.cell[0] * chargeDensity, k.jscale);
         }
         {  // J_y: rotation (2,0,1)
             float const q0[3] = {a[2], a[0], a[1]};
             float const q1[3] = {b[2], b[0], b[1]};
             cpt1D<TG::pz(1), 1, TG::py(1)>(Esirkepov<SUPP>::template cornerOf<TG>(jt, 1, x, y, z), q0, q1,
-                                           k.cell[1] * chargeDensity / k.dt, k.jscale);
+                                           k.cell[1] * chargeDensity, k.jscale);
         }
         cpt1D<1, TG::py(2), TG::pz(2)>(Esirkepov<SUPP>::template cornerOf<TG>(jt, 2, x, y, z), a, b,
-                                       k.cell[2] * chargeDensity / k.dt, k.jscale);  // J_z
+                                       k.cell[2] * chargeDensity, k.jscale);  // J_z
     }
 
     // Deposit one particle: (cx,cy,cz) its cell in J-tile coordinates, pos
@@ -968,7 +1105,7 @@ struct EmZ {
     template <class TG>
     __device__ __forceinline__ static void deposit(unsigned long long* __restrict__ jt, int cx, int cy, int cz, Vec3 pos,
                                                    Vec3 vel, float charge, const DepositConsts& k) {
-        float const dp[3] = {vel.x * k.dt / k.cell[0], vel.y * k.dt / k.cell[1], vel.z * k.dt / k.cell[2]};
+        float const dp[3] = {divExact(vel.x, k.rcell[0]), divExact(vel.y, k.rcell[1]), divExact(vel.z, k.rcell[2])};
         depositDp<TG>(jt, cx, cy, cz, pos, dp, charge, k);
     }
 
@@ -993,7 +1130,7 @@ struct EmZ {
                 relay[d] = s0[d] == s1[d] ? p1[d] : (float)(s0[d] + s1[d]) / 2.0f;
             }
         }
-        float const chargeDensity = charge / (k.cell[0] * k.cell[1] * k.cell[2]);
+        float const chargeDensity = divExact(charge, k.rvol);  // charge / (cell_x cell_y cell_z)
         float a[3], b[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {

@@ -31,7 +31,6 @@ struct SpeciesDev {
     const uint64_t* base;
     const uint32_t* capOf;
     int32_t cap;         // the largest capacity of a supercell (slots)
-    int32_t lists;       // 1: the push kernel builds the leaver lists of this species
     int32_t reflect;     // bit d: particles crossing an open border of axis d are reflected
     float mass;          // frame::getMass()
     float charge;        // frame::getCharge()
@@ -91,7 +90,8 @@ struct PushArgs {
     const float* B[3];
     float* J[3];
     float cell[3];
-    float dt, c, c2, rc2;
+    double rcell[3];  // 1 / cell and 1 / float(cell volume), for divExact
+    double rvol;
     float inv_vdt;
     double jscale;    // 2^e
     double jinv;      // 2^-e
@@ -156,10 +156,8 @@ struct RunMove {
 hipError_t launchMoveRuns(void* dst, const void* src, uint32_t bytesPerSlot, const RunMove* moves, int n,
                           hipStream_t s);
 hipError_t launchCollect(const GridDev& g, const SpeciesDev& sp, hipStream_t s);
-// the push kernel builds leaver lists for species with at most this many slots per supercell
 constexpr int kPushThreadsPerBlock = 512;
 constexpr int kPushMaxIters = 32;  // bits of a leaveBits word
-constexpr int kListMaxSlots = kPushThreadsPerBlock * kPushMaxIters;
 hipError_t launchFill(float* p, size_t n, float v, hipStream_t s);
 // J = 0 at the start of a step (skipped while halted)
 hipError_t launchCurrentReset(const GridDev& g, float* const J[3], size_t n, hipStream_t s);

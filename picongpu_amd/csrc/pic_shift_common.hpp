@@ -9,6 +9,17 @@ namespace pic {
 
 __device__ __forceinline__ unsigned long long laneMaskLt() { return (1ull << (threadIdx.x & 63)) - 1ull; }
 
+// inclusive prefix sum over the 64 lanes of a wave
+__device__ __forceinline__ uint32_t waveInclusiveScan(uint32_t v) {
+    int const lane = threadIdx.x & 63;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        uint32_t const t = __shfl_up(v, o);
+        if (lane >= o) v += t;
+    }
+    return v;
+}
+
 // Exclusive rank of `pred` in thread order within one block-wide chunk;
 // *total receives the chunk's count. NW = waves per block.
 template <int NW>

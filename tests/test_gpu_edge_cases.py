@@ -96,6 +96,19 @@ def test_supercell_beyond_the_leaver_lists():
     assert int(out.sum()) == sum(counts)
 
 
+@pytest.mark.parametrize("count,u", [(700, 0.3), (5000, 2.0), (14000, 2.0)])
+def test_leaver_list_sizes(count, u):
+    """Leavers of one supercell within one round of the workgroup (about 80),
+    over several rounds (about 1,200) and beyond the list the push keeps in
+    LDS (about 3,400 of 2,048), next to small supercells; bit-exact."""
+    st = thermal(frames=66)
+    counts = [count, 900, 0, 513, 1, 64, 0, 130, 0, 0, 65, 2]
+    print(f"case leavers of {count} particles, u={u}", flush=True)
+    cells, pos, mom, w = crafted(st, counts, seed=21, u=u)
+    out = run_pair(st, cells, pos, mom, w, frames=66, nsteps=2)
+    assert int(out.sum()) == sum(counts)
+
+
 def test_cell_border_positions():
     """In-cell positions exactly on the cell borders (0, -0, the largest
     float below 1) and at 1/2, moved across the borders in both directions."""

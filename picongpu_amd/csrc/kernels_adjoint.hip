@@ -22,68 +22,83 @@
 
 namespace pic {
 
+// v in [-n, 2n) wrapped into [0, n)
 __device__ __forceinline__ int wrapI(int v, int n) {
-    v %= n;
-    return v < 0 ? v + n : v;
+    v = v < 0 ? v + n : v;
+    return v >= n ? v - n : v;
 }
 
 __device__ __forceinline__ size_t gidx(const GridDev& g, int x, int y, int z) {
     return (size_t)wrapI(x, g.nx) + (size_t)g.nx * ((size_t)wrapI(y, g.ny) + (size_t)g.ny * (size_t)wrapI(z, g.nz));
 }
 
-// Signed periodic difference in [-n/2, n/2).
+// Signed periodic difference in [-n/2, n/2) of two cells of [0, n).
 __device__ __forceinline__ int wrapDiff(int d, int n) {
-    d %= n;
     if (d >= (n + 1) / 2) d -= n;
     if (d < -(n / 2)) d += n;
     return d;
 }
 
-// Window of the grid around one block's particles: accumulation goes to LDS
-// when the window holds every node the block's particles touch, and the
-// window is added to global memory once at the end of the block.
+// Window of the grid around one block's particles, held in LDS: the fields the
+// block gathers from and its accumulators. A particle whose nodes it does not
+// hold goes to global memory instead.
+constexpr int kWinLo = 1, kWinHi = 2;  // nodes c-1 .. c+2 around a particle's cell
 struct BlockWindow {
     int ref[3];  // reference cell (the block's first particle)
     int lo[3];   // window origin relative to ref
     int ext[3];  // window extent in cells
     int vol;
-    bool lds;
+    float rx, ry;  // 1 / ext of x and y, for the element's coordinates
 };
 
-// Every thread of the block calls this (it synchronises). c: the particle's
-// cell, active: whether the thread has a particle; nodes c-LO .. c+HI per
-// axis must fit. rel receives c relative to the reference cell.
-template <int LO, int HI>
+// minimum over the wave of two int16 per word
+__device__ __forceinline__ int waveMinPair(int v) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        int const t = __shfl_xor(v, o);
+        int const a = min((int)(short)v, (int)(short)t);
+        int const b = min(v >> 16, t >> 16);
+        v = (a & 0xffff) | (b << 16);
+    }
+    return v;
+}
+
+// Every thread of the block (NT threads) calls this (it synchronises). c: the
+// particle's cell, active: whether the thread has a particle. rel receives c
+// relative to the reference cell. sBox: 3 + 3 words per wave.
+template <int NT>
 __device__ __forceinline__ BlockWindow blockWindow(const GridDev& g, bool active, const int* c, int* rel, int* sBox,
                                                    int capCells) {
     int const n[3] = {g.nx, g.ny, g.nz};
     if (threadIdx.x == 0) {
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            sBox[d] = c[d];
-            sBox[3 + d] = 0x7fffffff;
-            sBox[6 + d] = -0x7fffffff;
-        }
+        for (int d = 0; d < 3; ++d) sBox[d] = c[d];
     }
     __syncthreads();
     BlockWindow w;
+    int box[3];  // (rel, -rel) as two int16: their minima are the minimum and minus the maximum
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         w.ref[d] = sBox[d];
         rel[d] = active ? wrapDiff(c[d] - w.ref[d], n[d]) : 0;
+        int const r = max(-32000, min(32000, rel[d]));
+        box[d] = waveMinPair((r & 0xffff) | (-r << 16));
     }
-    if (active) {
+    if ((threadIdx.x & 63) == 0) {
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            atomicMin(&sBox[3 + d], rel[d]);
-            atomicMax(&sBox[6 + d], rel[d]);
-        }
+        for (int d = 0; d < 3; ++d) sBox[3 + (threadIdx.x >> 6) * 3 + d] = box[d];
     }
     __syncthreads();
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        w.lo[d] = sBox[3 + d] - LO;
-        w.ext[d] = sBox[6 + d] + HI - w.lo[d] + 1;
+        int lo = 0x7fff, hi = 0x7fff;
+        for (int v = 0; v < NT / 64; ++v) {
+            int const b = sBox[3 + v * 3 + d];
+            lo = min(lo, (int)(short)b);
+            hi = min(hi, b >> 16);
+        }
+        w.lo[d] = __builtin_amdgcn_readfirstlane(lo - kWinLo);
+        w.ext[d] = __builtin_amdgcn_readfirstlane(-hi + kWinHi - (lo - kWinLo) + 1);
     }
     // a box larger than the LDS capacity is trimmed, one cell at a time from
     // alternating ends of its longest axis; particles whose nodes then leave
@@ -101,49 +116,100 @@ __device__ __forceinline__ BlockWindow blockWindow(const GridDev& g, bool active
         }
     }
     w.vol = w.ext[0] * w.ext[1] * w.ext[2];
-    w.lds = true;
-    __syncthreads();  // sBox is reused by the next call
+    w.rx = 1.0f / (float)w.ext[0];
+    w.ry = 1.0f / (float)w.ext[1];
     return w;
 }
 
-// whether the nodes rel-LO .. rel+HI of a particle lie in the window
-template <int LO, int HI>
-__device__ __forceinline__ bool windowHolds(const BlockWindow& w, const int* rel) {
+// whether the nodes at .. at + LAST (relative to the reference cell) lie in the window
+template <int LAST>
+__device__ __forceinline__ bool windowHolds(const BlockWindow& w, const int* at) {
     bool in = true;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) in = in && rel[d] - LO >= w.lo[d] && rel[d] + HI < w.lo[d] + w.ext[d];
+    for (int d = 0; d < 3; ++d) in = in && at[d] >= w.lo[d] && at[d] + LAST < w.lo[d] + w.ext[d];
     return in;
 }
+// the same for every node a particle of cell rel can touch in a step
+__device__ __forceinline__ bool windowHoldsCell(const BlockWindow& w, const int* rel) {
+    int const low[3] = {rel[0] - kWinLo, rel[1] - kWinLo, rel[2] - kWinLo};
+    return windowHolds<kWinLo + kWinHi>(w, low);
+}
 
-// global linear index of window element e (x fastest within the window)
+// global linear index of window element e < vol (x fastest within the
+// window). The quotients by the extents are exact: e + 1/2 lies at least
+// 1/(2 ext) from a multiple, far above the product's rounding (vol < 2^12).
 __device__ __forceinline__ uint32_t windowToGlobal(const GridDev& g, const BlockWindow& w, int e) {
-    int const lx = e % w.ext[0];
-    int const ly = (e / w.ext[0]) % w.ext[1];
-    int const lz = e / (w.ext[0] * w.ext[1]);
+    int const row = (int)(((float)e + 0.5f) * w.rx);
+    int const lx = e - row * w.ext[0];
+    int const lz = (int)(((float)row + 0.5f) * w.ry);
+    int const ly = row - lz * w.ext[1];
     return (uint32_t)wrapI(w.ref[0] + w.lo[0] + lx, g.nx) +
            (uint32_t)g.nx * ((uint32_t)wrapI(w.ref[1] + w.lo[1] + ly, g.ny) +
                              (uint32_t)g.ny * (uint32_t)wrapI(w.ref[2] + w.lo[2] + lz, g.nz));
 }
 
+// The window's six field components, plane by plane in sF (vol floats each).
+template <int NT>
+__device__ __forceinline__ void stageFields(const GridDev& g, const BlockWindow& w, const float* const* E,
+                                            const float* const* B, float* sF) {
+    for (int e = threadIdx.x; e < w.vol; e += NT) {
+        uint32_t const at = windowToGlobal(g, w, e);
+        float v[6];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            v[c] = E[c][at];
+            v[3 + c] = B[c][at];
+        }
+#pragma unroll
+        for (int c = 0; c < 6; ++c) sF[c * w.vol + e] = v[c];
+    }
+}
+
+// Offsets of a particle's nodes: per axis the nodes first-1+{0,1,2} times the
+// axis' stride, in the window (LDS) or on the grid.
+struct NodeOffsets {
+    uint32_t o[3][3];  // cells c-1, c, c+1
+};
+__device__ __forceinline__ NodeOffsets windowOffsets(const BlockWindow& w, const int* rel) {
+    NodeOffsets n;
+    uint32_t const stride[3] = {1u, (uint32_t)w.ext[0], (uint32_t)(w.ext[0] * w.ext[1])};
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int m = 0; m < 3; ++m) n.o[d][m] = (uint32_t)(rel[d] - 1 + m - w.lo[d]) * stride[d];
+    return n;
+}
+__device__ __forceinline__ NodeOffsets gridOffsets(const GridDev& g, const int* c) {
+    NodeOffsets n;
+    int const ext[3] = {g.nx, g.ny, g.nz};
+    uint32_t const stride[3] = {1u, (uint32_t)g.nx, (uint32_t)g.nx * (uint32_t)g.ny};
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int m = 0; m < 3; ++m) n.o[d][m] = (uint32_t)wrapI(c[d] - 1 + m, ext[d]) * stride[d];
+    return n;
+}
+
 // ---------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------
-// FieldToParticleInterpolation<CIC> on global memory: same arithmetic as gather1<2>.
-__device__ __forceinline__ float gatherGlobalCIC(const float* __restrict__ F, const GridDev& g, int cx, int cy, int cz,
-                                                 Vec3 pos, float fx, float fy, float fz) {
-    float p[3] = {pos.x, pos.y, pos.z};
-    float const f[3] = {fx, fy, fz};
-    int is[3];
+// FieldToParticleInterpolation<CIC> of component C (yeeHalf) from a plane of
+// the window or of the grid: same arithmetic as gather1<2>. A half position's
+// first node is the cell below or the cell itself, an integer one's the cell.
+template <int C, typename Plane>
+__device__ __forceinline__ float gatherCIC(Plane F, const NodeOffsets& n, Vec3 pos) {
+    float const q[3] = {pos.x, pos.y, pos.z};
+    float w[3][2];
+    uint32_t o[3][2];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        float const v_pos = p[d] - f[d] - 0.5f;
-        is[d] = v_pos >= -0.5f ? 0 : -1;
-        p[d] = v_pos - (float)is[d] + 0.5f;
+        float const v = yeeHalf(C, d) ? q[d] - 0.5f - 0.5f : q[d] - 0.5f;
+        bool const below = yeeHalf(C, d) && !(v >= -0.5f);
+        float const p = v - (below ? -1.0f : 0.0f) + 0.5f;
+        Shape<2>::onSupport(p, w[d]);
+        o[d][0] = below ? n.o[d][0] : n.o[d][1];
+        o[d][1] = below ? n.o[d][1] : n.o[d][2];
     }
-    float sx[2], sy[2], sz[2];
-    Shape<2>::onSupport(p[0], sx);
-    Shape<2>::onSupport(p[1], sy);
-    Shape<2>::onSupport(p[2], sz);
     // partial sums start at their first term and add the others as
     // multiply-adds, as gather1
     float result_z = 0.0f;
@@ -152,16 +218,14 @@ __device__ __forceinline__ float gatherGlobalCIC(const float* __restrict__ F, co
         float result_y = 0.0f;
 #pragma unroll
         for (int y = 0; y < 2; ++y) {
-            float const result_x = mad(F[gidx(g, cx + is[0] + 1, cy + is[1] + y, cz + is[2] + z)], sx[1],
-                                       F[gidx(g, cx + is[0], cy + is[1] + y, cz + is[2] + z)] * sx[0]);
-            result_y = y == 0 ? result_x * sy[0] : mad(result_x, sy[y], result_y);
+            uint32_t const row = o[1][y] + o[2][z];
+            float const result_x = mad(F[row + o[0][1]], w[0][1], F[row + o[0][0]] * w[0][0]);
+            result_y = y == 0 ? result_x * w[1][0] : mad(result_x, w[1][y], result_y);
         }
-        result_z = z == 0 ? result_y * sz[0] : mad(result_y, sz[z], result_z);
+        result_z = z == 0 ? result_y * w[2][0] : mad(result_y, w[2][z], result_z);
     }
     return result_z;
 }
-
-
 
 // Wrapped offsets of the nodes b, b+1, b+2 along one axis, times the axis stride.
 __device__ __forceinline__ void axisOffsets(int b, int n, uint32_t stride, uint32_t* o) {
@@ -221,16 +285,15 @@ __device__ __forceinline__ void cptGlobal(unsigned long long* __restrict__ J, co
 
 // Esirkepov<CIC> deposit of one particle (Esirkepov.hpp:61-242, the float
 // arithmetic of Esirkepov<2>::deposit) into int64 accumulators: the block's
-// LDS window (LDS = true; rel is the cell relative to the window reference) or
-// global memory. The particle sits in global cell c at in-cell position pos
-// after its move.
-template <bool LDS>
+// LDS window where it holds the particle's nodes, else global memory. The
+// particle sits in global cell c (rel relative to the window's reference) at
+// in-cell position pos after its move.
 __device__ __forceinline__ void depositCIC(const DiffArgs& a, unsigned long long* sJ, const BlockWindow& w,
                                            const int* c, const int* rel, Vec3 pos, Vec3 vel, float charge) {
     float const np[3] = {pos.x, pos.y, pos.z};
-    float const dp[3] = {vel.x * a.dt / a.cell[0], vel.y * a.dt / a.cell[1], vel.z * a.dt / a.cell[2]};
+    float const dp[3] = {divExact(vel.x, a.rcell[0]), divExact(vel.y, a.rcell[1]), divExact(vel.z, a.rcell[2])};
     float p0[3], p1[3];
-    int gs[3], st[3];
+    int st[3], at[3], gs[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         p0[d] = np[d] - dp[d];
@@ -241,110 +304,117 @@ __device__ __forceinline__ void depositCIC(const DiffArgs& a, unsigned long long
         st[d] = (gs[d] == iS ? 2 : 0) | (gs[d] == iE ? 4 : 0) | (iS != iE ? 1 : 0);
         p0[d] -= (float)gs[d];
         p1[d] -= (float)gs[d];
+        at[d] = rel[d] + gs[d];
     }
+    float const csd[3] = {charge * a.inv_vdt * a.cell[0], charge * a.inv_vdt * a.cell[1], charge * a.inv_vdt * a.cell[2]};
+    // rotations of Esirkepov.hpp:106-124: J_x (i,j,k) = (y,z,x), J_y (z,x,y), J_z (x,y,z)
     uint32_t off[3][3];
-    unsigned long long* J[3];
-    if (LDS) {
+    if (windowHolds<2>(w, at)) {
         uint32_t const ls[3] = {1u, (uint32_t)w.ext[0], (uint32_t)(w.ext[0] * w.ext[1])};
 #pragma unroll
         for (int d = 0; d < 3; ++d)
 #pragma unroll
-            for (int m = 0; m < 3; ++m) off[d][m] = (uint32_t)(rel[d] + gs[d] + m - w.lo[d]) * ls[d];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) J[d] = sJ + d * w.vol;
-    } else {
+            for (int m = 0; m < 3; ++m) off[d][m] = (uint32_t)(at[d] + m - w.lo[d]) * ls[d];
+        cptGlobal<1, 2, 0, true>(sJ, off, p0, p1, st, csd[0], a.jscale);
+        cptGlobal<2, 0, 1, true>(sJ + w.vol, off, p0, p1, st, csd[1], a.jscale);
+        cptGlobal<0, 1, 2, true>(sJ + 2 * w.vol, off, p0, p1, st, csd[2], a.jscale);
+    } else {  // outside a trimmed window, or a position that is no particle's (non-finite data)
         axisOffsets(c[0] + gs[0], a.g.nx, 1u, off[0]);
         axisOffsets(c[1] + gs[1], a.g.ny, (uint32_t)a.g.nx, off[1]);
         axisOffsets(c[2] + gs[2], a.g.nz, (uint32_t)a.g.nx * (uint32_t)a.g.ny, off[2]);
-#pragma unroll
-        for (int d = 0; d < 3; ++d) J[d] = a.Jfix[d];
+        cptGlobal<1, 2, 0, false>(a.Jfix[0], off, p0, p1, st, csd[0], a.jscale);
+        cptGlobal<2, 0, 1, false>(a.Jfix[1], off, p0, p1, st, csd[1], a.jscale);
+        cptGlobal<0, 1, 2, false>(a.Jfix[2], off, p0, p1, st, csd[2], a.jscale);
     }
-    // rotations of Esirkepov.hpp:106-124: J_x (i,j,k) = (y,z,x), J_y (z,x,y), J_z (x,y,z)
-    cptGlobal<1, 2, 0, LDS>(J[0], off, p0, p1, st, charge * a.inv_vdt * a.cell[0], a.jscale);
-    cptGlobal<2, 0, 1, LDS>(J[1], off, p0, p1, st, charge * a.inv_vdt * a.cell[1], a.jscale);
-    cptGlobal<0, 1, 2, LDS>(J[2], off, p0, p1, st, charge * a.inv_vdt * a.cell[2], a.jscale);
 }
 
-// int64 LDS window of the forward deposit: 3 components of this many cells
-constexpr int kDiffLdsCells = 1024;
-
-__global__ __launch_bounds__(256) void kDiffPush(DiffArgs a, DiffParticles P) {
-    __shared__ unsigned long long sJ[3 * kDiffLdsCells];
-    __shared__ int sBox[9];
-    int64_t const i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    bool const active = i < P.n;
+// One particle's step: the gather from the window (LDS) or the grid, the push
+// and the deposit. c: its cell, rel relative to the window's reference.
+template <bool LDS>
+__device__ __forceinline__ void diffParticle(const DiffArgs& a, const DiffParticles& P, int64_t i, const int* c,
+                                             const int* rel, const BlockWindow& win, const float* sF,
+                                             unsigned long long* sJ) {
     int64_t const n = P.n;
-    int nc[3] = {0, 0, 0};
-    float p[3] = {0.0f, 0.0f, 0.0f};
-    Vec3 vel{0.0f, 0.0f, 0.0f};
-    float charge = 0.0f;
-    if (active) {
-        int const cx = P.cell[i], cy = P.cell[n + i], cz = P.cell[2 * n + i];
-        Vec3 const pos{P.pos[i], P.pos[n + i], P.pos[2 * n + i]};
-        Vec3 mom{P.mom[i], P.mom[n + i], P.mom[2 * n + i]};
-        float const w = P.w[i];
-        float const mass = a.mass * w;
-        charge = a.charge * w;
-        Vec3 const e{gatherGlobalCIC(a.E[0], a.g, cx, cy, cz, pos, 0.5f, 0.0f, 0.0f),
-                     gatherGlobalCIC(a.E[1], a.g, cx, cy, cz, pos, 0.0f, 0.5f, 0.0f),
-                     gatherGlobalCIC(a.E[2], a.g, cx, cy, cz, pos, 0.0f, 0.0f, 0.5f)};
-        Vec3 const b{gatherGlobalCIC(a.B[0], a.g, cx, cy, cz, pos, 0.0f, 0.5f, 0.5f),
-                     gatherGlobalCIC(a.B[1], a.g, cx, cy, cz, pos, 0.5f, 0.0f, 0.5f),
-                     gatherGlobalCIC(a.B[2], a.g, cx, cy, cz, pos, 0.5f, 0.5f, 0.0f)};
-        pushBoris(e, b, mom, vel, mass, charge, weightTerms<PIC_PUSHER_BORIS>(mass, charge));
-        p[0] = pos.x;
-        p[1] = pos.y;
-        p[2] = pos.z;
-        p[0] += (vel.x * a.dt) / a.cell[0];
-        p[1] += (vel.y * a.dt) / a.cell[1];
-        p[2] += (vel.z * a.dt) / a.cell[2];
-        int dir[3], idxUnused, maskUnused;
-        moveParticle(p, 0, dir, idxUnused, maskUnused);
-        nc[0] = wrapI(cx + dir[0], a.g.nx);
-        nc[1] = wrapI(cy + dir[1], a.g.ny);
-        nc[2] = wrapI(cz + dir[2], a.g.nz);
-        P.cellOut[i] = nc[0];
-        P.cellOut[n + i] = nc[1];
-        P.cellOut[2 * n + i] = nc[2];
-        P.posOut[i] = p[0];
-        P.posOut[n + i] = p[1];
-        P.posOut[2 * n + i] = p[2];
-        P.momOut[i] = mom.x;
-        P.momOut[n + i] = mom.y;
-        P.momOut[2 * n + i] = mom.z;
-    }
-    // deposit nodes of a particle in cell c: c-1 .. c+2 per axis
-    int rel[3];
-    BlockWindow const win = blockWindow<1, 2>(a.g, active, nc, rel, sBox, kDiffLdsCells);
-    if (win.lds) {
-        for (int e = threadIdx.x; e < 3 * win.vol; e += blockDim.x) sJ[e] = 0ull;
-        __syncthreads();
-        if (active) {
-            // nodes c-1..c+2 lie in the window when the cell is held and the
-            // start and end positions lie in (-1,2) and [0,1); any other
-            // particle (outside a trimmed window, a position rounded onto the
-            // cell edge, non-finite data) deposits to global memory with
-            // wrapped indices instead
-            bool fits = windowHolds<1, 2>(win, rel);
+    Vec3 const pos{P.pos[i], P.pos[n + i], P.pos[2 * n + i]};
+    Vec3 mom{P.mom[i], P.mom[n + i], P.mom[2 * n + i]};
+    float const w = P.w[i];
+    float const mass = a.mass * w;
+    float const charge = a.charge * w;
+    NodeOffsets const o = LDS ? windowOffsets(win, rel) : gridOffsets(a.g, c);
+    auto plane = [&](int k) { return LDS ? sF + k * win.vol : (k < 3 ? a.E[k] : a.B[k - 3]); };
+    Vec3 const e{gatherCIC<0>(plane(0), o, pos), gatherCIC<1>(plane(1), o, pos), gatherCIC<2>(plane(2), o, pos)};
+    Vec3 const b{gatherCIC<3>(plane(3), o, pos), gatherCIC<4>(plane(4), o, pos), gatherCIC<5>(plane(5), o, pos)};
+    Vec3 vel;
+    pushBoris(e, b, mom, vel, mass, charge, weightTerms<PIC_PUSHER_BORIS>(mass, charge));
+    float p[3] = {pos.x, pos.y, pos.z};
+    p[0] += divExact(vel.x, a.rcell[0]);
+    p[1] += divExact(vel.y, a.rcell[1]);
+    p[2] += divExact(vel.z, a.rcell[2]);
+    int dir[3];
+    moveAxes(p, dir);
+    int const nc[3] = {wrapI(c[0] + dir[0], a.g.nx), wrapI(c[1] + dir[1], a.g.ny), wrapI(c[2] + dir[2], a.g.nz)};
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                float const vd = d == 0 ? vel.x : (d == 1 ? vel.y : vel.z);
-                float const p0 = p[d] - vd * a.dt / a.cell[d];
-                fits = fits && p[d] >= 0.0f && p[d] < 1.0f && p0 > -1.0f && p0 < 2.0f;
-            }
-            if (fits)
-                depositCIC<true>(a, sJ, win, nc, rel, Vec3{p[0], p[1], p[2]}, vel, charge);
-            else
-                depositCIC<false>(a, sJ, win, nc, rel, Vec3{p[0], p[1], p[2]}, vel, charge);
+    for (int d = 0; d < 3; ++d) {
+        P.cellOut[d * n + i] = nc[d];
+        P.posOut[d * n + i] = p[d];
+    }
+    P.momOut[i] = mom.x;
+    P.momOut[n + i] = mom.y;
+    P.momOut[2 * n + i] = mom.z;
+    int const nrel[3] = {rel[0] + dir[0], rel[1] + dir[1], rel[2] + dir[2]};
+    depositCIC(a, sJ, win, nc, nrel, Vec3{p[0], p[1], p[2]}, vel, charge);
+}
+
+// One thread per particle. The block's window holds the six field components
+// (gathered from LDS) and the current's accumulators; CAP cells of it. The
+// particles it does not hold (they drift up to half a cell a step between
+// two sorts) are listed and done afterwards by full waves: in place, every
+// wave with one of them ran both forms.
+template <int NT, int CAP>
+__global__ __launch_bounds__(NT) void kDiffPush(DiffArgs a, DiffParticles P) {
+    __shared__ unsigned long long sJ[3 * CAP];
+    __shared__ float sF[6 * CAP];
+    __shared__ int sBox[3 + 3 * NT / 64];
+    __shared__ uint16_t sOut[NT];
+    __shared__ int sOutN;
+    int64_t const first = (int64_t)blockIdx.x * NT;
+    int64_t const i = first + threadIdx.x;
+    bool const active = i < P.n;
+    int c[3] = {0, 0, 0}, rel[3];
+    if (active) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) c[d] = P.cell[d * P.n + i];
+    }
+    if (threadIdx.x == 0) sOutN = 0;
+    BlockWindow const win = blockWindow<NT>(a.g, active, c, rel, sBox, CAP);
+    stageFields<NT>(a.g, win, a.E, a.B, sF);
+    for (int e = threadIdx.x; e < 3 * win.vol; e += NT) sJ[e] = 0ull;
+    __syncthreads();
+    if (active) {
+        if (windowHoldsCell(win, rel))
+            diffParticle<true>(a, P, i, c, rel, win, sF, sJ);
+        else
+            sOut[atomicAdd(&sOutN, 1)] = (uint16_t)threadIdx.x;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < sOutN) {
+        int64_t const k = first + sOut[threadIdx.x];
+        int cell[3], at[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            cell[d] = P.cell[d * P.n + k];
+            at[d] = wrapDiff(cell[d] - win.ref[d], d == 0 ? a.g.nx : (d == 1 ? a.g.ny : a.g.nz));
         }
-        __syncthreads();
-        for (int e = threadIdx.x; e < 3 * win.vol; e += blockDim.x) {
-            unsigned long long const v = sJ[e];
-            if (v != 0ull) {
-                int const comp = e / win.vol;
-                __hip_atomic_fetch_add(a.Jfix[comp] + windowToGlobal(a.g, win, e - comp * win.vol), v,
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
+        diffParticle<false>(a, P, k, cell, at, win, sF, sJ);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < win.vol; e += NT) {
+        uint32_t const at = windowToGlobal(a.g, win, e);
+#pragma unroll
+        for (int comp = 0; comp < 3; ++comp) {
+            unsigned long long const v = sJ[comp * win.vol + e];
+            if (v != 0ull)
+                __hip_atomic_fetch_add(a.Jfix[comp] + at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }
@@ -422,11 +492,6 @@ __device__ __forceinline__ R opaque(R x) {
     asm volatile("" : "+v"(x));
     return x;
 }
-__device__ __forceinline__ int opaqueI(int x) {
-    asm volatile("" : "+v"(x));
-    return x;
-}
-
 // Phase boundary: no instruction is scheduled across it, so each phase's
 // loads and temporaries stay within the phase.
 __device__ __forceinline__ void phaseBarrier() {
@@ -454,30 +519,27 @@ struct YeeOff {
     }
 };
 
-// Node offsets and CIC weights of the interpolation of one Yee component at
-// in-cell position r of cell c (ShiftCoordinateSystem for an even support).
+// CIC weights of the interpolation of one Yee component at in-cell position
+// r (ShiftCoordinateSystem for an even support) and its nodes among c-1 .. c+1.
 template <int FIELD, int COMP, typename R>
-__device__ __forceinline__ void interpNodes(const GridDev& g, const int* c, const R* r, uint32_t (&o)[3][2],
-                                            R (&w)[3][2]) {
-    int const n[3] = {g.nx, g.ny, g.nz};
-    uint32_t const stride[3] = {1u, (uint32_t)g.nx, (uint32_t)g.nx * (uint32_t)g.ny};
+__device__ __forceinline__ void interpNodes(const NodeOffsets& n, const R* r, uint32_t (&o)[3][2], R (&w)[3][2]) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         R const v = r[d] - R(YeeOff<FIELD, COMP>::f(d)) - R(0.5);
-        int const s = v >= -R(0.5) ? 0 : -1;
-        R const p = v - (R)s + R(0.5);
+        bool const below = YeeOff<FIELD, COMP>::f(d) != 0.0 && !(v >= -R(0.5));
+        R const p = v - (below ? R(-1.0) : R(0.0)) + R(0.5);
         w[d][0] = R(1.0) - p;
         w[d][1] = p;
-        o[d][0] = (uint32_t)wrapI(c[d] + s, n[d]) * stride[d];
-        o[d][1] = (uint32_t)wrapI(c[d] + s + 1, n[d]) * stride[d];
+        o[d][0] = below ? n.o[d][0] : n.o[d][1];
+        o[d][1] = below ? n.o[d][1] : n.o[d][2];
     }
 }
 
-template <int FIELD, int COMP, typename R>
-__device__ __forceinline__ R gatherD(const float* __restrict__ F, const GridDev& g, const int* c, const R* r) {
+template <int FIELD, int COMP, typename R, typename Plane>
+__device__ __forceinline__ R gatherD(Plane F, const NodeOffsets& n, const R* r) {
     uint32_t o[3][2];
     R w[3][2];
-    interpNodes<FIELD, COMP>(g, c, r, o, w);
+    interpNodes<FIELD, COMP>(n, r, o, w);
     R v = R(0.0);
 #pragma unroll
     for (int zz = 0; zz < 2; ++zz)
@@ -490,26 +552,14 @@ __device__ __forceinline__ R gatherD(const float* __restrict__ F, const GridDev&
 }
 
 // Reverse of the interpolation of one component: adds lam * weight to the
-// field adjoint at the 8 nodes (the block's LDS window plane L when LDS, with
-// rel the cell relative to the window reference; the global plane otherwise)
-// and lam * d(value)/dX to gX.
-template <int FIELD, int COMP, bool LDS, typename R>
-__device__ __forceinline__ void gatherAdj(const float* __restrict__ F, double* __restrict__ L, const GridDev& g,
-                                          const BlockWindow& win, const int* c, const int* rel, const R* r,
-                                          R lam, R* gX) {
+// field adjoint L at the 8 nodes (the block's LDS window when LDS, the grid
+// otherwise; F and L are planes of the same one) and lam * d(value)/dX to gX.
+template <int FIELD, int COMP, bool LDS, typename R, typename Plane>
+__device__ __forceinline__ void gatherAdj(Plane F, double* __restrict__ L, const NodeOffsets& n, const R* r, R lam,
+                                          R* gX) {
     uint32_t o[3][2];
     R w[3][2];
-    interpNodes<FIELD, COMP>(g, c, r, o, w);
-    uint32_t lo[3][2];
-    if (LDS) {
-        uint32_t const ls[3] = {1u, (uint32_t)win.ext[0], (uint32_t)(win.ext[0] * win.ext[1])};
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            int const sh = (r[d] - R(YeeOff<FIELD, COMP>::f(d)) - R(0.5)) >= -R(0.5) ? 0 : -1;
-            lo[d][0] = (uint32_t)(rel[d] + sh - win.lo[d]) * ls[d];
-            lo[d][1] = lo[d][0] + ls[d];
-        }
-    }
+    interpNodes<FIELD, COMP>(n, r, o, w);
     R gx = R(0.0), gy = R(0.0), gz = R(0.0);
 #pragma unroll
     for (int zz = 0; zz < 2; ++zz)
@@ -525,8 +575,7 @@ __device__ __forceinline__ void gatherAdj(const float* __restrict__ F, double* _
                 gz += f * w[0][xx] * w[1][yy] * sz;
                 double const v = (double)(lam * (w[0][xx] * w[1][yy] * w[2][zz]));
                 if (LDS)
-                    __hip_atomic_fetch_add(L + (lo[0][xx] + lo[1][yy] + lo[2][zz]), v, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                    __hip_atomic_fetch_add(L + at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 else
                     unsafeAtomicAdd(L + at, v);
             }
@@ -543,32 +592,27 @@ __device__ __forceinline__ void gatherAdj(const float* __restrict__ F, double* _
 // -csd W(i,j) C(k), W = S0a S0b + (DSa S0b + S0a DSb)/2 + DSa DSb/3 and C(k)
 // the prefix sum of DS along c (Esirkepov.hpp:140-240). Accumulates
 // dF/dX0 into l0 and dF/dX1 into l1 per axis.
-template <int COMP, typename R>
-__device__ __forceinline__ void esirkepovAdjComp(const double* __restrict__ lJ, const GridDev& g, const int* bc,
-                                                 const R* X0, const R* X1, R csd, R* l0,
-                                                 R* l1) {
+// off: the offsets of the stencil's nodes bc .. bc+2 per axis in lJ, the
+// window's (already in R) or the grid's plane.
+template <int COMP, typename R, typename Plane>
+__device__ __forceinline__ void esirkepovAdjComp(Plane lJ, const uint32_t (&off)[3][3], const R* X0, const R* X1,
+                                                 R csd, R* l0, R* l1) {
     constexpr int A = (COMP + 1) % 3;  // rotated i axis
     constexpr int B = (COMP + 2) % 3;  // rotated j axis
-    int const n[3] = {g.nx, g.ny, g.nz};
-    uint32_t const stride[3] = {1u, (uint32_t)g.nx, (uint32_t)g.nx * (uint32_t)g.ny};
-    uint32_t const k0 = (uint32_t)wrapI(bc[COMP], n[COMP]) * stride[COMP];
-    uint32_t const k1 = (uint32_t)wrapI(bc[COMP] + 1, n[COMP]) * stride[COMP];
-    uint32_t ob[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) ob[j] = (uint32_t)wrapI(bc[B] + j, n[B]) * stride[B];
+    uint32_t const k0 = off[COMP][0], k1 = off[COMP][1];
     R const C0 = cicD(R(0.0), X1[COMP]) - cicD(R(0.0), X0[COMP]);
     R const C1 = C0 + (cicD(R(1.0), X1[COMP]) - cicD(R(1.0), X0[COMP]));
     R dC0 = R(0.0), dC1 = R(0.0);
     R l0a = R(0.0), l1a = R(0.0), l0b = R(0.0), l1b = R(0.0);
 #pragma unroll 1
     for (int i = 0; i < 3; ++i) {
-        uint32_t const oa = (uint32_t)wrapI(bc[A] + i, n[A]) * stride[A];
+        uint32_t const oa = i == 0 ? off[A][0] : (i == 1 ? off[A][1] : off[A][2]);
         // the six current adjoints of this row, loaded together
         R m[3][2];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-            m[j][0] = lJ[oa + ob[j] + k0];
-            m[j][1] = lJ[oa + ob[j] + k1];
+            m[j][0] = (R)lJ[oa + off[B][j] + k0];
+            m[j][1] = (R)lJ[oa + off[B][j] + k1];
         }
         R const s0a = cicD((R)i, X0[A]);
         R const dsa = cicD((R)i, X1[A]) - s0a;
@@ -608,83 +652,106 @@ struct BorisFwd {
     R g, f, beta, hq;
 };
 
-// Boris push in the adjoint's precision (particlePusherBoris.hpp:41-90)
+// Boris push in the adjoint's precision (particlePusherBoris.hpp:41-90); dt = c = 1
 template <typename R>
-__device__ __forceinline__ BorisFwd<R> borisFwd(V3<R> p0, V3<R> E, V3<R> B, R m, R q, R dt, R rc2) {
+__device__ __forceinline__ BorisFwd<R> borisFwd(V3<R> p0, V3<R> E, V3<R> B, R m, R q) {
     BorisFwd<R> b;
-    b.hq = R(0.5) * q * dt;
+    b.hq = R(0.5) * q;
     b.pm = axpy(b.hq, E, p0);
-    b.g = sqrt(R(1.0) + dotD(b.pm, b.pm) * rc2 / (m * m));
-    b.beta = R(0.5) * (q / m) * dt;
+    b.g = sqrtAbove1(R(1.0) + dotD(b.pm, b.pm) / (m * m));
+    b.beta = R(0.5) * (q / m);
     b.t = scale3(b.beta / b.g, B);
-    b.f = R(1.0) / (R(1.0) + dotD(b.t, b.t));
+    b.f = recipAbove1(R(1.0) + dotD(b.t, b.t));
     b.s = scale3(R(2.0) * b.f, b.t);
     b.pp = add3(b.pm, crossD(b.pm, b.t));
     b.p1 = axpy(b.hq, E, add3(b.pm, crossD(b.pp, b.s)));
     return b;
 }
 
-template <typename R>
+template <bool LDS, typename R>
 __device__ __forceinline__ void adjointParticle(const AdjPartArgs& a, const AdjState& S, int64_t idx, const int* c,
-                                                const BlockWindow& win, const int* rel, double* sL, bool lds) {
+                                                const BlockWindow& win, const int* rel, const float* sF,
+                                                const R* sLJ, double* sL) {
     int64_t const n = S.n;
     R const r[3] = {(R)S.pos[idx], (R)S.pos[n + idx], (R)S.pos[2 * n + idx]};
     V3<R> const p0{(R)S.mom[idx], (R)S.mom[n + idx], (R)S.mom[2 * n + idx]};
     R const w = (R)S.w[idx];
     R const m = (R)a.mass * w;
     R const q = (R)a.charge * w;
-    R const dt = (R)a.dt;
-    R const rc2 = (R)a.rc2;
     R const cellR[3] = {(R)a.cell[0], (R)a.cell[1], (R)a.cell[2]};
     R const ivdt = (R)a.inv_vdt;
+    // the planes of the fields and of their adjoints, and the particle's nodes in them
+    NodeOffsets const no = LDS ? windowOffsets(win, rel) : gridOffsets(a.g, c);
+    auto plane = [&](int k) { return LDS ? sF + k * win.vol : (k < 3 ? a.E[k] : a.B[k - 3]); };
+    auto adjoint = [&](int k) { return LDS ? sL + k * win.vol : (k < 3 ? a.lE[k] : a.lB[k - 3]); };
 
     // ---- forward recompute: gather, Boris, velocity ----
-    V3<R> const E{gatherD<0, 0>(a.E[0], a.g, c, r), gatherD<0, 1>(a.E[1], a.g, c, r), gatherD<0, 2>(a.E[2], a.g, c, r)};
+    V3<R> const E{gatherD<0, 0>(plane(0), no, r), gatherD<0, 1>(plane(1), no, r), gatherD<0, 2>(plane(2), no, r)};
     phaseBarrier();
-    V3<R> const B{gatherD<1, 0>(a.B[0], a.g, c, r), gatherD<1, 1>(a.B[1], a.g, c, r), gatherD<1, 2>(a.B[2], a.g, c, r)};
+    V3<R> const B{gatherD<1, 0>(plane(3), no, r), gatherD<1, 1>(plane(4), no, r), gatherD<1, 2>(plane(5), no, r)};
     phaseBarrier();
     V3<R> p1;
     {
-        BorisFwd<R> const b = borisFwd(p0, E, B, m, q, dt, rc2);
+        BorisFwd<R> const b = borisFwd(p0, E, B, m, q);
         p1 = b.p1;
     }
-    R const G = sqrt(m * m + dotD(p1, p1) * rc2);
+    R const G = sqrt(m * m + dotD(p1, p1));
     R const v[3] = {p1.x / G, p1.y / G, p1.z / G};
 
     // ---- reverse Esirkepov ----
     R lX1[3], lv[3];
     {
         R X0[3], X1[3];
-        int bc[3];
+        int gs3[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            X1[d] = r[d] + v[d] * dt / cellR[d];
-            X0[d] = X1[d] - v[d] * dt / cellR[d];
+            R const step = divExact(v[d], a.rcell[d]);  // v dt / cell
+            X1[d] = r[d] + step;
+            X0[d] = X1[d] - step;
             int const gs = (int)fmin(floor(X0[d]), floor(X1[d]));
             X0[d] -= (R)gs;
             X1[d] -= (R)gs;
-            bc[d] = c[d] + gs;
+            gs3[d] = gs;
         }
         R l0[3] = {R(0.0), R(0.0), R(0.0)}, l1[3] = {R(0.0), R(0.0), R(0.0)};
         phaseBarrier();
-        esirkepovAdjComp<0>(a.lJ[0], a.g, bc, X0, X1, q * ivdt * cellR[0], l0, l1);
-        phaseBarrier();
-        esirkepovAdjComp<1>(a.lJ[1], a.g, bc, X0, X1, q * ivdt * cellR[1], l0, l1);
-        phaseBarrier();
-        esirkepovAdjComp<2>(a.lJ[2], a.g, bc, X0, X1, q * ivdt * cellR[2], l0, l1);
-        phaseBarrier();
+        int const at[3] = {rel[0] + gs3[0], rel[1] + gs3[1], rel[2] + gs3[2]};
+        uint32_t off[3][3];
+        if (LDS && windowHolds<2>(win, at)) {
+            uint32_t const ls[3] = {1u, (uint32_t)win.ext[0], (uint32_t)(win.ext[0] * win.ext[1])};
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) off[d][k] = (uint32_t)(at[d] + k - win.lo[d]) * ls[d];
+            esirkepovAdjComp<0>(sLJ, off, X0, X1, q * ivdt * cellR[0], l0, l1);
+            phaseBarrier();
+            esirkepovAdjComp<1>(sLJ + win.vol, off, X0, X1, q * ivdt * cellR[1], l0, l1);
+            phaseBarrier();
+            esirkepovAdjComp<2>(sLJ + 2 * win.vol, off, X0, X1, q * ivdt * cellR[2], l0, l1);
+            phaseBarrier();
+        } else {
+            axisOffsets(c[0] + gs3[0], a.g.nx, 1u, off[0]);
+            axisOffsets(c[1] + gs3[1], a.g.ny, (uint32_t)a.g.nx, off[1]);
+            axisOffsets(c[2] + gs3[2], a.g.nz, (uint32_t)a.g.nx * (uint32_t)a.g.ny, off[2]);
+            esirkepovAdjComp<0>(a.lJ[0], off, X0, X1, q * ivdt * cellR[0], l0, l1);
+            phaseBarrier();
+            esirkepovAdjComp<1>(a.lJ[1], off, X0, X1, q * ivdt * cellR[1], l0, l1);
+            phaseBarrier();
+            esirkepovAdjComp<2>(a.lJ[2], off, X0, X1, q * ivdt * cellR[2], l0, l1);
+            phaseBarrier();
+        }
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             // X1 = X + v dt/cell, X0 = X1 - v dt/cell
             lX1[d] = (R)S.lX[d * n + idx] + l0[d] + l1[d];
-            lv[d] = (lX1[d] - l0[d]) * dt / cellR[d];
+            lv[d] = divExact(lX1[d] - l0[d], a.rcell[d]);
         }
     }
 
     phaseBarrier();
     // ---- reverse velocity: v = p1 / sqrt(m^2 + |p1|^2 rc2) ----
     V3<R> const LV{lv[0], lv[1], lv[2]};
-    R const kv = dotD(p1, LV) * rc2 / (G * G * G);
+    R const kv = dotD(p1, LV) / (G * G * G);
     V3<R> const l1{(R)S.lP[idx] + LV.x / G - p1.x * kv, (R)S.lP[n + idx] + LV.y / G - p1.y * kv,
                    (R)S.lP[2 * n + idx] + LV.z / G - p1.z * kv};
 
@@ -694,7 +761,7 @@ __device__ __forceinline__ void adjointParticle(const AdjPartArgs& a, const AdjS
         V3<R> const p0o{opaque(p0.x), opaque(p0.y), opaque(p0.z)};
         V3<R> const Eo{opaque(E.x), opaque(E.y), opaque(E.z)};
         V3<R> const Bo{opaque(B.x), opaque(B.y), opaque(B.z)};
-        BorisFwd<R> const b = borisFwd(p0o, Eo, Bo, m, q, dt, rc2);
+        BorisFwd<R> const b = borisFwd(p0o, Eo, Bo, m, q);
         lE = scale3(b.hq, l1);                   // p1 = pl + hq E
         V3<R> lpm = l1;                             // pl = pm + pp x s
         V3<R> const lpp = crossD(b.s, l1);
@@ -705,7 +772,7 @@ __device__ __forceinline__ void adjointParticle(const AdjPartArgs& a, const AdjS
         V3<R> const lt = add3(lt1, add3(scale3(R(2.0) * b.f, ls), scale3(-R(4.0) * b.f * b.f * tls, b.t)));
         lB = scale3(b.beta / b.g, lt);                 // t = beta B / g
         R const lg = -b.beta * dotD(B, lt) / (b.g * b.g);
-        lpm = axpy(lg * rc2 / (m * m * b.g), b.pm, lpm);  // g = sqrt(1 + |pm|^2 rc2/m^2)
+        lpm = axpy(lg / (m * m * b.g), b.pm, lpm);  // g = sqrt(1 + |pm|^2 / m^2)
         lE = axpy(b.hq, lpm, lE);                      // pm = p0 + hq E
         lp0 = lpm;
     }
@@ -713,33 +780,18 @@ __device__ __forceinline__ void adjointParticle(const AdjPartArgs& a, const AdjS
     phaseBarrier();
     // ---- reverse gather (weights recomputed, not kept from the forward gather) ----
     R lX0[3] = {lX1[0], lX1[1], lX1[2]};
-    int const co[3] = {opaqueI(c[0]), opaqueI(c[1]), opaqueI(c[2])};
     R const ro[3] = {opaque(r[0]), opaque(r[1]), opaque(r[2])};
-    if (lds) {
-        gatherAdj<0, 0, true>(a.E[0], sL, a.g, win, co, rel, ro, lE.x, lX0);
-        phaseBarrier();
-        gatherAdj<0, 1, true>(a.E[1], sL + win.vol, a.g, win, co, rel, ro, lE.y, lX0);
-        phaseBarrier();
-        gatherAdj<0, 2, true>(a.E[2], sL + 2 * win.vol, a.g, win, co, rel, ro, lE.z, lX0);
-        phaseBarrier();
-        gatherAdj<1, 0, true>(a.B[0], sL + 3 * win.vol, a.g, win, co, rel, ro, lB.x, lX0);
-        phaseBarrier();
-        gatherAdj<1, 1, true>(a.B[1], sL + 4 * win.vol, a.g, win, co, rel, ro, lB.y, lX0);
-        phaseBarrier();
-        gatherAdj<1, 2, true>(a.B[2], sL + 5 * win.vol, a.g, win, co, rel, ro, lB.z, lX0);
-    } else {
-        gatherAdj<0, 0, false>(a.E[0], a.lE[0], a.g, win, co, rel, ro, lE.x, lX0);
-        phaseBarrier();
-        gatherAdj<0, 1, false>(a.E[1], a.lE[1], a.g, win, co, rel, ro, lE.y, lX0);
-        phaseBarrier();
-        gatherAdj<0, 2, false>(a.E[2], a.lE[2], a.g, win, co, rel, ro, lE.z, lX0);
-        phaseBarrier();
-        gatherAdj<1, 0, false>(a.B[0], a.lB[0], a.g, win, co, rel, ro, lB.x, lX0);
-        phaseBarrier();
-        gatherAdj<1, 1, false>(a.B[1], a.lB[1], a.g, win, co, rel, ro, lB.y, lX0);
-        phaseBarrier();
-        gatherAdj<1, 2, false>(a.B[2], a.lB[2], a.g, win, co, rel, ro, lB.z, lX0);
-    }
+    gatherAdj<0, 0, LDS>(plane(0), adjoint(0), no, ro, lE.x, lX0);
+    phaseBarrier();
+    gatherAdj<0, 1, LDS>(plane(1), adjoint(1), no, ro, lE.y, lX0);
+    phaseBarrier();
+    gatherAdj<0, 2, LDS>(plane(2), adjoint(2), no, ro, lE.z, lX0);
+    phaseBarrier();
+    gatherAdj<1, 0, LDS>(plane(3), adjoint(3), no, ro, lB.x, lX0);
+    phaseBarrier();
+    gatherAdj<1, 1, LDS>(plane(4), adjoint(4), no, ro, lB.y, lX0);
+    phaseBarrier();
+    gatherAdj<1, 2, LDS>(plane(5), adjoint(5), no, ro, lB.z, lX0);
     S.lX[idx] = lX0[0];
     S.lX[n + idx] = lX0[1];
     S.lX[2 * n + idx] = lX0[2];
@@ -749,20 +801,27 @@ __device__ __forceinline__ void adjointParticle(const AdjPartArgs& a, const AdjS
 }
 
 
-// FP64 LDS window of the field adjoint scatter: 6 components of this many cells
-constexpr int kAdjLdsCells = 640;
-
 // Precision of the per-particle adjoint arithmetic (Jacobian-vector
 // products); the adjoint state (lambda of particles and fields) is always
 // accumulated in FP64.
 using AdjReal = float;
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void kAdjParticles(AdjPartArgs a,
-                                                                                                 AdjState S) {
-    __shared__ double sL[6 * kAdjLdsCells];
-    __shared__ int sBox[9];
-    int64_t const idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// One thread per particle. The block's window holds the fields and the
+// current's adjoint it gathers from (as floats) and the FP64 accumulators of
+// the field adjoints; CAP cells of it. Bound by the LDS: 48 FP64 atomic adds
+// and 150 reads per particle.
+template <int NT, int CAP>
+__global__ __launch_bounds__(NT, NT == 512 ? 4 : 2) void kAdjParticles(AdjPartArgs a, AdjState S) {
+    __shared__ double sL[6 * CAP];
+    __shared__ float sF[6 * CAP];
+    __shared__ AdjReal sLJ[3 * CAP];
+    __shared__ int sBox[3 + 3 * NT / 64];
+    __shared__ uint16_t sOut[NT];
+    __shared__ int sOutN;
+    int64_t const first = (int64_t)blockIdx.x * NT;
+    int64_t const idx = first + threadIdx.x;
     bool const active = idx < S.n;
+    if (threadIdx.x == 0) sOutN = 0;
     int64_t const n = S.n;
     int c[3] = {0, 0, 0};
     if (active) {
@@ -770,21 +829,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         c[1] = S.cell[n + idx];
         c[2] = S.cell[2 * n + idx];
     }
-    // interpolation nodes of a particle in cell c: c-1 .. c+1 per axis
     int rel[3];
-    BlockWindow const win = blockWindow<1, 1>(a.g, active, c, rel, sBox, kAdjLdsCells);
-    if (win.lds) {
-        for (int e = threadIdx.x; e < 6 * win.vol; e += blockDim.x) sL[e] = 0.0;
-        __syncthreads();
-        if (active) adjointParticle<AdjReal>(a, S, idx, c, win, rel, sL, windowHolds<1, 1>(win, rel));
-        __syncthreads();
-        for (int e = threadIdx.x; e < 6 * win.vol; e += blockDim.x) {
-            double const v = sL[e];
-            if (v != 0.0) {
-                int const plane = e / win.vol;
-                double* const dst = plane < 3 ? a.lE[plane] : a.lB[plane - 3];
-                unsafeAtomicAdd(dst + windowToGlobal(a.g, win, e - plane * win.vol), v);
-            }
+    BlockWindow const win = blockWindow<NT>(a.g, active, c, rel, sBox, CAP);
+    for (int e = threadIdx.x; e < win.vol; e += NT) {
+        uint32_t const at = windowToGlobal(a.g, win, e);
+        double v[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) v[d] = a.lJ[d][at];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) sLJ[d * win.vol + e] = (AdjReal)v[d];
+    }
+    stageFields<NT>(a.g, win, a.E, a.B, sF);
+    for (int e = threadIdx.x; e < 6 * win.vol; e += NT) sL[e] = 0.0;
+    __syncthreads();
+    if (active) {
+        if (windowHoldsCell(win, rel))
+            adjointParticle<true, AdjReal>(a, S, idx, c, win, rel, sF, sLJ, sL);
+        else
+            sOut[atomicAdd(&sOutN, 1)] = (uint16_t)threadIdx.x;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < sOutN) {  // the particles outside the window, by full waves (as kDiffPush)
+        int64_t const k = first + sOut[threadIdx.x];
+        int const cell[3] = {S.cell[k], S.cell[n + k], S.cell[2 * n + k]};
+        adjointParticle<false, AdjReal>(a, S, k, cell, win, rel, sF, sLJ, sL);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < win.vol; e += NT) {
+        uint32_t const at = windowToGlobal(a.g, win, e);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            double const v = sL[k * win.vol + e];
+            if (v != 0.0) unsafeAtomicAdd((k < 3 ? a.lE[k] : a.lB[k - 3]) + at, v);
         }
     }
 }
@@ -797,7 +873,10 @@ __global__ __launch_bounds__(256) void kFillD(double* p, size_t n, double v) {
 // ---------------------------------------------------------------------------
 // re-tiling of the particle order at checkpoints
 // ---------------------------------------------------------------------------
-// key = tile of 8x4x1 cells of the particle's cell (x-fastest tile order), value = slot
+// key = tile of 8x4x2 cells of the particle's cell, value = slot. The tiles
+// follow each other x-fastest in a serpentine (every other row and layer
+// backwards), so that a block whose particles span two consecutive tiles has
+// a compact window also at the end of a row.
 __global__ __launch_bounds__(256) void kTileKeys(const int32_t* __restrict__ cell, int64_t n, GridDev g,
                                                  uint32_t* __restrict__ keys, int32_t* __restrict__ vals) {
     int64_t const i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -805,7 +884,8 @@ __global__ __launch_bounds__(256) void kTileKeys(const int32_t* __restrict__ cel
     uint32_t const ntx = (uint32_t)g.nx / kTileX, nty = (uint32_t)g.ny / kTileY;
     uint32_t const tx = (uint32_t)cell[i] / kTileX, ty = (uint32_t)cell[n + i] / kTileY;
     uint32_t const tz = (uint32_t)cell[2 * n + i] / kTileZ;
-    keys[i] = tx + ntx * (ty + nty * tz);
+    uint32_t const row = (tz & 1u ? nty - 1u - ty : ty) + nty * tz;
+    keys[i] = (row & 1u ? ntx - 1u - tx : tx) + ntx * row;
     vals[i] = (int32_t)i;
 }
 
@@ -878,9 +958,29 @@ hipError_t launchScatterAdjoint(const int32_t* perm, const double* src, double* 
 // ---------------------------------------------------------------------------
 static inline unsigned blocksOf(size_t n) { return (unsigned)((n + 255) / 256); }
 
+// Threads per block by the particles per tile of 8 x 4 x 2 cells, and the cells
+// of the LDS window: a block of the tiled order spans t = threads / particles
+// per tile and one more tile along x, (8 (t + 1) + 3) x 7 x 5 cells with the
+// nodes around them, and more as the particles drift (up to two cells before
+// the next sort). 512 threads share a window where a tile fills them: more
+// waves per CU for the same LDS. The windows are the largest that leave two
+// blocks of 512 per CU (48 B a cell in the forward kernel, 84 B in the
+// adjoint one). 64^3 cells, 8 particles per cell, us a launch, forward and
+// adjoint kernel: 229 and 412 with the fields gathered from memory by wrapped
+// indices and 256 threads; 88 and 287 now (129 and 447 with 768 cells, where
+// more particles lie outside the window).
+constexpr int kAdjDenseTile = 448;
+static bool denseTiles(int64_t particles, const GridDev& g) {
+    double const tiles = (double)(g.nx / kTileX) * (g.ny / kTileY) * (g.nz / kTileZ);
+    return (double)particles >= kAdjDenseTile * tiles;
+}
+
 hipError_t launchDiffPush(const DiffArgs& a, const DiffParticles& P, hipStream_t s) {
     if (P.n == 0) return hipSuccess;
-    hipLaunchKernelGGL(kDiffPush, dim3(blocksOf((size_t)P.n)), dim3(256), 0, s, a, P);
+    if (denseTiles(P.n, a.g))
+        hipLaunchKernelGGL((kDiffPush<512, 1536>), dim3((unsigned)((P.n + 511) / 512)), dim3(512), 0, s, a, P);
+    else
+        hipLaunchKernelGGL((kDiffPush<256, 960>), dim3((unsigned)((P.n + 255) / 256)), dim3(256), 0, s, a, P);
     return hipGetLastError();
 }
 
@@ -915,7 +1015,10 @@ hipError_t launchFillD(double* p, size_t n, double v, hipStream_t s) {
 
 hipError_t launchAdjParticles(const AdjPartArgs& a, const AdjState& st, hipStream_t s) {
     if (st.n == 0) return hipSuccess;
-    hipLaunchKernelGGL(kAdjParticles, dim3(blocksOf((size_t)st.n)), dim3(256), 0, s, a, st);
+    if (denseTiles(st.n, a.g))
+        hipLaunchKernelGGL((kAdjParticles<512, 928>), dim3((unsigned)((st.n + 511) / 512)), dim3(512), 0, s, a, st);
+    else
+        hipLaunchKernelGGL((kAdjParticles<256, 928>), dim3((unsigned)((st.n + 255) / 256)), dim3(256), 0, s, a, st);
     return hipGetLastError();
 }
 

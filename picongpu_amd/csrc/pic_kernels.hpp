@@ -317,7 +317,7 @@ struct DiffArgs {
     const float* B[3];
     unsigned long long* Jfix[3];  // int64 fixed-point current, zero on entry
     float cell[3];
-    float dt, c2, rc2, c;
+    double rcell[3];  // 1 / cell, for divExact
     float inv_vdt;
     double jscale;
     float mass;    // frame mass
@@ -339,8 +339,7 @@ struct AdjPartArgs {
     double* lE[3];  // accumulated with atomics
     double* lB[3];
     double cell[3];
-    double dt;
-    double rc2;
+    double rcell[3];  // 1 / cell, for divExact
     double mass;    // frame mass
     double charge;  // frame charge
     double inv_vdt;
@@ -361,9 +360,9 @@ hipError_t launchFixToFloat(unsigned long long* fix, float* const J[3], size_t n
 hipError_t launchAdjFields(const AdjFieldArgs& a, double dt, double c2, double coeff, double* lJ[3], hipStream_t s);
 hipError_t launchAdjParticles(const AdjPartArgs& a, const AdjState& st, hipStream_t s);
 hipError_t launchFillD(double* p, size_t n, double v, hipStream_t s);
-// particle order of the differentiable form: tiles of 8x4x1 cells (grids are
+// particle order of the differentiable form: tiles of 8x4x2 cells (grids are
 // multiples of the supercell, so of the tile)
-constexpr int kTileX = 8, kTileY = 4, kTileZ = 1;
+constexpr int kTileX = 8, kTileY = 4, kTileZ = 2;
 hipError_t sortTempBytes(int64_t n, size_t* bytes);
 // stable sort of the slots by tile; *perm receives vals[1] (new slot -> old slot)
 hipError_t launchTileSort(const int32_t* cell, int64_t n, const GridDev& g, uint32_t* keys[2], int32_t* vals[2],

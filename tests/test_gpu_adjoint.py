@@ -95,6 +95,48 @@ def test_adjoint_matches_fp64_tape():
     pic.close()
 
 
+@pytest.mark.parametrize("ppc", [2, 7, 9])
+def test_hot_particles_match_fp64_tape(ppc):
+    """Forward and gradients with particles that move up to half a cell a step
+    in every direction, so that many lie outside the windows of their thread
+    blocks, in sparse tiles (blocks of 256 particles) and dense ones (512)."""
+    nsteps, every, grid = 6, 4, (16, 16, 8)
+    print(f"case adjoint hot grid={grid} ppc={ppc} steps={nsteps}", flush=True)
+    st = setups.differentiable(grid=grid, ppc=ppc, steps=nsteps)
+    cell, pos, mom, w = adjoint.cold_plasma(st)
+    rng = np.random.default_rng(ppc)
+    mass = float(setups.abi_free_constants(st)["base_mass"]) * float(w[0])
+    mom = (rng.standard_normal(mom.shape) * 0.7 * mass).astype(np.float32)
+    pic = adjoint.DifferentiablePIC(st, cell, pos, mom, w, nsteps, every)
+    g = T.grid_from_constants(st.grid, pic.sim.constants(), w[0])
+    X = torch.tensor((cell.astype(np.float64) + pos.astype(np.float64)).T.copy())
+    p = torch.tensor(mom.astype(np.float64).T.copy())
+    theta = torch.tensor([1.0, 0.5, 0.05], dtype=F64)
+    E0, B0 = adjoint.gaussian_pulse(st, theta.cuda(), amp=pulse_amp(st))
+    lo, hi = (4, 4, 2), (12, 12, 6)
+    E, B = pic.forward_raw(E0, B0)
+    Ed = E.double().requires_grad_(True)
+    Bd = B.double().requires_grad_(True)
+    adjoint.probe_energy(st, Ed, Bd, lo, hi).backward()
+    dE0, dB0, dX0, dP0 = pic.backward_raw(Ed.grad, Bd.grad, particles=True)
+    e0 = torch.tensor(E0.float().cpu().numpy().astype(np.float64))
+    b0 = torch.tensor(B0.float().cpu().numpy().astype(np.float64))
+    with torch.no_grad():
+        Xt, pt, Et, Bt = X.clone(), p.clone(), e0, b0
+        for _ in range(nsteps):
+            Xt, pt, Et, Bt = T.step(g, Xt, pt, Et, Bt)
+    f, tE, tB, tX, tP = T.gradient_all(g, X, p, e0, b0, nsteps, lo, hi)
+    err = {"E": rel_max(E.cpu().numpy(), Et.numpy()), "B": rel_max(B.cpu().numpy(), Bt.numpy())}
+    grad = {"dE0": rel_max(dE0.cpu().numpy(), tE.numpy()), "dB0": rel_max(dB0.cpu().numpy(), tB.numpy()),
+            "dX0": rel_max(dX0.cpu().numpy(), tX.numpy().T), "dP0": rel_max(dP0.cpu().numpy(), tP.numpy().T)}
+    print("hot particles vs FP64 tape:", err, grad)
+    for nm, e in err.items():
+        assert e < 1e-5, (nm, e)
+    for nm, e in grad.items():
+        assert e < 1e-4, (nm, e)
+    pic.close()
+
+
 def test_parameter_gradient_matches_central_differences():
     """dF/dtheta through the torch.autograd.Function (pulse built in torch on
     the device, HIP forward and adjoint) against FP64 central differences of

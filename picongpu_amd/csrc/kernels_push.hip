@@ -723,122 +723,132 @@ size_t pushTileElems(int supp) {
     }
 }
 
-// The supercells whose J tile of component c covers global cell g along axis
-// a (tile origin at the supercell's origin minus DLO, extent ext): the
-// candidates' supercell index along the axis (wrapped on a periodic axis)
-// and the cell's tile coordinate, ordered by the axis' checkerboard colour
-// (colour[s]). Returns their number (at most 3).
-template <int SUPP>
-__device__ __forceinline__ int coveringAlong(int g, int scSize, int ext, int nsc, bool open,
-                                             const uint8_t* __restrict__ colour, int* scOut, int* tOut) {
-    constexpr int DLO = Esirkepov<SUPP>::lowerMargin;
-    int n = 0;
+// One axis of a supercell's neighbourhood for the gather flush: the steps -1,
+// 0, 1 to the supercells whose J tiles reach into it, in ascending
+// checkerboard colour, and those supercells' indices (-1 beyond an open
+// border). All values are uniform in the block.
+struct CoverAxis {
+    int step[3], sc[3];
+};
+__device__ __forceinline__ CoverAxis coverAxis(int s, int nsc, bool open, const uint8_t* __restrict__ colour) {
+    CoverAxis a;
     int col[3];
-    int const hi = (g + DLO) >= 0 ? (g + DLO) / scSize : -((-(g + DLO) + scSize - 1) / scSize);  // floor
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        int const s = hi - k;
-        int const t = g + DLO - s * scSize;
-        if (t < 0 || t >= ext) continue;
-        int sw = s;
-        if (open) {
-            if (s < 0 || s >= nsc) continue;
-        } else {
-            sw = ((s % nsc) + nsc) % nsc;
-        }
-        int const cs = colour[sw];
-        int m = n++;
-        for (; m > 0 && col[m - 1] > cs; --m) {
-            col[m] = col[m - 1];
-            scOut[m] = scOut[m - 1];
-            tOut[m] = tOut[m - 1];
-        }
-        col[m] = cs;
-        scOut[m] = sw;
-        tOut[m] = t;
+    for (int k = 0; k < 3; ++k) {  // the supercell above first, as equal colours (rings of two) stay in order
+        int t = s + 1 - k;
+        bool const beyond = t < 0 || t >= nsc;
+        t = t < 0 ? t + nsc : (t >= nsc ? t - nsc : t);
+        a.step[k] = 1 - k;
+        a.sc[k] = beyond && open ? -1 : t;
+        col[k] = colour[t];
     }
-    return n;
+#pragma unroll
+    for (int pass = 0; pass < 3; ++pass) {  // (0,1), (1,2), (0,1)
+        int const m = pass & 1;
+        if (col[m] > col[m + 1]) {
+            int const c = col[m], st = a.step[m], sc = a.sc[m];
+            col[m] = col[m + 1], a.step[m] = a.step[m + 1], a.sc[m] = a.sc[m + 1];
+            col[m + 1] = c, a.step[m + 1] = st, a.sc[m + 1] = sc;
+        }
+    }
+    return a;
 }
 
-// One thread per J cell: for each component the covering supercells' tile
-// values, added as the flush adds them, in ascending checkerboard phase. A
-// phase's index is colour_x + ncol_x (colour_y + ncol_y colour_z), so
-// visiting z, then y, then x candidates each in ascending colour is
-// ascending phase (every supercell covering a cell lies in another phase).
-template <int SUPP>
-__device__ __forceinline__ void gatherFlushCell(const GridDev& g, const float* __restrict__ tiles,
-                                                const uint8_t* __restrict__ colour, float* J0, float* J1, float* J2,
-                                                size_t i) {
-    using TG = JTileGeom<Esirkepov<SUPP>::lowerMargin, Esirkepov<SUPP>::upperMargin>;
+// Component C of one supercell's 256 J cells, a thread each: the values of
+// the at most 2 x 2 x 3 tiles that cover a cell, all loaded before the first
+// addition, then added as the flush adds them, in ascending checkerboard
+// phase (zeros add nothing). A phase's index is colour_x + ncol_x (colour_y +
+// ncol_y colour_z), so visiting z, then y, then x neighbours each in
+// ascending colour is ascending phase (every supercell covering a cell lies
+// in another phase).
+template <int SUPP, int C>
+__device__ __forceinline__ void gatherFlushComponent(const GridDev& g, const float* __restrict__ tiles,
+                                                     const CoverAxis& ax, const CoverAxis& ay, const CoverAxis& az,
+                                                     float* __restrict__ J, size_t cell, bool fresh) {
+    constexpr int DLO = Esirkepov<SUPP>::lowerMargin;
+    using TG = JTileGeom<DLO, Esirkepov<SUPP>::upperMargin>;
     constexpr int J_ELEMS = PushLds<SUPP, 1>::J_ELEMS;
-    int const x = (int)(i % g.nx);
-    int const y = (int)((i / g.nx) % g.ny);
-    int const z = (int)(i / ((size_t)g.nx * g.ny));
-    float* const Jc[3] = {J0, J1, J2};
+    constexpr int EX = TG::ext(C, 0), EY = TG::ext(C, 1), EZ = TG::ext(C, 2);
+    int const tid = threadIdx.x;
+    int const lx = tid & 7, ly = (tid >> 3) & 7, lz = tid >> 6;
+    int const lane = (lz * EY + ly) * EX + lx;
+    float w[27];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        int sx[3], tx[3], sy[3], ty[3], sz[3], tz[3];
-        int const nx = coveringAlong<SUPP>(x, SCX, TG::ext(c, 0), g.nscx, (g.open & 1) != 0, colour, sx, tx);
-        int const ny = coveringAlong<SUPP>(y, SCY, TG::ext(c, 1), g.nscy, (g.open & 2) != 0, colour + g.nscx, sy, ty);
-        int const nz = coveringAlong<SUPP>(z, SCZ, TG::ext(c, 2), g.nscz, (g.open & 4) != 0,
-                                           colour + g.nscx + g.nscy, sz, tz);
-        float v = Jc[c][i];
-        bool any = false;
-        for (int a = 0; a < nz; ++a)
-            for (int b = 0; b < ny; ++b)
-                for (int d = 0; d < nx; ++d) {
-                    int const sc = sx[d] + g.nscx * (sy[b] + g.nscy * sz[a]);
-                    float const w =
-                        tiles[(size_t)sc * J_ELEMS + TG::off(c) + (tz[a] * TG::ext(c, 1) + ty[b]) * TG::ext(c, 0) + tx[d]];
-                    if (w == 0.0f) continue;
-                    v += w;
-                    any = true;
-                }
-        if (any) Jc[c][i] = v;
+    for (int k = 0; k < 27; ++k) {
+        int const a = k / 9, b = (k / 3) % 3, d = k % 3;
+        int const ox = DLO - SCX * ax.step[d], oy = DLO - SCY * ay.step[b], oz = DLO - SCZ * az.step[a];
+        w[k] = 0.0f;
+        if (ax.sc[d] < 0 || ay.sc[b] < 0 || az.sc[a] < 0) continue;  // uniform
+        int const sc = ax.sc[d] + g.nscx * (ay.sc[b] + g.nscy * az.sc[a]);
+        const float* const t = tiles + (size_t)sc * J_ELEMS + TG::off(C) + (oz * EY + oy) * EX + ox;
+        if ((unsigned)(lx + ox) < (unsigned)EX && (unsigned)(ly + oy) < (unsigned)EY &&
+            (unsigned)(lz + oz) < (unsigned)EZ)
+            w[k] = t[lane];
     }
+    float v = fresh ? 0.0f : J[cell];
+#pragma unroll
+    for (int k = 0; k < 27; ++k) v += w[k];
+    J[cell] = v;
+}
+
+// J of one supercell (256 threads). fresh: J holds nothing yet (the sums
+// start at zero and every cell is written), so the step needs no reset of J.
+// 64^3 cells (CIC): 21 us a launch plus 5 for the reset with a loop of
+// dependent loads over the candidates of every cell.
+template <int SUPP>
+__device__ __forceinline__ void gatherFlushSC(const GridDev& g, const float* __restrict__ tiles,
+                                              const uint8_t* __restrict__ colour, float* J0, float* J1, float* J2,
+                                              int sc, bool fresh) {
+    int const sx = sc % g.nscx, sy = (sc / g.nscx) % g.nscy, sz = sc / (g.nscx * g.nscy);
+    CoverAxis const ax = coverAxis(sx, g.nscx, (g.open & 1) != 0, colour);
+    CoverAxis const ay = coverAxis(sy, g.nscy, (g.open & 2) != 0, colour + g.nscx);
+    CoverAxis const az = coverAxis(sz, g.nscz, (g.open & 4) != 0, colour + g.nscx + g.nscy);
+    int const tid = threadIdx.x;
+    size_t const cell = (size_t)(sx * SCX + (tid & 7)) +
+                        (size_t)g.nx * ((size_t)(sy * SCY + ((tid >> 3) & 7)) + (size_t)g.ny * (sz * SCZ + (tid >> 6)));
+    gatherFlushComponent<SUPP, 0>(g, tiles, ax, ay, az, J0, cell, fresh);
+    gatherFlushComponent<SUPP, 1>(g, tiles, ax, ay, az, J1, cell, fresh);
+    gatherFlushComponent<SUPP, 2>(g, tiles, ax, ay, az, J2, cell, fresh);
 }
 
 template <int SUPP>
-__global__ __launch_bounds__(256) void kGatherFlush(GridDev g, const float* __restrict__ tiles,
+__global__ __launch_bounds__(SCV) void kGatherFlush(GridDev g, const float* __restrict__ tiles,
                                                      const uint8_t* __restrict__ colour, float* J0, float* J1,
-                                                     float* J2) {
+                                                     float* J2, int fresh) {
     if (halted(g)) return;
-    size_t const n = (size_t)g.nx * g.ny * g.nz;
-    size_t const i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) gatherFlushCell<SUPP>(g, tiles, colour, J0, J1, J2, i);
+    gatherFlushSC<SUPP>(g, tiles, colour, J0, J1, J2, (int)blockIdx.x, fresh != 0);
 }
 
 template <int SUPP>
-__global__ __launch_bounds__(256) void kGatherFlushBatch(const GatherEntry* __restrict__ table,
-                                                          const int2* __restrict__ blocks) {
+__global__ __launch_bounds__(SCV) void kGatherFlushBatch(const GatherEntry* __restrict__ table,
+                                                          const int2* __restrict__ blocks, int fresh) {
     int2 const it = blocks[blockIdx.x];
     const GatherEntry& e = table[it.x];
     if (halted(e.g)) return;
-    size_t const n = (size_t)e.g.nx * e.g.ny * e.g.nz;
-    size_t const i = (size_t)it.y * blockDim.x + threadIdx.x;
-    if (i < n) gatherFlushCell<SUPP>(e.g, e.tiles, e.colour, e.J[0], e.J[1], e.J[2], i);
+    gatherFlushSC<SUPP>(e.g, e.tiles, e.colour, e.J[0], e.J[1], e.J[2], it.y, fresh != 0);
 }
 
-hipError_t launchGatherFlushBatch(int supp, const GatherEntry* table, const int2* blocks, int nblocks,
+hipError_t launchGatherFlushBatch(int supp, const GatherEntry* table, const int2* blocks, int nblocks, bool fresh,
                                   hipStream_t s) {
     if (nblocks <= 0) return hipSuccess;
+    dim3 const grid(nblocks), block(SCV);
     switch (supp) {
-        case 2: hipLaunchKernelGGL(kGatherFlushBatch<2>, dim3(nblocks), dim3(256), 0, s, table, blocks); break;
-        case 3: hipLaunchKernelGGL(kGatherFlushBatch<3>, dim3(nblocks), dim3(256), 0, s, table, blocks); break;
-        case 4: hipLaunchKernelGGL(kGatherFlushBatch<4>, dim3(nblocks), dim3(256), 0, s, table, blocks); break;
+        case 2: hipLaunchKernelGGL(kGatherFlushBatch<2>, grid, block, 0, s, table, blocks, fresh ? 1 : 0); break;
+        case 3: hipLaunchKernelGGL(kGatherFlushBatch<3>, grid, block, 0, s, table, blocks, fresh ? 1 : 0); break;
+        case 4: hipLaunchKernelGGL(kGatherFlushBatch<4>, grid, block, 0, s, table, blocks, fresh ? 1 : 0); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
 hipError_t launchGatherFlush(int supp, const GridDev& g, const float* tiles, const uint8_t* colour,
-                             float* const J[3], hipStream_t s) {
-    size_t const n = (size_t)g.nx * g.ny * g.nz;
-    dim3 const grid((unsigned)((n + 255) / 256));
+                             float* const J[3], bool fresh, hipStream_t s) {
+    dim3 const grid((unsigned)(g.nscx * g.nscy * g.nscz)), block(SCV);
+    int const f = fresh ? 1 : 0;
     switch (supp) {
-        case 2: hipLaunchKernelGGL(kGatherFlush<2>, grid, dim3(256), 0, s, g, tiles, colour, J[0], J[1], J[2]); break;
-        case 3: hipLaunchKernelGGL(kGatherFlush<3>, grid, dim3(256), 0, s, g, tiles, colour, J[0], J[1], J[2]); break;
-        case 4: hipLaunchKernelGGL(kGatherFlush<4>, grid, dim3(256), 0, s, g, tiles, colour, J[0], J[1], J[2]); break;
+        case 2: hipLaunchKernelGGL(kGatherFlush<2>, grid, block, 0, s, g, tiles, colour, J[0], J[1], J[2], f); break;
+        case 3: hipLaunchKernelGGL(kGatherFlush<3>, grid, block, 0, s, g, tiles, colour, J[0], J[1], J[2], f); break;
+        case 4: hipLaunchKernelGGL(kGatherFlush<4>, grid, block, 0, s, g, tiles, colour, J[0], J[1], J[2], f); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

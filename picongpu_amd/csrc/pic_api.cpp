@@ -1079,7 +1079,8 @@ std::vector<std::vector<int>> pushGroups(pic_ctx* c, int32_t species, bool byPus
     return groups;
 }
 
-int runPush(pic_ctx* c, int32_t species, int mode, bool stageShift = false) {
+// freshJ: J holds nothing yet and the first group's gather flush writes it
+int runPush(pic_ctx* c, int32_t species, int mode, bool stageShift = false, bool freshJ = false) {
     bool const byPusher = mode != 2;
     auto groups = pushGroups(c, species, byPusher);
     for (const auto& grp : groups) {
@@ -1108,7 +1109,8 @@ int runPush(pic_ctx* c, int32_t species, int mode, bool stageShift = false) {
             a.tileOut = plan->tiles;
             TimerScope ts(c, PIC_TIMER_PUSH);
             PIC_HIP(pic::launchPush(supp, pusher, mode, scheme, a, c->nsc, c->stream));
-            PIC_HIP(pic::launchGatherFlush(supp, c->g, plan->tiles, plan->colour, c->J, c->stream));
+            PIC_HIP(pic::launchGatherFlush(supp, c->g, plan->tiles, plan->colour, c->J, freshJ, c->stream));
+            freshJ = false;
             continue;
         }
         for (size_t ph = 0; ph < plan->count.size(); ++ph) {
@@ -2268,8 +2270,17 @@ int fieldStep(pic_ctx* c) {
 // field stages fused
 int oneStep(pic_ctx* c) {
     int r;
-    if ((r = pic_current_reset(c)) != PIC_OK) return r;
-    if ((r = runPush(c, -1, 1, true)) != PIC_OK) return r;
+    // where the first push leaves its tiles to the gather flush, that flush
+    // writes every cell of J and the reset is left out
+    bool freshJ = false;
+    auto const groups = pushGroups(c, -1, true);
+    if (!groups.empty()) {
+        PhasePlan* plan = nullptr;
+        if ((r = getPlan(c, supportOf(c->sp[groups[0][0]].desc.shape), true, &plan)) != PIC_OK) return r;
+        freshJ = plan->single;
+    }
+    if (!freshJ && (r = pic_current_reset(c)) != PIC_OK) return r;
+    if ((r = runPush(c, -1, 1, true, freshJ)) != PIC_OK) return r;
     if ((r = runShift(c, -1)) != PIC_OK) return r;
     return fieldStep(c);
 }
@@ -3041,14 +3052,15 @@ int ensSyncMembers(pic_ensemble* e) {
 // fused field step; the members' E/Ealt swap as in pic_step
 int ensOneStep(pic_ensemble* e) {
     int const p = e->parity;
-    PIC_HIP(pic::launchCurrentResetBatch(e->dField[p], e->dBlocks, e->nBlocks, e->stream));
+    // (with the tiles gathered, that launch writes every cell of J)
+    if (!e->single) PIC_HIP(pic::launchCurrentResetBatch(e->dField[p], e->dBlocks, e->nBlocks, e->stream));
     for (size_t ph = 0; ph < e->phaseCount.size(); ++ph) {
         int const m = e->phaseCount[ph];
         int const grid = e->blocksPerCu > 0 ? std::min(m, e->blocksPerCu * e->cus) : m;
         PIC_HIP(pic::launchPushBatch(e->supp, e->pusher, e->dPush[p], e->dPhaseWork + e->phaseOffset[ph], m, grid,
                                      e->stream));
     }
-    if (e->single) PIC_HIP(pic::launchGatherFlushBatch(e->supp, e->dGather, e->dBlocks, e->nBlocks, e->stream));
+    if (e->single) PIC_HIP(pic::launchGatherFlushBatch(e->supp, e->dGather, e->dBlocks, e->nBlocks, true, e->stream));
     PIC_HIP(pic::launchShiftBatch(e->dShift, e->dShiftWork, e->nShiftWork, e->stream));
     PIC_HIP(pic::launchFieldStepBatch(e->solver, e->dField[p], e->dTiles, e->nTiles, e->dBlocks, e->nBlocks,
                                       e->stream));

@@ -135,9 +135,10 @@ size_t pushTileElems(int supp);
 // checkerboard phases: the float additions, in the same order, of the
 // phase-by-phase flush, so J is the same bit for bit. colour: the
 // checkerboard colour of every supercell index along x, then y, then z
-// (nscx + nscy + nscz entries).
+// (nscx + nscy + nscz entries). fresh: J holds nothing yet; the sums start at
+// zero and every cell is written.
 hipError_t launchGatherFlush(int supp, const GridDev& g, const float* tiles, const uint8_t* colour,
-                             float* const J[3], hipStream_t s);
+                             float* const J[3], bool fresh, hipStream_t s);
 // shift of one species: `staged` = the push epilogue already moved the leavers
 // to the outbox and compacted every supercell (then only the insert runs).
 // redo: the insert again after the supercells grew, from count - incoming
@@ -292,7 +293,8 @@ struct GatherEntry {
     const uint8_t* colour;
     float* J[3];
 };
-hipError_t launchGatherFlushBatch(int supp, const GatherEntry* table, const int2* blocks, int nblocks,
+// blocks: (member, supercell) items
+hipError_t launchGatherFlushBatch(int supp, const GatherEntry* table, const int2* blocks, int nblocks, bool fresh,
                                   hipStream_t s);
 // end of a batched step: every member's step flags as the end-of-step kernel of pic_step sets them
 hipError_t launchEndStepBatch(const FieldBatchEntry* table, int n, hipStream_t s);

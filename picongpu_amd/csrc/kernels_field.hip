@@ -37,45 +37,45 @@ __device__ __forceinline__ void unit(int d, int& ux, int& uy, int& uz) {
 }
 
 // forward difference of component f along axis d at offset (ox,oy,oz)
-__device__ __forceinline__ float fwd(const float* f, const Idx& I, int d, int ox, int oy, int oz, float step) {
+__device__ __forceinline__ float fwd(const float* f, const Idx& I, int d, int ox, int oy, int oz, double rstep) {
     int ux, uy, uz;
     unit(d, ux, uy, uz);
-    return (I.get(f, ox + ux, oy + uy, oz + uz) - I.get(f, ox, oy, oz)) / step;
+    return divExact(I.get(f, ox + ux, oy + uy, oz + uz) - I.get(f, ox, oy, oz), rstep);
 }
 
 // Lehe derivative along axis d of component f (Lehe/Derivative.hpp:132-145 for
 // d == Cherenkov-free axis, :212-224 otherwise)
 __device__ __forceinline__ float leheDeriv(const float* f, const Idx& I, int d, const FieldArgs& a) {
     int const L = a.lehe_dir;
-    float const step = a.cell[d];
+    double const rstep = a.rcell[d];
     if (d == L) {
         int const d1 = (d + 1) % 3, d2 = (d + 2) % 3;
         int u1x, u1y, u1z, u2x, u2y, u2z, u0x, u0y, u0z;
         unit(d1, u1x, u1y, u1z);
         unit(d2, u2x, u2y, u2z);
         unit(d, u0x, u0y, u0z);
-        float r = a.lehe_alpha * fwd(f, I, d, 0, 0, 0, step);
-        r = r + a.lehe_beta1 * fwd(f, I, d, u1x, u1y, u1z, step);
-        r = r + a.lehe_beta1 * fwd(f, I, d, -u1x, -u1y, -u1z, step);
-        r = r + a.lehe_beta2 * fwd(f, I, d, u2x, u2y, u2z, step);
-        r = r + a.lehe_beta2 * fwd(f, I, d, -u2x, -u2y, -u2z, step);
-        r = r + a.lehe_delta * (I.get(f, 2 * u0x, 2 * u0y, 2 * u0z) - I.get(f, -u0x, -u0y, -u0z)) / step;
+        float r = a.lehe_alpha * fwd(f, I, d, 0, 0, 0, rstep);
+        r = r + a.lehe_beta1 * fwd(f, I, d, u1x, u1y, u1z, rstep);
+        r = r + a.lehe_beta1 * fwd(f, I, d, -u1x, -u1y, -u1z, rstep);
+        r = r + a.lehe_beta2 * fwd(f, I, d, u2x, u2y, u2z, rstep);
+        r = r + a.lehe_beta2 * fwd(f, I, d, -u2x, -u2y, -u2z, rstep);
+        r = r + divExact(a.lehe_delta * (I.get(f, 2 * u0x, 2 * u0y, 2 * u0z) - I.get(f, -u0x, -u0y, -u0z)), rstep);
         return r;
     }
     int ulx, uly, ulz;
     unit(L, ulx, uly, ulz);
     float const beta = 0.125f;
     float const alpha = 1.0f - 2.0f * beta;
-    float r = alpha * fwd(f, I, d, 0, 0, 0, step);
-    r = r + beta * fwd(f, I, d, ulx, uly, ulz, step);
-    r = r + beta * fwd(f, I, d, -ulx, -uly, -ulz, step);
+    float r = alpha * fwd(f, I, d, 0, 0, 0, rstep);
+    r = r + beta * fwd(f, I, d, ulx, uly, ulz, rstep);
+    r = r + beta * fwd(f, I, d, -ulx, -uly, -ulz, rstep);
     return r;
 }
 
 template <int SOLVER>
 __device__ __forceinline__ float derivE(const float* f, const Idx& I, int d, const FieldArgs& a) {
     if (SOLVER == PIC_SOLVER_LEHE) return leheDeriv(f, I, d, a);
-    return fwd(f, I, d, 0, 0, 0, a.cell[d]);
+    return fwd(f, I, d, 0, 0, 0, a.rcell[d]);
 }
 
 // a cell known to lie outside every PML layer (FieldArgs::inner)
@@ -100,10 +100,10 @@ __global__ __launch_bounds__(256) void kBHalf(FieldArgs a) {
     a.B[2][i] = a.B[2][i] - cz * 0.5f * a.dt;
 }
 
-__device__ __forceinline__ float bwd(const float* f, const Idx& I, int d, float step) {
+__device__ __forceinline__ float bwd(const float* f, const Idx& I, int d, double rstep) {
     int ux, uy, uz;
     unit(d, ux, uy, uz);
-    return (I.get(f, 0, 0, 0) - I.get(f, -ux, -uy, -uz)) / step;
+    return divExact(I.get(f, 0, 0, 0) - I.get(f, -ux, -uy, -uz), rstep);
 }
 
 __global__ __launch_bounds__(256) void kEFull(FieldArgs a) {
@@ -112,9 +112,9 @@ __global__ __launch_bounds__(256) void kEFull(FieldArgs a) {
     size_t const i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     Idx I{a.g, (int)(i % a.g.nx), (int)((i / a.g.nx) % a.g.ny), (int)(i / ((size_t)a.g.nx * a.g.ny))};
-    float const cx = bwd(a.B[2], I, 1, a.cell[1]) - bwd(a.B[1], I, 2, a.cell[2]);
-    float const cy = bwd(a.B[0], I, 2, a.cell[2]) - bwd(a.B[2], I, 0, a.cell[0]);
-    float const cz = bwd(a.B[1], I, 0, a.cell[0]) - bwd(a.B[0], I, 1, a.cell[1]);
+    float const cx = bwd(a.B[2], I, 1, a.rcell[1]) - bwd(a.B[1], I, 2, a.rcell[2]);
+    float const cy = bwd(a.B[0], I, 2, a.rcell[2]) - bwd(a.B[2], I, 0, a.rcell[0]);
+    float const cz = bwd(a.B[1], I, 0, a.rcell[0]) - bwd(a.B[0], I, 1, a.rcell[1]);
     a.E[0][i] = a.E[0][i] + cx * a.c2 * a.dt;
     a.E[1][i] = a.E[1][i] + cy * a.c2 * a.dt;
     a.E[2][i] = a.E[2][i] + cz * a.c2 * a.dt;
@@ -254,9 +254,9 @@ template <bool ADDJ>
 __device__ __forceinline__ void eFullPmlCell(const FieldArgs& a, const PmlArgs& p, float* const* Eout, size_t i) {
     int const x = (int)(i % a.g.nx), y = (int)((i / a.g.nx) % a.g.ny), z = (int)(i / ((size_t)a.g.nx * a.g.ny));
     Idx I{a.g, x, y, z};
-    float const dBdxY = bwd(a.B[1], I, 0, a.cell[0]), dBdxZ = bwd(a.B[2], I, 0, a.cell[0]);
-    float const dBdyX = bwd(a.B[0], I, 1, a.cell[1]), dBdyZ = bwd(a.B[2], I, 1, a.cell[1]);
-    float const dBdzX = bwd(a.B[0], I, 2, a.cell[2]), dBdzY = bwd(a.B[1], I, 2, a.cell[2]);
+    float const dBdxY = bwd(a.B[1], I, 0, a.rcell[0]), dBdxZ = bwd(a.B[2], I, 0, a.rcell[0]);
+    float const dBdyX = bwd(a.B[0], I, 1, a.rcell[1]), dBdyZ = bwd(a.B[2], I, 1, a.rcell[1]);
+    float const dBdzX = bwd(a.B[0], I, 2, a.rcell[2]), dBdzY = bwd(a.B[1], I, 2, a.rcell[2]);
     if (!innerCell(a, x, y, z)) {
         eFullPmlApply<ADDJ>(a, p, Eout, x, y, z, i, dBdxY, dBdxZ, dBdyX, dBdyZ, dBdzX, dBdzY);
         return;
@@ -289,9 +289,9 @@ __global__ __launch_bounds__(256) void kEFullJ(FieldArgs a, float* En0, float* E
     size_t const i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     Idx I{a.g, (int)(i % a.g.nx), (int)((i / a.g.nx) % a.g.ny), (int)(i / ((size_t)a.g.nx * a.g.ny))};
-    float const cx = bwd(a.B[2], I, 1, a.cell[1]) - bwd(a.B[1], I, 2, a.cell[2]);
-    float const cy = bwd(a.B[0], I, 2, a.cell[2]) - bwd(a.B[2], I, 0, a.cell[0]);
-    float const cz = bwd(a.B[1], I, 0, a.cell[0]) - bwd(a.B[0], I, 1, a.cell[1]);
+    float const cx = bwd(a.B[2], I, 1, a.rcell[1]) - bwd(a.B[1], I, 2, a.rcell[2]);
+    float const cy = bwd(a.B[0], I, 2, a.rcell[2]) - bwd(a.B[2], I, 0, a.rcell[0]);
+    float const cz = bwd(a.B[1], I, 0, a.rcell[0]) - bwd(a.B[0], I, 1, a.rcell[1]);
     float const e0 = a.E[0][i] + cx * a.c2 * a.dt;
     float const e1 = a.E[1][i] + cy * a.c2 * a.dt;
     float const e2 = a.E[2][i] + cz * a.c2 * a.dt;
@@ -347,34 +347,34 @@ __device__ __forceinline__ void curlE(const FieldArgs& a, float* const* E, const
 template <int SY, int SZ>
 struct LdsStencil {
     static __device__ __forceinline__ int off(int d) { return d == 0 ? 1 : (d == 1 ? SY : SZ); }
-    static __device__ __forceinline__ float fwd(const float* f, int h, int d, float step) {
-        return (f[h + off(d)] - f[h]) / step;
+    static __device__ __forceinline__ float fwd(const float* f, int h, int d, double rstep) {
+        return divExact(f[h + off(d)] - f[h], rstep);
     }
     static __device__ __forceinline__ float lehe(const float* f, int h, int d, const FieldArgs& a) {
         int const L = a.lehe_dir;
-        float const step = a.cell[d];
+        double const rstep = a.rcell[d];
         if (d == L) {
             int const o1 = off((d + 1) % 3), o2 = off((d + 2) % 3), o0 = off(d);
-            float r = a.lehe_alpha * fwd(f, h, d, step);
-            r = r + a.lehe_beta1 * fwd(f, h + o1, d, step);
-            r = r + a.lehe_beta1 * fwd(f, h - o1, d, step);
-            r = r + a.lehe_beta2 * fwd(f, h + o2, d, step);
-            r = r + a.lehe_beta2 * fwd(f, h - o2, d, step);
-            r = r + a.lehe_delta * (f[h + 2 * o0] - f[h - o0]) / step;
+            float r = a.lehe_alpha * fwd(f, h, d, rstep);
+            r = r + a.lehe_beta1 * fwd(f, h + o1, d, rstep);
+            r = r + a.lehe_beta1 * fwd(f, h - o1, d, rstep);
+            r = r + a.lehe_beta2 * fwd(f, h + o2, d, rstep);
+            r = r + a.lehe_beta2 * fwd(f, h - o2, d, rstep);
+            r = r + divExact(a.lehe_delta * (f[h + 2 * o0] - f[h - o0]), rstep);
             return r;
         }
         int const oL = off(L);
         float const beta = 0.125f;
         float const alpha = 1.0f - 2.0f * beta;
-        float r = alpha * fwd(f, h, d, step);
-        r = r + beta * fwd(f, h + oL, d, step);
-        r = r + beta * fwd(f, h - oL, d, step);
+        float r = alpha * fwd(f, h, d, rstep);
+        r = r + beta * fwd(f, h + oL, d, rstep);
+        r = r + beta * fwd(f, h - oL, d, rstep);
         return r;
     }
     template <int SOLVER>
     static __device__ __forceinline__ float deriv(const float* f, int h, int d, const FieldArgs& a) {
         if (SOLVER == PIC_SOLVER_LEHE) return lehe(f, h, d, a);
-        return fwd(f, h, d, a.cell[d]);
+        return fwd(f, h, d, a.rcell[d]);
     }
     // curl of E with components at f0, f1, f2 (each a plane of the staged tile)
     template <int SOLVER>
@@ -407,50 +407,97 @@ struct FieldLds {
     float B[3][kFHV];
 };
 
-// tile b of the grid: every thread of the 256-thread workgroup calls it
+// Stages NP planes of the nodes (x0 - HALO ..) of a tile of X x Y x Z nodes in
+// LDS, plane by plane: a thread's node offsets are formed once for the planes
+// and its loads are all in flight before the first LDS write (a loop of load
+// and write waited for memory ten times).
+template <int X, int Y, int Z, int HALO, bool OPEN, int NP>
+__device__ __forceinline__ void stageTile(const GridDev& g, int x0, int y0, int z0, const float* const (&src)[NP],
+                                          float* const (&dst)[NP]) {
+    constexpr int N = X * Y * Z, NU = (N + 255) / 256;
+    float v[NP][NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+        int const t = (int)threadIdx.x + u * 256 < N ? (int)threadIdx.x + u * 256 : 0;
+        int const x = t % X - HALO, y = (t / X) % Y - HALO, z = t / (X * Y) - HALO;
+        size_t const gi = wrapAt(g, x0, y0, z0, x, y, z);
+        bool const out = outsideIf<OPEN>(g, x0 + x, y0 + y, z0 + z);
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            float const f = src[p][gi];
+            v[p][u] = out ? 0.0f : f;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+        int const t = (int)threadIdx.x + u * 256;
+        if (t < N) {
+#pragma unroll
+            for (int p = 0; p < NP; ++p) dst[p][t] = v[p][u];
+        }
+    }
+}
+
+// tile b of the grid: every thread of the 256-thread workgroup calls it. The
+// Yee curl reaches one node, the Lehe curl two. 64^3 cells: 14.7 us a launch
+// with serial staging loops, a halo of two nodes and full divisions.
 template <int SOLVER, bool OPEN>
 __device__ __forceinline__ void fieldBeforeAddTile(const FieldArgs& a, float* const* Enew, int b, FieldLds& L) {
+    constexpr int kEH = SOLVER == PIC_SOLVER_LEHE ? pic::kEH : 1;
+    constexpr int kEX = kFTX + 2 * kEH, kEY = kFTY + 2 * kEH, kEZ = kFTZ + 2 * kEH;
     int const ntx = a.g.nx / kFTX, nty = a.g.ny / kFTY;
     int const x0 = (b % ntx) * kFTX, y0 = ((b / ntx) % nty) * kFTY, z0 = (b / (ntx * nty)) * kFTZ;
-    for (int t = threadIdx.x; t < 3 * kEV; t += blockDim.x) {
-        int const c = t / kEV, r = t - c * kEV;
-        int const ex = r % kEX, ey = (r / kEX) % kEY, ez = r / (kEX * kEY);
-        bool const out = outsideIf<OPEN>(a.g, x0 + ex - kEH, y0 + ey - kEH, z0 + ez - kEH);
-        L.E[c][r] = out ? 0.0f : a.E[c][wrapAt(a.g, x0, y0, z0, ex - kEH, ey - kEH, ez - kEH)];
+    int const lx = threadIdx.x % kFTX, ly = (threadIdx.x / kFTX) % kFTY, lz = threadIdx.x / (kFTX * kFTY);
+    size_t const i = (size_t)(x0 + lx) + (size_t)a.g.nx * ((size_t)(y0 + ly) + (size_t)a.g.ny * (size_t)(z0 + lz));
+    // B of the tile and its lower halo, and the cell's J: loaded along with E
+    constexpr int NB = (kFHV + 255) / 256;
+    float bOld[NB][3];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+        int const t = (int)threadIdx.x + u * 256 < kFHV ? (int)threadIdx.x + u * 256 : 0;
+        size_t const bi = wrapAt(a.g, x0, y0, z0, t % kFHX - 1, (t / kFHX) % kFHY - 1, t / (kFHX * kFHY) - 1);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) bOld[u][c] = a.B[c][bi];
+    }
+    float const j0 = a.J[0][i], j1 = a.J[1][i], j2 = a.J[2][i];
+    {
+        const float* const src[3] = {a.E[0], a.E[1], a.E[2]};
+        float* const dst[3] = {L.E[0], L.E[1], L.E[2]};
+        stageTile<kEX, kEY, kEZ, kEH, OPEN, 3>(a.g, x0, y0, z0, src, dst);
     }
     __syncthreads();
     using SE = LdsStencil<kEX, kEX * kEY>;
-    for (int t = threadIdx.x; t < kFHV; t += blockDim.x) {
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+        int const t = (int)threadIdx.x + u * 256;
+        if (t >= kFHV) break;
         int const hx = t % kFHX, hy = (t / kFHX) % kFHY, hz = t / (kFHX * kFHY);
         // B' at tile offset (hx-1, hy-1, hz-1)
         int const he = (hx - 1 + kEH) + kEX * ((hy - 1 + kEH) + kEY * (hz - 1 + kEH));
-        size_t const i = wrapAt(a.g, x0, y0, z0, hx - 1, hy - 1, hz - 1);
         if (outsideIf<OPEN>(a.g, x0 + hx - 1, y0 + hy - 1, z0 + hz - 1)) {  // B beyond an open border stays zero
             L.B[0][t] = L.B[1][t] = L.B[2][t] = 0.0f;
             continue;
         }
         float cx, cy, cz;
         SE::template curl<SOLVER>(L.E[0], L.E[1], L.E[2], he, a, cx, cy, cz);
-        L.B[0][t] = a.B[0][i] - cx * 0.5f * a.dt;
-        L.B[1][t] = a.B[1][i] - cy * 0.5f * a.dt;
-        L.B[2][t] = a.B[2][i] - cz * 0.5f * a.dt;
+        L.B[0][t] = bOld[u][0] - cx * 0.5f * a.dt;
+        L.B[1][t] = bOld[u][1] - cy * 0.5f * a.dt;
+        L.B[2][t] = bOld[u][2] - cz * 0.5f * a.dt;
     }
     __syncthreads();
-    int const lx = threadIdx.x % kFTX, ly = (threadIdx.x / kFTX) % kFTY, lz = threadIdx.x / (kFTX * kFTY);
-    size_t const i = (size_t)(x0 + lx) + (size_t)a.g.nx * ((size_t)(y0 + ly) + (size_t)a.g.ny * (size_t)(z0 + lz));
     int const h = (lx + 1) + kFHX * ((ly + 1) + kFHY * (lz + 1));
     int const he = (lx + kEH) + kEX * ((ly + kEH) + kEY * (lz + kEH));
     constexpr int SY = kFHX, SZ = kFHX * kFHY;
     // backward differences of B' (BackwardDerivative.hpp:44-65), curl as kEFull
-    float const cx = (L.B[2][h] - L.B[2][h - SY]) / a.cell[1] - (L.B[1][h] - L.B[1][h - SZ]) / a.cell[2];
-    float const cy = (L.B[0][h] - L.B[0][h - SZ]) / a.cell[2] - (L.B[2][h] - L.B[2][h - 1]) / a.cell[0];
-    float const cz = (L.B[1][h] - L.B[1][h - 1]) / a.cell[0] - (L.B[0][h] - L.B[0][h - SY]) / a.cell[1];
+    float const cx = divExact(L.B[2][h] - L.B[2][h - SY], a.rcell[1]) - divExact(L.B[1][h] - L.B[1][h - SZ], a.rcell[2]);
+    float const cy = divExact(L.B[0][h] - L.B[0][h - SZ], a.rcell[2]) - divExact(L.B[2][h] - L.B[2][h - 1], a.rcell[0]);
+    float const cz = divExact(L.B[1][h] - L.B[1][h - 1], a.rcell[0]) - divExact(L.B[0][h] - L.B[0][h - SY], a.rcell[1]);
     float e0 = L.E[0][he] + cx * a.c2 * a.dt;
     float e1 = L.E[1][he] + cy * a.c2 * a.dt;
     float e2 = L.E[2][he] + cz * a.c2 * a.dt;
-    e0 = e0 + a.coeff * a.J[0][i];
-    e1 = e1 + a.coeff * a.J[1][i];
-    e2 = e2 + a.coeff * a.J[2][i];
+    e0 = e0 + a.coeff * j0;
+    e1 = e1 + a.coeff * j1;
+    e2 = e2 + a.coeff * j2;
     Enew[0][i] = e0;
     Enew[1][i] = e1;
     Enew[2][i] = e2;
@@ -560,12 +607,12 @@ __device__ __forceinline__ void yeeBeforeAddTile(const FieldArgs& a, float* cons
             }
             int const ex = bx, ey = by;              // its E-plane index (E plane starts at -1)
             float const e0 = L.E[s][0][ey][ex], e1 = L.E[s][1][ey][ex], e2 = L.E[s][2][ey][ex];
-            float const dEzdy = (L.E[s][2][ey + 1][ex] - e2) / a.cell[1];
-            float const dEydz = (L.E[s1][1][ey][ex] - e1) / a.cell[2];
-            float const dExdz = (L.E[s1][0][ey][ex] - e0) / a.cell[2];
-            float const dEzdx = (L.E[s][2][ey][ex + 1] - e2) / a.cell[0];
-            float const dEydx = (L.E[s][1][ey][ex + 1] - e1) / a.cell[0];
-            float const dExdy = (L.E[s][0][ey + 1][ex] - e0) / a.cell[1];
+            float const dEzdy = divExact(L.E[s][2][ey + 1][ex] - e2, a.rcell[1]);
+            float const dEydz = divExact(L.E[s1][1][ey][ex] - e1, a.rcell[2]);
+            float const dExdz = divExact(L.E[s1][0][ey][ex] - e0, a.rcell[2]);
+            float const dEzdx = divExact(L.E[s][2][ey][ex + 1] - e2, a.rcell[0]);
+            float const dEydx = divExact(L.E[s][1][ey][ex + 1] - e1, a.rcell[0]);
+            float const dExdy = divExact(L.E[s][0][ey + 1][ex] - e0, a.rcell[1]);
             float const cx = dEzdy - dEydz;
             float const cy = dExdz - dEzdx;
             float const cz = dEydx - dExdy;
@@ -593,12 +640,12 @@ __device__ __forceinline__ void yeeBeforeAddTile(const FieldArgs& a, float* cons
             int const s = k & 1, sm = (k - 1) & 1;
             int const bx = lx + 1, by = ly + 1;
             // backward differences of B' (BackwardDerivative.hpp:44-65), curl as kEFull
-            float const cx = (L.B[s][2][by][bx] - L.B[s][2][by - 1][bx]) / a.cell[1] -
-                             (L.B[s][1][by][bx] - L.B[sm][1][by][bx]) / a.cell[2];
-            float const cy = (L.B[s][0][by][bx] - L.B[sm][0][by][bx]) / a.cell[2] -
-                             (L.B[s][2][by][bx] - L.B[s][2][by][bx - 1]) / a.cell[0];
-            float const cz = (L.B[s][1][by][bx] - L.B[s][1][by][bx - 1]) / a.cell[0] -
-                             (L.B[s][0][by][bx] - L.B[s][0][by - 1][bx]) / a.cell[1];
+            float const cx = divExact(L.B[s][2][by][bx] - L.B[s][2][by - 1][bx], a.rcell[1]) -
+                             divExact(L.B[s][1][by][bx] - L.B[sm][1][by][bx], a.rcell[2]);
+            float const cy = divExact(L.B[s][0][by][bx] - L.B[sm][0][by][bx], a.rcell[2]) -
+                             divExact(L.B[s][2][by][bx] - L.B[s][2][by][bx - 1], a.rcell[0]);
+            float const cz = divExact(L.B[s][1][by][bx] - L.B[s][1][by][bx - 1], a.rcell[0]) -
+                             divExact(L.B[s][0][by][bx] - L.B[s][0][by - 1][bx], a.rcell[1]);
             size_t const i = ixy + plane * k;
             float e0 = L.E[s][0][ly + 1][lx + 1] + cx * a.c2 * a.dt;
             float e1 = L.E[s][1][ly + 1][lx + 1] + cy * a.c2 * a.dt;
@@ -681,9 +728,9 @@ __device__ __forceinline__ void yeeAfterTile(const FieldArgs& a, float* const* E
             // differences of the curl for every cell, the update per cell
             int const s = k & 1, s1 = (k + 1) & 1;
             float const f0 = L.E[s][0][ly][lx], f1 = L.E[s][1][ly][lx], f2 = L.E[s][2][ly][lx];
-            float const dxY = (L.E[s][1][ly][lx + 1] - f1) / a.cell[0], dxZ = (L.E[s][2][ly][lx + 1] - f2) / a.cell[0];
-            float const dyX = (L.E[s][0][ly + 1][lx] - f0) / a.cell[1], dyZ = (L.E[s][2][ly + 1][lx] - f2) / a.cell[1];
-            float const dzX = (L.E[s1][0][ly][lx] - f0) / a.cell[2], dzY = (L.E[s1][1][ly][lx] - f1) / a.cell[2];
+            float const dxY = divExact(L.E[s][1][ly][lx + 1] - f1, a.rcell[0]), dxZ = divExact(L.E[s][2][ly][lx + 1] - f2, a.rcell[0]);
+            float const dyX = divExact(L.E[s][0][ly + 1][lx] - f0, a.rcell[1]), dyZ = divExact(L.E[s][2][ly + 1][lx] - f2, a.rcell[1]);
+            float const dzX = divExact(L.E[s1][0][ly][lx] - f0, a.rcell[2]), dzY = divExact(L.E[s1][1][ly][lx] - f1, a.rcell[2]);
             size_t const i = ixy + plane * k;
             if (!innerCell(a, T.x0 + lx, T.y0 + ly, k)) {
                 bHalfPmlApply(a, *p, updatePsi, T.x0 + lx, T.y0 + ly, k, i, dxY, dxZ, dyX, dyZ, dzX, dzY);
@@ -698,9 +745,9 @@ __device__ __forceinline__ void yeeAfterTile(const FieldArgs& a, float* const* E
                             float& cz) {
                 // F: plane k, G: plane k+1 (forward differences, curl as kBHalf)
                 float const f0 = F[0][ly][lx], f1 = F[1][ly][lx], f2 = F[2][ly][lx];
-                cx = (F[2][ly + 1][lx] - f2) / a.cell[1] - (G[1][ly][lx] - f1) / a.cell[2];
-                cy = (G[0][ly][lx] - f0) / a.cell[2] - (F[2][ly][lx + 1] - f2) / a.cell[0];
-                cz = (F[1][ly][lx + 1] - f1) / a.cell[0] - (F[0][ly + 1][lx] - f0) / a.cell[1];
+                cx = divExact(F[2][ly + 1][lx] - f2, a.rcell[1]) - divExact(G[1][ly][lx] - f1, a.rcell[2]);
+                cy = divExact(G[0][ly][lx] - f0, a.rcell[2]) - divExact(F[2][ly][lx + 1] - f2, a.rcell[0]);
+                cz = divExact(F[1][ly][lx + 1] - f1, a.rcell[0]) - divExact(F[0][ly + 1][lx] - f0, a.rcell[1]);
             };
             size_t const i = ixy + plane * k;
             float cx, cy, cz;
@@ -742,33 +789,34 @@ __device__ __forceinline__ float lAt(const LehePlanes& P, int c, int x, int y, i
 }
 
 // fwd/leheDeriv of component c along d at tile cell (x, y) of plane k
-__device__ __forceinline__ float lFwd(const LehePlanes& P, int c, int d, int x, int y, int k, float step) {
-    return (lAt(P, c, x + (d == 0), y + (d == 1), k + (d == 2)) - lAt(P, c, x, y, k)) / step;
+__device__ __forceinline__ float lFwd(const LehePlanes& P, int c, int d, int x, int y, int k, double rstep) {
+    return divExact(lAt(P, c, x + (d == 0), y + (d == 1), k + (d == 2)) - lAt(P, c, x, y, k), rstep);
 }
 
 __device__ __forceinline__ float lDeriv(const LehePlanes& P, int c, int d, int x, int y, int k, const FieldArgs& a) {
     int const L = a.lehe_dir;
-    float const step = a.cell[d];
+    double const rstep = a.rcell[d];
     if (d == L) {
         int const d1 = (d + 1) % 3, d2 = (d + 2) % 3;
         int const u1x = d1 == 0, u1y = d1 == 1, u1z = d1 == 2;
         int const u2x = d2 == 0, u2y = d2 == 1, u2z = d2 == 2;
         int const u0x = d == 0, u0y = d == 1, u0z = d == 2;
-        float r = a.lehe_alpha * lFwd(P, c, d, x, y, k, step);
-        r = r + a.lehe_beta1 * lFwd(P, c, d, x + u1x, y + u1y, k + u1z, step);
-        r = r + a.lehe_beta1 * lFwd(P, c, d, x - u1x, y - u1y, k - u1z, step);
-        r = r + a.lehe_beta2 * lFwd(P, c, d, x + u2x, y + u2y, k + u2z, step);
-        r = r + a.lehe_beta2 * lFwd(P, c, d, x - u2x, y - u2y, k - u2z, step);
-        r = r + a.lehe_delta * (lAt(P, c, x + 2 * u0x, y + 2 * u0y, k + 2 * u0z) - lAt(P, c, x - u0x, y - u0y, k - u0z)) /
-                    step;
+        float r = a.lehe_alpha * lFwd(P, c, d, x, y, k, rstep);
+        r = r + a.lehe_beta1 * lFwd(P, c, d, x + u1x, y + u1y, k + u1z, rstep);
+        r = r + a.lehe_beta1 * lFwd(P, c, d, x - u1x, y - u1y, k - u1z, rstep);
+        r = r + a.lehe_beta2 * lFwd(P, c, d, x + u2x, y + u2y, k + u2z, rstep);
+        r = r + a.lehe_beta2 * lFwd(P, c, d, x - u2x, y - u2y, k - u2z, rstep);
+        r = r + divExact(a.lehe_delta * (lAt(P, c, x + 2 * u0x, y + 2 * u0y, k + 2 * u0z) -
+                                         lAt(P, c, x - u0x, y - u0y, k - u0z)),
+                         rstep);
         return r;
     }
     int const ulx = L == 0, uly = L == 1, ulz = L == 2;
     float const beta = 0.125f;
     float const alpha = 1.0f - 2.0f * beta;
-    float r = alpha * lFwd(P, c, d, x, y, k, step);
-    r = r + beta * lFwd(P, c, d, x + ulx, y + uly, k + ulz, step);
-    r = r + beta * lFwd(P, c, d, x - ulx, y - uly, k - ulz, step);
+    float r = alpha * lFwd(P, c, d, x, y, k, rstep);
+    r = r + beta * lFwd(P, c, d, x + ulx, y + uly, k + ulz, rstep);
+    r = r + beta * lFwd(P, c, d, x - ulx, y - uly, k - ulz, rstep);
     return r;
 }
 
@@ -881,24 +929,25 @@ template <int SOLVER, bool OPEN>
 __device__ __forceinline__ void fieldAfterTile(const FieldArgs& a, float* const* Enew, int b, AfterLds& L) {
     int const ntx = a.g.nx / kFTX, nty = a.g.ny / kFTY;
     int const x0 = (b % ntx) * kFTX, y0 = ((b / ntx) % nty) * kFTY, z0 = (b / (ntx * nty)) * kFTZ;
-    for (int t = threadIdx.x; t < 3 * kAV; t += blockDim.x) {
-        int const c = t / kAV, r = t - c * kAV;
-        int const ex = r % kAX, ey = (r / kAX) % kAY, ez = r / (kAX * kAY);
-        size_t const gi = wrapAt(a.g, x0, y0, z0, ex - 1, ey - 1, ez - 1);
-        bool const out = outsideIf<OPEN>(a.g, x0 + ex - 1, y0 + ey - 1, z0 + ez - 1);
-        L.E[c][r] = out ? 0.0f : a.E[c][gi];
-        L.En[c][r] = out ? 0.0f : Enew[c][gi];
+    // halo of the Lehe curl: 1 node below and 2 above; of the Yee curl: 1 above
+    constexpr int H = SOLVER == PIC_SOLVER_LEHE ? 1 : 0;
+    constexpr int kAX = kFTX + 1 + 2 * H, kAY = kFTY + 1 + 2 * H, kAZ = kFTZ + 1 + 2 * H;
+    int const lx = threadIdx.x % kFTX, ly = (threadIdx.x / kFTX) % kFTY, lz = threadIdx.x / (kFTX * kFTY);
+    size_t const i = (size_t)(x0 + lx) + (size_t)a.g.nx * ((size_t)(y0 + ly) + (size_t)a.g.ny * (size_t)(z0 + lz));
+    float const bOld[3] = {a.B[0][i], a.B[1][i], a.B[2][i]};
+    {
+        const float* const src[6] = {a.E[0], a.E[1], a.E[2], Enew[0], Enew[1], Enew[2]};
+        float* const dst[6] = {L.E[0], L.E[1], L.E[2], L.En[0], L.En[1], L.En[2]};
+        stageTile<kAX, kAY, kAZ, H, OPEN, 6>(a.g, x0, y0, z0, src, dst);
     }
     __syncthreads();
     using SA = LdsStencil<kAX, kAX * kAY>;
-    int const lx = threadIdx.x % kFTX, ly = (threadIdx.x / kFTX) % kFTY, lz = threadIdx.x / (kFTX * kFTY);
-    size_t const i = (size_t)(x0 + lx) + (size_t)a.g.nx * ((size_t)(y0 + ly) + (size_t)a.g.ny * (size_t)(z0 + lz));
-    int const h = (lx + 1) + kAX * ((ly + 1) + kAY * (lz + 1));
+    int const h = (lx + H) + kAX * ((ly + H) + kAY * (lz + H));
     float cx, cy, cz;
     SA::template curl<SOLVER>(L.E[0], L.E[1], L.E[2], h, a, cx, cy, cz);
-    float const b0 = a.B[0][i] - cx * 0.5f * a.dt;
-    float const b1 = a.B[1][i] - cy * 0.5f * a.dt;
-    float const b2 = a.B[2][i] - cz * 0.5f * a.dt;
+    float const b0 = bOld[0] - cx * 0.5f * a.dt;
+    float const b1 = bOld[1] - cy * 0.5f * a.dt;
+    float const b2 = bOld[2] - cz * 0.5f * a.dt;
     SA::template curl<SOLVER>(L.En[0], L.En[1], L.En[2], h, a, cx, cy, cz);
     a.B[0][i] = b0 - cx * 0.5f * a.dt;
     a.B[1][i] = b1 - cy * 0.5f * a.dt;

@@ -1035,6 +1035,7 @@ pic::FieldArgs makeFieldArgs(pic_ctx* c) {
         a.B[d] = c->B[d];
         a.J[d] = c->J[d];
         a.cell[d] = c->k.cell[d];
+        a.rcell[d] = 1.0 / static_cast<double>(c->k.cell[d]);
     }
     a.dt = c->k.dt;
     a.c2 = c->k.c * c->k.c;

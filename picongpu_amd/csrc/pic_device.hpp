@@ -83,13 +83,6 @@ __device__ __forceinline__ float sqrtAbove1(float x) {
     return ru > 0.0f ? up : t;
 }
 
-// RN(x / c) from rc = RN64(1 / c): the FP64 product is within 2^-52 of x / c
-// relatively, and no quotient of two floats lies closer than 2^-49 to the
-// midpoint of two neighbouring normal floats (|x - m c| is at least one unit
-// of a 49-bit product, and never 0 for a 25-bit m), so rounding the product
-// rounds the quotient. Three instructions instead of eleven.
-__device__ __forceinline__ float divExact(float x, double rc) { return (float)((double)x * rc); }
-
 // cross product (pmacc/math/vector/Vector.tpp:71-76)
 __device__ __forceinline__ Vec3 cross(Vec3 a, Vec3 b) {
     return Vec3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};

@@ -311,7 +311,7 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
         if (MODE != 2 && tid < kOffStride) {
             for (int s = 0; s < a.nsp; ++s) a.sp[s].outOff[(size_t)sc * kOffStride + tid] = 0u;
         }
-        if (MODE == 1 && a.tileOut)  // an empty tile for the gather flush
+        if (MODE != 0 && a.tileOut)  // an empty tile for the gather flush
             for (int t = tid; t < J_ELEMS; t += blockDim.x) a.tileOut[(size_t)sc * J_ELEMS + t] = 0.0f;
         return;
     }
@@ -534,7 +534,7 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
     }
     __syncthreads();
 
-    if (MODE == 1 && a.tileOut) {
+    if (MODE != 0 && a.tileOut) {
         // one launch for every supercell: the tile is left for the gather
         // flush as the floats the flush would add, zero where it adds
         // nothing (adding a zero would change nothing either: J never holds

@@ -709,7 +709,7 @@ struct PhasePlan {
     std::vector<int> count;   // per phase
     std::vector<int> host;    // the list on the host, launch order per phase
     int32_t* dList = nullptr;
-    // fused plans: every supercell in one launch, the tiles added to J by the
+    // one-launch plans: every supercell in one launch, the tiles added to J by the
     // gather flush in phase order (same J, bit for bit), instead of one
     // launch per phase; chosen when the phases are too small to fill the GPU
     bool single = false;
@@ -819,7 +819,7 @@ struct pic_ctx {
     double* diagBuf = nullptr;  // ncells doubles, allocated on first use
     int jexp = 40;
     // [supp-2][fused]
-    PhasePlan plans[3][2];
+    PhasePlan plans[3];
     int cus = 256;          // compute units of the device
     int pushSchedule = 0;   // PIC_PUSH_SCHEDULE_*
     bool member = false;    // owned by an ensemble, whose device tables hold its plans' scratch
@@ -906,8 +906,7 @@ int resolveTimers(pic_ctx* c) {
 // forms: a fused deposit runs in the frame of the particle's new cell, but
 // its cells lie within the margins of the old one (the path starts in the
 // old cell and moves less than a cell per axis).
-int buildPlan(pic_ctx* c, int supp, bool fused, PhasePlan& plan) {
-    (void)fused;
+int buildPlan(pic_ctx* c, int supp, PhasePlan& plan) {
     int const lo = depLower(supp);
     int const up = depUpper(supp);
     const int scs[3] = {pic::kSCX, pic::kSCY, pic::kSCZ};
@@ -950,8 +949,8 @@ int buildPlan(pic_ctx* c, int supp, bool fused, PhasePlan& plan) {
     // one launch for every supercell when the largest phase would leave more
     // than half of the CUs' workgroup slots idle (small boxes)
     int const most = *std::max_element(plan.count.begin(), plan.count.end());
-    plan.single = fused && (c->pushSchedule == PIC_PUSH_SCHEDULE_SINGLE ||
-                            (c->pushSchedule == PIC_PUSH_SCHEDULE_AUTO && most < 2 * c->cus));
+    plan.single = c->pushSchedule == PIC_PUSH_SCHEDULE_SINGLE ||
+                  (c->pushSchedule == PIC_PUSH_SCHEDULE_AUTO && most < 2 * c->cus);
     if (plan.single) {
         std::vector<uint8_t> colour;
         for (int d = 0; d < 3; ++d) {
@@ -968,10 +967,11 @@ int buildPlan(pic_ctx* c, int supp, bool fused, PhasePlan& plan) {
     return PIC_OK;
 }
 
-int getPlan(pic_ctx* c, int supp, bool fused, PhasePlan** out) {
-    PhasePlan& p = c->plans[supp - 2][fused ? 1 : 0];
+// the fused push and the deposit stage share the plan (and the tile scratch)
+int getPlan(pic_ctx* c, int supp, PhasePlan** out) {
+    PhasePlan& p = c->plans[supp - 2];
     if (!p.valid) {
-        int const r = buildPlan(c, supp, fused, p);
+        int const r = buildPlan(c, supp, p);
         if (r != PIC_OK) return r;
     }
     *out = &p;
@@ -1101,7 +1101,7 @@ int runPush(pic_ctx* c, int32_t species, int mode, bool stageShift = false, bool
             continue;
         }
         PhasePlan* plan = nullptr;
-        int const r = getPlan(c, supp, mode == 1, &plan);
+        int const r = getPlan(c, supp, &plan);
         if (r != PIC_OK) return r;
         if (plan->single) {
             // every supercell in one launch (phase-ordered list), then the
@@ -1657,7 +1657,7 @@ int pic_set_push_schedule(pic_ctx* c, int32_t schedule) {
     c->pushSchedule = schedule;
     dropGraphs(c);  // captured launches follow the old plans
     for (int supp = 0; supp < 3; ++supp) {
-        PhasePlan& p = c->plans[supp][1];
+        PhasePlan& p = c->plans[supp];
         if (!p.valid) continue;
         devFree(c, p.dList);
         devFree(c, p.tiles);
@@ -1670,18 +1670,19 @@ int pic_set_push_schedule(pic_ctx* c, int32_t schedule) {
 int32_t pic_push_schedule(const pic_ctx* c, int32_t support) {
     if (!c || support < 2 || support > 4) return -1;
     PhasePlan* p = nullptr;
-    if (getPlan(const_cast<pic_ctx*>(c), support, true, &p) != PIC_OK) return -1;
+    if (getPlan(const_cast<pic_ctx*>(c), support, &p) != PIC_OK) return -1;
     return p->single ? PIC_PUSH_SCHEDULE_SINGLE : PIC_PUSH_SCHEDULE_PHASES;
 }
 
 int32_t pic_num_push_phases(const pic_ctx* c, int32_t fused) {
+    (void)fused;  // both forms run over the same phases
     if (!c) return -1;
     pic_ctx* m = const_cast<pic_ctx*>(c);
     int maxPh = 0;
     for (const SpeciesMem& s : m->sp) {
         if (s.desc.pusher == PIC_PUSHER_NONE) continue;
         PhasePlan* p = nullptr;
-        if (getPlan(m, supportOf(s.desc.shape), fused != 0, &p) != PIC_OK) return -1;
+        if (getPlan(m, supportOf(s.desc.shape), &p) != PIC_OK) return -1;
         maxPh = std::max(maxPh, static_cast<int>(p->count.size()));
     }
     return maxPh;
@@ -2277,7 +2278,7 @@ int oneStep(pic_ctx* c) {
     auto const groups = pushGroups(c, -1, true);
     if (!groups.empty()) {
         PhasePlan* plan = nullptr;
-        if ((r = getPlan(c, supportOf(c->sp[groups[0][0]].desc.shape), true, &plan)) != PIC_OK) return r;
+        if ((r = getPlan(c, supportOf(c->sp[groups[0][0]].desc.shape), &plan)) != PIC_OK) return r;
         freshJ = plan->single;
     }
     if (!freshJ && (r = pic_current_reset(c)) != PIC_OK) return r;
@@ -2302,7 +2303,7 @@ int stepGraphs(pic_ctx* c, int32_t nsteps) {
             for (const SpeciesMem& m : c->sp) {
                 if (m.desc.pusher == PIC_PUSHER_NONE) continue;
                 PhasePlan* plan = nullptr;
-                int const r = getPlan(c, supportOf(m.desc.shape), true, &plan);
+                int const r = getPlan(c, supportOf(m.desc.shape), &plan);
                 if (r != PIC_OK) return r;
             }
             PIC_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
@@ -2944,7 +2945,7 @@ int ensUploadTables(pic_ensemble* e) {
                 if (m.desc.pusher != PIC_PUSHER_NONE) a.sp[k++] = m.dev;
             a.nsp = k;
             a.scList = nullptr;
-            if (e->single) a.tileOut = c->plans[e->supp - 2][1].tiles;
+            if (e->single) a.tileOut = c->plans[e->supp - 2].tiles;
             push[i] = a;
             pic::FieldArgs f = makeFieldArgs(c);
             for (int d = 0; d < 3; ++d) {
@@ -2961,7 +2962,7 @@ int ensUploadTables(pic_ensemble* e) {
         std::vector<pic::GatherEntry> gather(n);
         for (int i = 0; i < n; ++i) {
             pic_ctx* c = e->sims[i];
-            const PhasePlan& plan = c->plans[e->supp - 2][1];
+            const PhasePlan& plan = c->plans[e->supp - 2];
             gather[i] = pic::GatherEntry{c->g, plan.tiles, plan.colour, {c->J[0], c->J[1], c->J[2]}};
         }
         if (!e->dGather && ensAlloc(e, &e->dGather, static_cast<size_t>(n)) != PIC_OK) return PIC_E_HIP;
@@ -2992,7 +2993,7 @@ int ensBuildWork(pic_ensemble* e) {
     std::vector<PhasePlan*> plans(n);
     size_t nph = 0;
     for (int i = 0; i < n; ++i) {
-        int const r = getPlan(e->sims[i], e->supp, true, &plans[i]);
+        int const r = getPlan(e->sims[i], e->supp, &plans[i]);
         if (r != PIC_OK) return r;
         nph = std::max(nph, plans[i]->count.size());
     }

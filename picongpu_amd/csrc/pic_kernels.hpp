@@ -106,7 +106,7 @@ struct PushArgs {
     SpeciesDev sp[PIC_MAX_SPECIES];
     const int32_t* scList;  // supercells of this launch, in launch order
     int stageShift;  // 1: the epilogue also moves the leavers to the outbox and compacts the supercell
-    // non-null (fused push + deposit only): every supercell in one launch,
+    // non-null (fused and deposit only): every supercell in one launch,
     // each leaving its J tile at tileOut[sc * tile elements], as the floats
     // the flush would add to J (zero where it adds none), for
     // launchGatherFlush instead of adding it to J

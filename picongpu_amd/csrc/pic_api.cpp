@@ -818,7 +818,7 @@ struct pic_ctx {
     unsigned long long* countOut = nullptr;
     double* diagBuf = nullptr;  // ncells doubles, allocated on first use
     int jexp = 40;
-    // [supp-2][fused]
+    // [supp-2]
     PhasePlan plans[3];
     int cus = 256;          // compute units of the device
     int pushSchedule = 0;   // PIC_PUSH_SCHEDULE_*
@@ -946,11 +946,17 @@ int buildPlan(pic_ctx* c, int supp, PhasePlan& plan) {
     plan.host = list;
     if (devAlloc(c, &plan.dList, list.size()) != PIC_OK) return PIC_E_HIP;
     PIC_HIP(hipMemcpyAsync(plan.dList, list.data(), list.size() * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
-    // one launch for every supercell when the largest phase would leave more
-    // than half of the CUs' workgroup slots idle (small boxes)
     int const most = *std::max_element(plan.count.begin(), plan.count.end());
+    // One launch for every supercell below six supercells per CU in the
+    // largest phase: a phase of a few rounds of workgroups ends with a partly
+    // empty one, every phase again, which costs more than the tiles' way
+    // through memory. Measured, ms a step by phases and in one launch: 768 a
+    // phase 1.40 and 0.99 (laser box 96x512x64, PQS), 1.64 and 1.46 (TSC);
+    // 1024 a phase 6.27 and 5.91 (two species, TSC); 1536 a phase 0.865 and
+    // 0.855 (CIC); 2304 a phase 1.97 and 2.05 (laser, PQS); 4096 a phase 2.06
+    // and 2.15 (CIC), 4.50 and 5.04 (laser).
     plan.single = c->pushSchedule == PIC_PUSH_SCHEDULE_SINGLE ||
-                  (c->pushSchedule == PIC_PUSH_SCHEDULE_AUTO && most < 2 * c->cus);
+                  (c->pushSchedule == PIC_PUSH_SCHEDULE_AUTO && most < 6 * c->cus);
     if (plan.single) {
         std::vector<uint8_t> colour;
         for (int d = 0; d < 3; ++d) {

@@ -100,6 +100,30 @@ def test_deposit_unfused_bit_exact(name, make):
     sim.close()
 
 
+@pytest.mark.parametrize("schedule", [abi.PUSH_SCHEDULE_PHASES, abi.PUSH_SCHEDULE_SINGLE], ids=["phases", "single"])
+@pytest.mark.parametrize("open_", [False, True], ids=["periodic", "open"])
+@pytest.mark.parametrize("shape", [abi.SHAPE_CIC, abi.SHAPE_TSC, abi.SHAPE_PQS], ids=["cic", "tsc", "pqs"])
+def test_deposit_stage_schedules_bit_exact(shape, open_, schedule):
+    """The stages one by one with two depositing species (the second one's
+    deposit adds to the first one's J), in phases and in one launch."""
+    st = small_two_species(shape)
+    if open_:
+        open_box(st, boundary=(1, 1, 0))
+    print(f"case deposit stage shape={shape} grid={st.grid} open={open_} schedule={schedule}", flush=True)
+    sim, ora, _ = H.make_pair(st, e_amp=1e-3, b_amp=1e-3)
+    sim.set_push_schedule(schedule)
+    for it in range(2):
+        for x in (sim, ora):
+            x.current_reset()
+            x.push(-1, False)
+            x.shift(-1)
+            x.deposit(-1)
+        for sp in range(len(st.species)):
+            H.assert_frames_equal(sim.read_frames(sp), ora.get_frames(sp), f"stages step {it} species {sp}")
+        H.assert_field_equal(sim.read_field(abi.FIELD_J), ora.get_field(abi.FIELD_J), f"stages step {it} J")
+    sim.close()
+
+
 @pytest.mark.parametrize("open_", [False, True], ids=["periodic", "open"])
 def test_shift_bit_exact(open_):
     st = small_thermal(abi.SHAPE_CIC, abi.PUSHER_BORIS, u=0.3)

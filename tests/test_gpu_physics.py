@@ -253,6 +253,23 @@ def test_gauss_residual_matches_oracle():
     sim.close()
 
 
+@pytest.mark.parametrize("grid", [(16, 16, 8), (24, 16, 12)], ids=["16x16x8", "24x16x12"])
+@pytest.mark.parametrize("shape", [abi.SHAPE_CIC, abi.SHAPE_PQS], ids=["cic", "pqs"])
+def test_charge_tile_matches_oracle(shape, grid):
+    """The per-supercell charge tile of the Gauss residual: with two supercells
+    along an axis its nodes meet the same neighbour's on both sides."""
+    st = small_thermal(shape, grid=grid)
+    print(f"case charge tile shape={shape} grid={grid}", flush=True)
+    sim, ora, _ = H.make_pair(st)
+    k = sim.constants()
+    r_gpu = sim.gauss_residual()
+    rho = ora.charge_density()
+    r_ora = float(np.float32(k.eps0)) * ora.div_e() - rho
+    # as above: 1e-12 of the density is far above FP64 round-off of the sums
+    assert np.abs(r_gpu - r_ora).max() <= 1e-12 * np.abs(rho).max()
+    sim.close()
+
+
 def test_full_size_kelvin_helmholtz_properties():
     """256^3, 2 x 16 ppc (536,870,912 particles): counts conserved, no capacity
     error, Gauss residual unchanged to FP32 round-off (charge conservation),

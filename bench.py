@@ -47,7 +47,7 @@ HBM_PEAK_GBS = 8000.0
 # Command: rocprofv3 --pmc FETCH_SIZE (then WRITE_SIZE) -- python3 bench.py
 # --steps 1 --warmup 1 --no-cpu-baseline --no-adjoint --no-ensemble --calibrate-copy
 MEASURED_TRAFFIC = {
-    ("kelvin_helmholtz", (256, 256, 256)): {"fetch_kib": 896118.6, "write_kib": 1340060.5, "fetch_scale": 2.0,
+    ("kelvin_helmholtz", (256, 256, 256)): {"fetch_kib": 1094990.0, "write_kib": 1084480.0, "fetch_scale": 2.0,
                                             "write_scale": 1.0},
 }
 # Instruction counters of the fused push/deposit kernel on this workload,
@@ -60,12 +60,12 @@ MEASURED_TRAFFIC = {
 # the push kernel that also damps the weightings in the layers
 # (kPushDepositPml).
 MEASURED_INSTS = {
-    ("kelvin_helmholtz", (256, 256, 256), "none"): {"valu": 826.64e6, "lds": 90.875e6, "lds_bank_conflict": 488.81e6,
-                                                    "grbm_gui_active": 31.881e6},
-    ("laser_plasma", (192, 1536, 192), "exponential"): {"valu": 495.28e6, "lds": 52.231e6,
-                                                        "lds_bank_conflict": 197.88e6, "grbm_gui_active": 20.089e6},
-    ("laser_plasma", (192, 1536, 192), "pml"): {"valu": 517.90e6, "lds": 52.208e6, "lds_bank_conflict": 197.81e6,
-                                                "grbm_gui_active": 22.487e6},
+    ("kelvin_helmholtz", (256, 256, 256), "none"): {"valu": 708.50e6, "lds": 98.163e6, "lds_bank_conflict": 323.53e6,
+                                                    "grbm_gui_active": 25.764e6},
+    ("laser_plasma", (192, 1536, 192), "exponential"): {"valu": 375.31e6, "lds": 52.880e6,
+                                                        "lds_bank_conflict": 134.53e6, "grbm_gui_active": 14.656e6},
+    ("laser_plasma", (192, 1536, 192), "pml"): {"valu": 390.52e6, "lds": 52.857e6, "lds_bank_conflict": 134.46e6,
+                                                "grbm_gui_active": 15.930e6},
 }
 # VALU issue peak: a wave64 VALU instruction occupies one of the 1,024 SIMDs
 # (256 CUs x 4) for 4 cycles at the 2.4 GHz peak engine clock

@@ -125,7 +125,9 @@ struct PushLds {
                         kLeaverListLds * 4;
     // 16-byte multiple: the int64 J tile that follows needs 8-byte aligned LDS addresses
     static constexpr int LO_BYTES = (((EB_BYTES > EPI_BYTES ? EB_BYTES : EPI_BYTES) + 15) / 16) * 16;
-    static constexpr int BYTES = LO_BYTES + J_ELEMS * 8;
+    // odd support: a byte per wave, whether it staged a non-finite node
+    static constexpr int BAD_AT = LO_BYTES + J_ELEMS * 8;
+    static constexpr int BYTES = BAD_AT + (MODE != 2 && EBTile<SUPP>::ODD ? kPushWaves : 0);
 };
 
 // J += the tile's component C. A thread's J values are loaded together, then
@@ -293,6 +295,7 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
     uint32_t* const sWaveCnt = sPre + kPushMaxIters * kPushWaves + 1;
     GroupScratch& sGroup = *reinterpret_cast<GroupScratch*>(sWaveCnt + kPushWaves * kNumDirs);
     uint32_t* const sList = reinterpret_cast<uint32_t*>(&sGroup + 1);
+    uint8_t* const sBad = reinterpret_cast<uint8_t*>(smem + PushLds<SUPP, MODE>::BAD_AT);
 
     if (halted(a.g)) return;  // uniform: a later step of an overflowed simulation
     int const sx = sc % a.g.nscx;
@@ -350,6 +353,15 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
 #pragma unroll
             for (int u = 0; u < NU; ++u) v[c][u] = src[gi[u]];
         }
+        if (T::ODD) {
+            // the sum of all is non-finite if one is (an overflow of finite ones only costs time)
+            float sum = 0.0f;
+#pragma unroll
+            for (int u = 0; u < NU; ++u)
+                sum += ((v[0][u] + v[1][u]) + (v[2][u] + v[3][u])) + (v[4][u] + v[5][u]);
+            uint8_t const any = __ballot(__builtin_amdgcn_classf(sum, 0x207)) != 0ull ? 1 : 0;  // NaN, -Inf, +Inf
+            if ((tid & 63) == 0) sBad[tid >> 6] = any;
+        }
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
             int tx, ty, tz;
@@ -378,6 +390,14 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
         for (int t = tid; t < J_ELEMS / 2; t += kPushThreads) reinterpret_cast<ulonglong2*>(sJ)[t] = make_ulonglong2(0ull, 0ull);
     }
     __syncthreads();
+    // the same in every lane: not 0 when the tile holds a non-finite node (odd
+    // support; read here, first needed after the particle's loads)
+    uint32_t badNodes = 0u;
+    if (MODE != 2 && EBTile<SUPP>::ODD) {
+        static_assert(kPushWaves == 8, "a byte per wave");
+        uint2 const b = *reinterpret_cast<const uint2*>(sBad);
+        badNodes = b.x | b.y;
+    }
 
     DepositConsts dk;
     dk.cell[0] = a.cell[0];
@@ -428,8 +448,10 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
                 if (MODE != 2) {
                     WeightTerms const terms = weightTerms<PUSHER>(mass, charge);
                     GatherWeights<SUPP> const gw(pos, lx, ly, lz);
-                    Vec3 const e{gather1<SUPP, 0>(sEB, gw), gather1<SUPP, 1>(sEB, gw), gather1<SUPP, 2>(sEB, gw)};
-                    Vec3 const b{gather1<SUPP, 3>(sEB, gw), gather1<SUPP, 4>(sEB, gw), gather1<SUPP, 5>(sEB, gw)};
+                    Vec3 e{gather1<SUPP, 0>(sEB, gw), gather1<SUPP, 1>(sEB, gw), gather1<SUPP, 2>(sEB, gw)};
+                    Vec3 b{gather1<SUPP, 3>(sEB, gw), gather1<SUPP, 4>(sEB, gw), gather1<SUPP, 5>(sEB, gw)};
+                    if constexpr (EBTile<SUPP>::ODD)
+                        if (badNodes) gatherStencil<SUPP>(sEB, pos, lx, ly, lz, e, b);
                     Vec3 vel;
                     if (PUSHER == PIC_PUSHER_VAY)
                         pushVay(e, b, mom, vel, mass, charge, terms);

@@ -330,7 +330,8 @@ struct GatherWeights {
 // Component C at the particle. Each partial sum starts at its first term; the
 // reference adds that term to 0.0, which differs only in the sign of an
 // all-zero sum (a zero field value adds nothing to a momentum, whatever its
-// sign), as does the term of a padded zero weight. Every further term is a
+// sign), as does the term of a padded zero weight while its node is finite
+// (gatherStencil below covers the others). Every further term is a
 // multiply-add. One address for the stencil's first node: the others are
 // constant offsets from it, which the LDS reads take as immediates.
 template <int SUPP, int C>
@@ -364,6 +365,63 @@ __device__ __forceinline__ float gather1(const float* __restrict__ tile, const G
         result_z = z == 0 ? result_y * g.w[2][hz][0] : mad(result_y, g.w[2][hz][z], result_z);
     }
     return result_z;
+}
+
+// The six components from a tile of odd support that holds a non-finite node:
+// gather1's padded node lies outside the stencil and 0 * Inf is NaN, so here
+// the rows are read node by node. Rare, so it is kept small instead of fast: a
+// loop over the components that forms its weights anew (gather1 again, with
+// the padded node masked, made the particle loop spill). Finding out whether a
+// tile needs it costs finite boxes 0.3 to 0.7 % of a step (256^3 shear flow
+// 126.9 and 127.3 ms a pass, 72x88x36 streams 1.921 and 1.935 ms).
+template <int SUPP>
+__device__ __forceinline__ void gatherStencil(const float* __restrict__ tile, Vec3 pos, int lx, int ly, int lz, Vec3& e,
+                                              Vec3& b) {
+    using T = EBTile<SUPP>;
+    static_assert(T::ODD && SUPP == 3, "even supports read exactly their stencil");
+    // opaque, so that nothing of gather1's is kept alive for this
+    asm volatile("" : "+v"(pos.x), "+v"(pos.y), "+v"(pos.z), "+v"(lx), "+v"(ly), "+v"(lz));
+#pragma unroll 1
+    for (int c = 0; c < 6; ++c) {
+        // the component's geometry (uniform)
+        int off = 0, pitch = 0, plane = 0, lox = 0, loy = 0, loz = 0;
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+            if (k == c) {
+                off = T::off(k);
+                pitch = T::pitch(k);
+                plane = T::plane(k);
+                lox = T::lo(k, 0);
+                loy = T::lo(k, 1);
+                loz = T::lo(k, 2);
+            }
+        bool const hx = c < 3 ? c == 0 : c != 3, hy = c < 3 ? c == 1 : c != 4, hz = c < 3 ? c == 2 : c != 5;
+        float wx[SUPP], wy[SUPP], wz[SUPP];
+        int const bx = lx + (hx ? nodeWeights<SUPP, true>(pos.x, wx) : nodeWeights<SUPP, false>(pos.x, wx)) + T::begin + lox;
+        int const by = ly + (hy ? nodeWeights<SUPP, true>(pos.y, wy) : nodeWeights<SUPP, false>(pos.y, wy)) + T::begin + loy;
+        int const bz = lz + (hz ? nodeWeights<SUPP, true>(pos.z, wz) : nodeWeights<SUPP, false>(pos.z, wz)) + T::begin + loz;
+        const float* const corner = tile + off + (bz * plane + by * pitch + bx);
+        float result_z = 0.0f;
+#pragma unroll
+        for (int z = 0; z < SUPP; ++z) {
+            float result_y = 0.0f;
+#pragma unroll
+            for (int y = 0; y < SUPP; ++y) {
+                const float* const row = corner + z * plane + y * pitch;
+                float result_x = row[0] * wx[0];
+#pragma unroll
+                for (int x = 1; x < SUPP; ++x) result_x = mad(row[x], wx[x], result_x);
+                result_y = y == 0 ? result_x * wy[0] : mad(result_x, wy[y], result_y);
+            }
+            result_z = z == 0 ? result_y * wz[0] : mad(result_y, wz[z], result_z);
+        }
+        if (c == 0) e.x = result_z;
+        if (c == 1) e.y = result_z;
+        if (c == 2) e.z = result_z;
+        if (c == 3) b.x = result_z;
+        if (c == 4) b.y = result_z;
+        if (c == 5) b.z = result_z;
+    }
 }
 
 // ---------------------------------------------------------------------------

@@ -131,6 +131,53 @@ def test_ultra_relativistic_momenta(pusher):
     run_pair(st, cells, pos, mom, w, frames=6, nsteps=3)
 
 
+@pytest.mark.parametrize("open_", [0, 1], ids=["periodic", "open-x"])
+@pytest.mark.parametrize("shape", [abi.SHAPE_CIC, abi.SHAPE_TSC, abi.SHAPE_PQS], ids=["cic", "tsc", "pqs"])
+def test_non_finite_nodes_outside_the_stencil(shape, open_):
+    """NaN and Inf nodes reach the particles whose stencil holds them and no
+    others: every particle keeps its distance to them along x by a node more
+    than its support at least, on both sides, at both parities of the row's
+    first node, and is pushed as the oracle pushes it."""
+    st = thermal(shape=shape, frames=6)
+    st.boundary = (open_, 0, 0)
+    counts = [600] * 12
+    print(f"case non-finite nodes shape={shape} open={open_}", flush=True)
+    cells, pos, mom, w = crafted(st, counts, seed=31)
+    planes = {4: np.nan, 11: np.inf}  # x of the non-finite nodes; every component lies at x or x + 1/2
+    half = {abi.SHAPE_CIC: 1.0, abi.SHAPE_TSC: 1.5, abi.SHAPE_PQS: 2.0}[shape]
+    x = cells[:, 0] + pos[:, 0].astype(np.float64)
+    far = np.ones(len(x), bool)
+    for px in planes:
+        for d in (px, px + 0.5):
+            dist = np.abs((x - d + GRID[0] / 2) % GRID[0] - GRID[0] / 2)
+            far &= dist > half
+    assert far.sum() > 1000
+    f = setups.bin_frames(st, 0, cells[far], pos[far], mom[far], w[far], frames_per_sc=6)
+    E, B = H.random_fields(st, 17, 1e-3, 1e-3)
+    for fld in (E, B):
+        v = fld.reshape(3, GRID[2], GRID[1], GRID[0])
+        for px, value in planes.items():
+            v[:, ::2, :, px] = value
+            v[:, 1::2, :, px] = -value
+    sim = abi.Simulation(st.config())
+    sim.write_frames(0, f)
+    sim.load_field(abi.FIELD_E, E)
+    sim.load_field(abi.FIELD_B, B)
+    ora = O.Oracle(st, 32, 0, jexp=sim.j_scale_exp())
+    ora.set_frames(0, f)
+    ora.set_field(abi.FIELD_E, E)
+    ora.set_field(abi.FIELD_B, B)
+    for q in (sim, ora):
+        q.current_reset()
+        q.push(-1, True)
+    out = sim.read_frames(0)
+    assert np.isfinite(out["mom"][:, H.occupied(out)]).all()
+    H.assert_frames_equal(out, ora.get_frames(0), "push beside non-finite nodes")
+    H.assert_field_equal(sim.read_field(abi.FIELD_J), ora.get_field(abi.FIELD_J), "J")
+    sim.close()
+    ora.close()
+
+
 def converging(st, counts, seed, u):
     """crafted() particles whose momenta point towards the box centre, so the
     supercells there fill up over the steps."""

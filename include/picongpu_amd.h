@@ -438,7 +438,9 @@ int32_t pic_num_push_phases(const pic_ctx* ctx, int32_t fused);
  * adding its covering tiles in phase order. Both give the same J, bit for
  * bit; SINGLE fills the GPU when a phase holds fewer supercells than the
  * device has workgroup slots. AUTO (the default) takes SINGLE when the
- * largest phase has fewer supercells than six times the compute units. The
+ * largest phase has fewer supercells than six times the compute units. SINGLE
+ * keeps a tile per supercell in device memory (9.1 KB with CIC, 16.6 KB with
+ * TSC and PQS, per shape support in use: at most about 0.4 GB under AUTO). The
  * deposit stage (pic_deposit) follows the same schedule. An
  * ensemble member's schedule cannot change (PIC_E_INVALID): the ensemble's
  * batched launches use its plans. pic_push_schedule reports the schedule of

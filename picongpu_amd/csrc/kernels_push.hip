@@ -314,8 +314,7 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
         if (MODE != 2 && tid < kOffStride) {
             for (int s = 0; s < a.nsp; ++s) a.sp[s].outOff[(size_t)sc * kOffStride + tid] = 0u;
         }
-        if (MODE != 0 && a.tileOut)  // an empty tile for the gather flush
-            for (int t = tid; t < J_ELEMS; t += blockDim.x) a.tileOut[(size_t)sc * J_ELEMS + t] = 0.0f;
+        if (MODE != 0 && a.tileOut && tid == 0) a.tileHeld[sc] = 0u;  // the gather flush passes its tile over
         return;
     }
 
@@ -565,6 +564,7 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
             long long const acc = fixedTileValue(sJ[t]);
             a.tileOut[(size_t)sc * J_ELEMS + t] = acc == 0 ? 0.0f : (float)((double)acc * a.jinv);
         }
+        if (tid == 0) a.tileHeld[sc] = 1u;
     } else if (MODE != 0) {
         bool const inside = ox >= DLO && ox + SCX + UPM <= a.g.nx && oy >= DLO && oy + SCY + UPM <= a.g.ny &&
                             oz >= DLO && oz + SCZ + UPM <= a.g.nz;
@@ -782,11 +782,12 @@ __device__ __forceinline__ CoverAxis coverAxis(int s, int nsc, bool open, const 
 // phase (zeros add nothing). A phase's index is colour_x + ncol_x (colour_y +
 // ncol_y colour_z), so visiting z, then y, then x neighbours each in
 // ascending colour is ascending phase (every supercell covering a cell lies
-// in another phase).
+// in another phase). Bit k of `held` is 0 for a neighbour beyond an open
+// border and for one whose tile is not written.
 template <int SUPP, int C>
 __device__ __forceinline__ void gatherFlushComponent(const GridDev& g, const float* __restrict__ tiles,
                                                      const CoverAxis& ax, const CoverAxis& ay, const CoverAxis& az,
-                                                     float* __restrict__ J, size_t cell, bool fresh) {
+                                                     uint32_t held, float* __restrict__ J, size_t cell, bool fresh) {
     constexpr int DLO = Esirkepov<SUPP>::lowerMargin;
     using TG = JTileGeom<DLO, Esirkepov<SUPP>::upperMargin>;
     constexpr int J_ELEMS = PushLds<SUPP, 1>::J_ELEMS;
@@ -800,12 +801,12 @@ __device__ __forceinline__ void gatherFlushComponent(const GridDev& g, const flo
         int const a = k / 9, b = (k / 3) % 3, d = k % 3;
         int const ox = DLO - SCX * ax.step[d], oy = DLO - SCY * ay.step[b], oz = DLO - SCZ * az.step[a];
         w[k] = 0.0f;
-        if (ax.sc[d] < 0 || ay.sc[b] < 0 || az.sc[a] < 0) continue;  // uniform
         int const sc = ax.sc[d] + g.nscx * (ay.sc[b] + g.nscy * az.sc[a]);
-        const float* const t = tiles + (size_t)sc * J_ELEMS + TG::off(C) + (oz * EY + oy) * EX + ox;
-        if ((unsigned)(lx + ox) < (unsigned)EX && (unsigned)(ly + oy) < (unsigned)EY &&
-            (unsigned)(lz + oz) < (unsigned)EZ)
-            w[k] = t[lane];
+        const float* const t = tiles + (ptrdiff_t)sc * J_ELEMS + TG::off(C) + (oz * EY + oy) * EX + ox;
+        // one predicate per load (no branch), so that the loads stay together
+        bool const covers = ((unsigned)(lx + ox) < (unsigned)EX) & ((unsigned)(ly + oy) < (unsigned)EY) &
+                            ((unsigned)(lz + oz) < (unsigned)EZ) & (((held >> k) & 1u) != 0u);
+        if (covers) w[k] = t[lane];
     }
     float v = fresh ? 0.0f : J[cell];
 #pragma unroll
@@ -816,9 +817,14 @@ __device__ __forceinline__ void gatherFlushComponent(const GridDev& g, const flo
 // J of one supercell (256 threads). fresh: J holds nothing yet (the sums
 // start at zero and every cell is written), so the step needs no reset of J.
 // 64^3 cells (CIC): 21 us a launch plus 5 for the reset with a loop of
-// dependent loads over the candidates of every cell.
+// dependent loads over the candidates of every cell. The tiles of supercells
+// without particles are neither written nor read: with zero tiles a nearly
+// empty box of 192x128x160 cells (TSC, 15,360 supercells) took 0.40 ms a step
+// in one launch and 0.28 by phases, now 0.25; a laser box of 96x512x64 cells,
+// four fifths vacuum, 8.76 and 7.59 ms for ten steps.
 template <int SUPP>
 __device__ __forceinline__ void gatherFlushSC(const GridDev& g, const float* __restrict__ tiles,
+                                              const uint32_t* __restrict__ tileHeld,
                                               const uint8_t* __restrict__ colour, float* J0, float* J1, float* J2,
                                               int sc, bool fresh) {
     int const sx = sc % g.nscx, sy = (sc / g.nscx) % g.nscy, sz = sc / (g.nscx * g.nscy);
@@ -826,19 +832,29 @@ __device__ __forceinline__ void gatherFlushSC(const GridDev& g, const float* __r
     CoverAxis const ay = coverAxis(sy, g.nscy, (g.open & 2) != 0, colour + g.nscx);
     CoverAxis const az = coverAxis(sz, g.nscz, (g.open & 4) != 0, colour + g.nscx + g.nscy);
     int const tid = threadIdx.x;
+    uint32_t held;
+    {  // lane k of each wave looks at neighbour k
+        int const k = tid & 63, a = k / 9, b = (k / 3) % 3, d = k % 3;
+        int const x = d == 0 ? ax.sc[0] : (d == 1 ? ax.sc[1] : ax.sc[2]);
+        int const y = b == 0 ? ay.sc[0] : (b == 1 ? ay.sc[1] : ay.sc[2]);
+        int const z = a == 0 ? az.sc[0] : (a == 1 ? az.sc[1] : az.sc[2]);
+        bool const inBox = k < 27 && x >= 0 && y >= 0 && z >= 0;
+        held = (uint32_t)__ballot(inBox && tileHeld[x + g.nscx * (y + g.nscy * z)] != 0u);
+    }
     size_t const cell = (size_t)(sx * SCX + (tid & 7)) +
                         (size_t)g.nx * ((size_t)(sy * SCY + ((tid >> 3) & 7)) + (size_t)g.ny * (sz * SCZ + (tid >> 6)));
-    gatherFlushComponent<SUPP, 0>(g, tiles, ax, ay, az, J0, cell, fresh);
-    gatherFlushComponent<SUPP, 1>(g, tiles, ax, ay, az, J1, cell, fresh);
-    gatherFlushComponent<SUPP, 2>(g, tiles, ax, ay, az, J2, cell, fresh);
+    gatherFlushComponent<SUPP, 0>(g, tiles, ax, ay, az, held, J0, cell, fresh);
+    gatherFlushComponent<SUPP, 1>(g, tiles, ax, ay, az, held, J1, cell, fresh);
+    gatherFlushComponent<SUPP, 2>(g, tiles, ax, ay, az, held, J2, cell, fresh);
 }
 
 template <int SUPP>
 __global__ __launch_bounds__(SCV) void kGatherFlush(GridDev g, const float* __restrict__ tiles,
+                                                     const uint32_t* __restrict__ held,
                                                      const uint8_t* __restrict__ colour, float* J0, float* J1,
                                                      float* J2, int fresh) {
     if (halted(g)) return;
-    gatherFlushSC<SUPP>(g, tiles, colour, J0, J1, J2, (int)blockIdx.x, fresh != 0);
+    gatherFlushSC<SUPP>(g, tiles, held, colour, J0, J1, J2, (int)blockIdx.x, fresh != 0);
 }
 
 template <int SUPP>
@@ -847,7 +863,7 @@ __global__ __launch_bounds__(SCV) void kGatherFlushBatch(const GatherEntry* __re
     int2 const it = blocks[blockIdx.x];
     const GatherEntry& e = table[it.x];
     if (halted(e.g)) return;
-    gatherFlushSC<SUPP>(e.g, e.tiles, e.colour, e.J[0], e.J[1], e.J[2], it.y, fresh != 0);
+    gatherFlushSC<SUPP>(e.g, e.tiles, e.held, e.colour, e.J[0], e.J[1], e.J[2], it.y, fresh != 0);
 }
 
 hipError_t launchGatherFlushBatch(int supp, const GatherEntry* table, const int2* blocks, int nblocks, bool fresh,
@@ -863,14 +879,14 @@ hipError_t launchGatherFlushBatch(int supp, const GatherEntry* table, const int2
     return hipGetLastError();
 }
 
-hipError_t launchGatherFlush(int supp, const GridDev& g, const float* tiles, const uint8_t* colour,
-                             float* const J[3], bool fresh, hipStream_t s) {
+hipError_t launchGatherFlush(int supp, const GridDev& g, const float* tiles, const uint32_t* held,
+                             const uint8_t* colour, float* const J[3], bool fresh, hipStream_t s) {
     dim3 const grid((unsigned)(g.nscx * g.nscy * g.nscz)), block(SCV);
     int const f = fresh ? 1 : 0;
     switch (supp) {
-        case 2: hipLaunchKernelGGL(kGatherFlush<2>, grid, block, 0, s, g, tiles, colour, J[0], J[1], J[2], f); break;
-        case 3: hipLaunchKernelGGL(kGatherFlush<3>, grid, block, 0, s, g, tiles, colour, J[0], J[1], J[2], f); break;
-        case 4: hipLaunchKernelGGL(kGatherFlush<4>, grid, block, 0, s, g, tiles, colour, J[0], J[1], J[2], f); break;
+        case 2: hipLaunchKernelGGL(kGatherFlush<2>, grid, block, 0, s, g, tiles, held, colour, J[0], J[1], J[2], f); break;
+        case 3: hipLaunchKernelGGL(kGatherFlush<3>, grid, block, 0, s, g, tiles, held, colour, J[0], J[1], J[2], f); break;
+        case 4: hipLaunchKernelGGL(kGatherFlush<4>, grid, block, 0, s, g, tiles, held, colour, J[0], J[1], J[2], f); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -714,6 +714,7 @@ struct PhasePlan {
     // launch per phase; chosen when the phases are too small to fill the GPU
     bool single = false;
     float* tiles = nullptr;               // nsc tiles
+    uint32_t* held = nullptr;             // PushArgs::tileHeld
     uint8_t* colour = nullptr;            // checkerboard colour per supercell index along x, y, z
 };
 
@@ -954,7 +955,10 @@ int buildPlan(pic_ctx* c, int supp, PhasePlan& plan) {
     // phase 1.40 and 0.99 (laser box 96x512x64, PQS), 1.64 and 1.46 (TSC);
     // 1024 a phase 6.27 and 5.91 (two species, TSC); 1536 a phase 0.865 and
     // 0.855 (CIC); 2304 a phase 1.97 and 2.05 (laser, PQS); 4096 a phase 2.06
-    // and 2.15 (CIC), 4.50 and 5.04 (laser).
+    // and 2.15 (CIC), 4.50 and 5.04 (laser). Boxes with 2,000 particles in one
+    // corner, where a phase costs little and supercells without particles
+    // leave no tile: 512 a phase 0.147 and 0.092 (CIC), 0.217 and 0.149 (TSC);
+    // 960 a phase 0.279 and 0.245 (TSC), 0.328 and 0.250 (PQS).
     plan.single = c->pushSchedule == PIC_PUSH_SCHEDULE_SINGLE ||
                   (c->pushSchedule == PIC_PUSH_SCHEDULE_AUTO && most < 6 * c->cus);
     if (plan.single) {
@@ -964,6 +968,7 @@ int buildPlan(pic_ctx* c, int supp, PhasePlan& plan) {
             for (int v : col[d]) colour.push_back(static_cast<uint8_t>(v));
         }
         if (devAlloc(c, &plan.tiles, static_cast<size_t>(c->nsc) * pic::pushTileElems(supp), false) != PIC_OK ||
+            devAlloc(c, &plan.held, static_cast<size_t>(c->nsc), false) != PIC_OK ||
             devAlloc(c, &plan.colour, colour.size(), false) != PIC_OK)
             return PIC_E_HIP;
         PIC_HIP(hipMemcpyAsync(plan.colour, colour.data(), colour.size(), hipMemcpyHostToDevice, c->stream));
@@ -1114,9 +1119,10 @@ int runPush(pic_ctx* c, int32_t species, int mode, bool stageShift = false, bool
             // tiles gathered into J in phase order
             a.scList = plan->dList;
             a.tileOut = plan->tiles;
+            a.tileHeld = plan->held;
             TimerScope ts(c, PIC_TIMER_PUSH);
             PIC_HIP(pic::launchPush(supp, pusher, mode, scheme, a, c->nsc, c->stream));
-            PIC_HIP(pic::launchGatherFlush(supp, c->g, plan->tiles, plan->colour, c->J, freshJ, c->stream));
+            PIC_HIP(pic::launchGatherFlush(supp, c->g, plan->tiles, plan->held, plan->colour, c->J, freshJ, c->stream));
             freshJ = false;
             continue;
         }
@@ -1667,6 +1673,7 @@ int pic_set_push_schedule(pic_ctx* c, int32_t schedule) {
         if (!p.valid) continue;
         devFree(c, p.dList);
         devFree(c, p.tiles);
+        devFree(c, p.held);
         devFree(c, p.colour);
         p = PhasePlan{};
     }
@@ -2951,7 +2958,10 @@ int ensUploadTables(pic_ensemble* e) {
                 if (m.desc.pusher != PIC_PUSHER_NONE) a.sp[k++] = m.dev;
             a.nsp = k;
             a.scList = nullptr;
-            if (e->single) a.tileOut = c->plans[e->supp - 2].tiles;
+            if (e->single) {
+                a.tileOut = c->plans[e->supp - 2].tiles;
+                a.tileHeld = c->plans[e->supp - 2].held;
+            }
             push[i] = a;
             pic::FieldArgs f = makeFieldArgs(c);
             for (int d = 0; d < 3; ++d) {
@@ -2969,7 +2979,7 @@ int ensUploadTables(pic_ensemble* e) {
         for (int i = 0; i < n; ++i) {
             pic_ctx* c = e->sims[i];
             const PhasePlan& plan = c->plans[e->supp - 2];
-            gather[i] = pic::GatherEntry{c->g, plan.tiles, plan.colour, {c->J[0], c->J[1], c->J[2]}};
+            gather[i] = pic::GatherEntry{c->g, plan.tiles, plan.held, plan.colour, {c->J[0], c->J[1], c->J[2]}};
         }
         if (!e->dGather && ensAlloc(e, &e->dGather, static_cast<size_t>(n)) != PIC_OK) return PIC_E_HIP;
         PIC_HIP(hipMemcpyAsync(e->dGather, gather.data(), n * sizeof(pic::GatherEntry), hipMemcpyHostToDevice,

@@ -111,6 +111,9 @@ struct PushArgs {
     // the flush would add to J (zero where it adds none), for
     // launchGatherFlush instead of adding it to J
     float* tileOut;
+    // with tileOut: a word per supercell, set to 1 with its tile and to 0 when
+    // it holds no particle of the launch; its tile is then not written
+    uint32_t* tileHeld;
     PmlDampArgs damp;  // axes == 0: no PML damping
 };
 
@@ -143,10 +146,10 @@ size_t pushTileElems(int supp);
 // checkerboard phases: the float additions, in the same order, of the
 // phase-by-phase flush, so J is the same bit for bit. colour: the
 // checkerboard colour of every supercell index along x, then y, then z
-// (nscx + nscy + nscz entries). fresh: J holds nothing yet; the sums start at
-// zero and every cell is written.
-hipError_t launchGatherFlush(int supp, const GridDev& g, const float* tiles, const uint8_t* colour,
-                             float* const J[3], bool fresh, hipStream_t s);
+// (nscx + nscy + nscz entries). held: PushArgs::tileHeld. fresh: J holds
+// nothing yet; the sums start at zero and every cell is written.
+hipError_t launchGatherFlush(int supp, const GridDev& g, const float* tiles, const uint32_t* held,
+                             const uint8_t* colour, float* const J[3], bool fresh, hipStream_t s);
 // shift of one species: `staged` = the push epilogue already moved the leavers
 // to the outbox and compacted every supercell (then only the insert runs).
 // redo: the insert again after the supercells grew, from count - incoming
@@ -298,6 +301,7 @@ hipError_t launchCurrentResetBatch(const FieldBatchEntry* table, const int2* blo
 struct GatherEntry {
     GridDev g;
     const float* tiles;
+    const uint32_t* held;
     const uint8_t* colour;
     float* J[3];
 };

@@ -125,6 +125,44 @@ def test_deposit_stage_schedules_bit_exact(shape, open_, schedule):
 
 
 @pytest.mark.parametrize("open_", [False, True], ids=["periodic", "open"])
+@pytest.mark.parametrize("shape", [abi.SHAPE_CIC, abi.SHAPE_TSC, abi.SHAPE_PQS], ids=["cic", "tsc", "pqs"])
+def test_one_launch_with_empty_supercells(shape, open_):
+    """Supercells without particles leave no tile to the gather flush: a clump
+    of particles that spreads over empty neighbours in one launch, eager and
+    from the graphs, against the oracle; every supercell that held a tile in
+    one step and is empty in a later one is passed over then (the clump drifts
+    by a supercell)."""
+    st = small_thermal(shape, grid=(24, 16, 16), ppc=2, u=0.1)
+    st.species[0].u_drift = (3.0, 0.0, 2.0)
+    if open_:
+        open_box(st, boundary=(1, 1, 0))
+    print(f"case empty supercells shape={shape} grid={st.grid} open={open_}", flush=True)
+    cells, pos, mom, w = setups.host_particles(st, 0)
+    keep = ((cells >= [8, 0, 4]) & (cells < [16, 8, 8])).all(axis=1)
+    f = setups.bin_frames(st, 0, cells[keep], pos[keep], mom[keep], w[keep])
+    E, B = H.random_fields(st, 5, 1e-3, 1e-3)
+    sim = abi.Simulation(st.config())
+    sim.write_frames(0, f)
+    sim.load_field(abi.FIELD_E, E)
+    sim.load_field(abi.FIELD_B, B)
+    sim.set_push_schedule(abi.PUSH_SCHEDULE_SINGLE)
+    ora = O.Oracle(st, 32, 0, jexp=sim.j_scale_exp())
+    ora.set_frames(0, f)
+    ora.set_field(abi.FIELD_E, E)
+    ora.set_field(abi.FIELD_B, B)
+    start = f["counts"].copy()
+    for n, step in ((1, sim.step), (7, sim.step), (8, sim.step_graph)):
+        step(n)
+        ora.step(n)
+        H.assert_frames_equal(sim.read_frames(0), ora.get_frames(0), f"after {n} more steps")
+        for fld in (abi.FIELD_E, abi.FIELD_B, abi.FIELD_J):
+            H.assert_field_equal(sim.read_field(fld), ora.get_field(fld), f"field {fld}")
+    end = sim.read_frames(0)["counts"]
+    assert ((start > 0) & (end == 0)).any() and (start == 0).any()
+    sim.close()
+
+
+@pytest.mark.parametrize("open_", [False, True], ids=["periodic", "open"])
 def test_shift_bit_exact(open_):
     st = small_thermal(abi.SHAPE_CIC, abi.PUSHER_BORIS, u=0.3)
     if open_:

@@ -61,6 +61,7 @@ __device__ __forceinline__ void boxCoords(int t, int& x, int& y, int& z) {
 // push formed: the unfused deposit does the same. Keeping the state in the
 // queue instead took 16 registers of every wave for the whole loop, and with
 // them the kernel spilled.
+static_assert(kMaxFrames * SCV <= 1 << 16, "a slot takes 16 bits");
 __device__ __forceinline__ uint32_t slowItem(int slot, int cx, int cy, int cz, int species) {
     return (uint32_t)slot | ((uint32_t)cx << 16) | ((uint32_t)cy << 20) | ((uint32_t)cz << 24) |
            ((uint32_t)species << 28);

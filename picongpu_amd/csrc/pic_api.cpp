@@ -69,7 +69,7 @@ int validateConfig(const pic_config& c) {
         if (d.pusher < PIC_PUSHER_NONE || d.pusher > PIC_PUSHER_HIGUERA_CARY) return fail(PIC_E_INVALID, "unknown pusher");
         if (d.current_solver != PIC_CURRENT_SOLVER_ESIRKEPOV && d.current_solver != PIC_CURRENT_SOLVER_EMZ)
             return fail(PIC_E_INVALID, "unknown current solver");
-        if (d.frames_per_sc <= 0 || d.frames_per_sc > 255)
+        if (d.frames_per_sc <= 0 || d.frames_per_sc > pic::kMaxFrames)
             return fail(PIC_E_INVALID, "frames_per_sc must be in [1,255]");
         if (!(d.mass_ratio > 0.0)) return fail(PIC_E_INVALID, "mass_ratio must be positive");
         for (int a = 0; a < 3; ++a) {
@@ -1352,10 +1352,6 @@ bool grownCaps(const SpeciesMem& m, const std::vector<uint32_t>& need, int maxFr
     return any;
 }
 
-// the most frames a supercell of a species may have (the configuration's
-// bound); the current tile's fixed-point range assumes it
-constexpr int kMaxFrames = 255;
-
 // grows the supercells of species s that must hold more than their slots
 // (`need` per supercell), at most to maxFrames frames
 int growFor(pic_ctx* c, int s, const std::vector<uint32_t>& need, int maxFrames) {
@@ -1370,12 +1366,10 @@ int growFor(pic_ctx* c, int s, const std::vector<uint32_t>& need, int maxFrames)
 }
 
 // frames for a supercell that must hold `count` particles: geometric growth
-// (half again) with at least two spare frames, at most maxFrames (0: no limit)
+// (half again) with at least two spare frames, at most maxFrames
 int grownFrames(int frames, uint32_t count, int maxFrames) {
     int const need = static_cast<int>((count + pic::kSCV - 1) / pic::kSCV);
-    int f = std::max(need + 2, frames + (frames + 1) / 2);
-    if (maxFrames > 0) f = std::min(f, maxFrames);
-    return f;
+    return std::min(std::max(need + 2, frames + (frames + 1) / 2), maxFrames);
 }
 
 // After steps: when a shift found a supercell full, the insert kept the true
@@ -1386,7 +1380,7 @@ int grownFrames(int frames, uint32_t count, int maxFrames) {
 // bit for bit), clear the flags and return the number of skipped steps in
 // *skipped. Each skipped fused field step swapped E and Ealt on the host
 // without writing, so an odd count is swapped back. maxFrames bounds the
-// growth (0: none); beyond it the counts are clamped, particles are lost and
+// growth; beyond it the counts are clamped, particles are lost and
 // the context refuses further steps.
 int recoverCapacity(pic_ctx* c, int* skipped, int maxFrames) {
     *skipped = 0;
@@ -1723,7 +1717,7 @@ int pic_load_particles(pic_ctx* c, int32_t s, int64_t n, const int32_t* cell, co
     }
     // supercells that receive more particles than they hold grow first
     {
-        if ((r = growFor(c, s, counts, kMaxFrames)) != PIC_OK) return r;
+        if ((r = growFor(c, s, counts, pic::kMaxFrames)) != PIC_OK) return r;
     }
     size_t const slots = m.slots;
     std::vector<float> hp[3], hm[3];
@@ -1862,7 +1856,7 @@ int pic_write_frames(pic_ctx* c, int32_t s, const uint32_t* counts, const float*
     // supercells whose new count exceeds their slots grow first
     if (counts) {
         std::vector<uint32_t> need(counts, counts + c->nsc);
-        if ((r = growFor(c, s, need, kMaxFrames)) != PIC_OK) return r;
+        if ((r = growFor(c, s, need, pic::kMaxFrames)) != PIC_OK) return r;
     }
     pic::SpeciesDev& d = m.dev;
     m.shiftReady = 0;
@@ -1957,7 +1951,7 @@ int pic_init_species(pic_ctx* c, int32_t s, const pic_init_desc* desc) {
     SpeciesMem& m = c->sp[s];
     {  // every supercell must hold ppc particles in each of its cells
         std::vector<uint32_t> need(c->nsc, static_cast<uint32_t>(desc->ppc) * pic::kSCV);
-        if ((r = growFor(c, s, need, kMaxFrames)) != PIC_OK) return r;
+        if ((r = growFor(c, s, need, pic::kMaxFrames)) != PIC_OK) return r;
     }
     double const vol = c->cfg.cell_si[0] * c->cfg.cell_si[1] * c->cfg.cell_si[2];
     pic::InitArgs a{};
@@ -2150,7 +2144,7 @@ int pic_shift(pic_ctx* c, int32_t species) {
     if (r != PIC_OK) return r;
     // a supercell that overflowed grows now, so the next stage sees every particle
     int skipped = 0;
-    return recoverCapacity(c, &skipped, kMaxFrames);
+    return recoverCapacity(c, &skipped, pic::kMaxFrames);
 }
 
 int pic_fdtd_before_current(pic_ctx* c) {
@@ -2364,7 +2358,7 @@ int pic_step(pic_ctx* c, int32_t nsteps) {
             int const r = oneStep(c);
             if (r != PIC_OK) return r;
         }
-        int const r = recoverCapacity(c, &todo, kMaxFrames);
+        int const r = recoverCapacity(c, &todo, pic::kMaxFrames);
         if (r != PIC_OK) return r;
     } while (todo > 0);
     return PIC_OK;
@@ -2380,7 +2374,7 @@ int pic_step_graph(pic_ctx* c, int32_t nsteps) {
         int const r = stepGraphs(c, todo);
         if (r != PIC_OK) return r;
         // a repacking growth drops the graphs: recaptured on the next replay
-        int const rr = recoverCapacity(c, &todo, kMaxFrames);
+        int const rr = recoverCapacity(c, &todo, pic::kMaxFrames);
         if (rr != PIC_OK) return rr;
     } while (todo > 0);
     return PIC_OK;

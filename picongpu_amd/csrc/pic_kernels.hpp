@@ -10,6 +10,9 @@
 namespace pic {
 
 constexpr int kSCX = 8, kSCY = 8, kSCZ = 4, kSCV = 256;
+// the most frames a supercell of a species may have; the fixed-point range of
+// the current tile and the push's 16-bit slots assume it
+constexpr int kMaxFrames = 255;
 constexpr int kNumDirs = 27;      // exchange codes 0..26 (0 = stays)
 constexpr int kOffStride = 28;    // per-supercell offset table entries
 

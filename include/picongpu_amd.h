@@ -486,10 +486,12 @@ int pic_adjoint_backward(pic_ctx* ctx, const double* dE, const double* dB, doubl
 
 /* --- batched ensembles -------------------------------------------------- */
 /* Many independent periodic simulations (each a pic_ctx, grids and particle
- * counts may differ) advanced together: one launch per checkerboard phase of
- * the fused push/deposit over every member's supercells, one launch each for
- * the shift's insert and compact passes, the fused field step and the current
- * reset, optionally replayed from a captured hipGraph. The reference runs one
+ * counts may differ) advanced together: the fused push/deposit over every
+ * member's supercells in one launch and their current tiles gathered in
+ * another (where every member's push schedule is SINGLE), or the current's
+ * reset and one launch per checkerboard phase; one launch for the shift's
+ * insert, and those of the fused field step; optionally replayed from a
+ * captured hipGraph. The reference runs one
  * simulation per process; there is no counterpart interface. Members are
  * created from the configurations and are then initialised, loaded, read and
  * diagnosed through the single-simulation calls on pic_ensemble_member();

@@ -2870,7 +2870,10 @@ int pic_adjoint_backward(pic_ctx* c, const double* dE, const double* dB, double*
 // ---------------------------------------------------------------------------
 // batched ensembles of independent simulations
 // ---------------------------------------------------------------------------
-// frames per supercell an ensemble's members are bound to
+// Frames per supercell an ensemble's members are bound to: the interface's
+// bound. The batched push itself takes supercells of any size (kMaxFrames),
+// but a workgroup does a supercell's whole work, so a launch over all members
+// would last as long as the largest supercell of any of them.
 constexpr int kEnsembleMaxFrames = 64;
 
 struct pic_ensemble {
@@ -3086,7 +3089,7 @@ int ensOneStep(pic_ensemble* e) {
 }
 
 // After batched steps: a member whose shift overflowed skipped the steps
-// after it; it grows (within the frames the batched push can list), and runs
+// after it; it grows (within the members' bound of frames), and runs
 // them on its own (its own steps equal its batched ones bit for bit). The
 // members' buffers may have moved, so the device tables are written again
 // (the captured ensemble graphs read them, so they stay valid).

@@ -421,6 +421,14 @@ int pic_gauss_residual(pic_ctx* ctx, double* out);
  * array: calls that overlap on one device race. Same output as
  * pic_gauss_residual (FP64 atomics: equal up to FP64 round-off). */
 int pic_gauss_residual_noalloc(pic_ctx* ctx, double* out);
+/* Check of the device's arithmetic (no counterpart in the reference): the push
+ * and field kernels take 1/x and sqrt(x) from the hardware's approximations
+ * with a correction, and quotients by the cell size as FP64 products. Every
+ * mantissa of their domains is compared with the correctly rounded value, the
+ * quotients for the n given divisors (positive, finite); mismatches[0..3]
+ * receive the differing inputs of 1/x for roots, 1/x and sqrt(x) for x >= 1,
+ * and x/divisor. All four are 0 on a gfx950 device. */
+int pic_arithmetic_mismatches(int32_t device, const float* divisors, int32_t n, uint64_t* mismatches);
 /* PIC_FLAG_* bits raised since the last call */
 #define PIC_FLAG_CAPACITY_GREW 1u /* a supercell overflowed and the species' supercells grew (nothing lost) */
 int pic_error_flags(pic_ctx* ctx, uint32_t* flags);

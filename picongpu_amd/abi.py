@@ -256,6 +256,7 @@ SIGNATURES = {
     "pic_field_energy": (C.c_int, [_P, _D]),
     "pic_gauss_residual": (C.c_int, [_P, _D]),
     "pic_gauss_residual_noalloc": (C.c_int, [_P, _D]),
+    "pic_arithmetic_mismatches": (C.c_int, [C.c_int32, _F, C.c_int32, C.POINTER(C.c_uint64)]),
     "pic_error_flags": (C.c_int, [_P, _U32]),
     "pic_timing_enable": (C.c_int, [_P, C.c_int32]),
     "pic_kernel_timer": (C.c_int, [_P, C.c_int32, _D, C.POINTER(C.c_int64)]),
@@ -366,6 +367,15 @@ def make_config(grid, cell_si, dt_si, density_si, ppc, species, solver=SOLVER_YE
         fill_incident_profile(cfg.incident[axis][side], **prof)
     fill_pml(cfg.pml, pml)
     return cfg
+
+
+def arithmetic_mismatches(divisors, device: int = 0) -> list[int]:
+    """pic_arithmetic_mismatches: inputs for which the kernels' shortened 1/x of
+    a root, 1/x and sqrt(x) of x >= 1 and x/divisor are not correctly rounded."""
+    d = np.ascontiguousarray(divisors, np.float32)
+    out = (C.c_uint64 * 4)()
+    check(load_library().pic_arithmetic_mismatches(device, ptr(d, C.c_float), d.size, out), "pic_arithmetic_mismatches")
+    return list(out)
 
 
 def constants_from_config(cfg: Config) -> Constants:

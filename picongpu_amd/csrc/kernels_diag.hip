@@ -142,4 +142,56 @@ hipError_t launchGaussResidual(const FieldArgs& f, const SpeciesDev* sp, const i
     return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------
+// The shortened FP32 operations against their IEEE values, mantissa by
+// mantissa. The references are FP64 operations rounded to FP32: 53 bits are
+// more than twice 24 and two, so the second rounding changes nothing.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void countDifferent(float a, float b, unsigned long long* bad) {
+    bool const same = __float_as_uint(a) == __float_as_uint(b) || (a != a && b != b);
+    unsigned long long const m = __ballot(!same);
+    if (m != 0ull && (threadIdx.x & 63) == 0) atomicAdd(bad, (unsigned long long)__popcll(m));
+}
+
+// every float of [2^e, 2^(e+1))
+__global__ __launch_bounds__(256) void kCheckReciprocals(int e, unsigned long long* bad) {
+    uint32_t const i = blockIdx.x * 256u + threadIdx.x;  // 2^23 threads
+    float const x = __uint_as_float(((uint32_t)(127 + e) << 23) | i);
+    float const inverse = (float)(1.0 / (double)x);
+    if (e <= 64) countDifferent(recipOfRoot(x), inverse, bad);  // a root lies below 2^64
+    if (e < 0) return;
+    countDifferent(recipAbove1(x), inverse, bad + 1);
+    countDifferent(sqrtAbove1(x), (float)sqrt((double)x), bad + 2);
+}
+
+// every mantissa and sign divided by c, the exponents spread over 2^-60 .. 2^59
+__global__ __launch_bounds__(256) void kCheckDivExact(float c, unsigned long long* bad) {
+    uint32_t const i = blockIdx.x * 256u + threadIdx.x;  // 2^24 threads
+    uint32_t h = i * 2654435761u;
+    h ^= h >> 15;
+    h *= 2246822519u;
+    h ^= h >> 13;
+    float const x = __uint_as_float(((127u - 60u + h % 120u) << 23) | (i & 0x7fffffu) | (i >> 23 << 31));
+    countDifferent(divExact(x, 1.0 / (double)c), (float)((double)x / (double)c), bad);
+}
+
+// zeros, infinities, NaN and the ends of the domains
+__global__ __launch_bounds__(64) void kCheckSpecial(unsigned long long* bad) {
+    float const inf = __uint_as_float(0x7f800000u), nan = __uint_as_float(0x7fc00000u);
+    float const root[4] = {0.0f, inf, nan, 1.0f}, above1[4] = {inf, nan, 1.0f, 3.4028235e38f};
+    float const r = root[threadIdx.x & 3], x = above1[threadIdx.x & 3];
+    countDifferent(recipOfRoot(r), (float)(1.0 / (double)r), bad);
+    countDifferent(recipAbove1(x), (float)(1.0 / (double)x), bad + 1);
+    countDifferent(sqrtAbove1(x), (float)sqrt((double)x), bad + 2);
+    float const q[4] = {0.0f, -0.0f, -inf, nan};
+    countDifferent(divExact(q[threadIdx.x & 3], 1.0 / 1.7416), q[threadIdx.x & 3], bad + 3);
+}
+
+hipError_t launchArithmeticCheck(const float* divisors, int n, unsigned long long* bad, hipStream_t s) {
+    for (int e = -75; e <= 127; ++e) hipLaunchKernelGGL(kCheckReciprocals, dim3(1u << 15), dim3(256), 0, s, e, bad);
+    for (int k = 0; k < n; ++k) hipLaunchKernelGGL(kCheckDivExact, dim3(1u << 16), dim3(256), 0, s, divisors[k], bad + 3);
+    hipLaunchKernelGGL(kCheckSpecial, dim3(1), dim3(64), 0, s, bad);
+    return hipGetLastError();
+}
+
 }  // namespace pic

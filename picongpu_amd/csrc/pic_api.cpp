@@ -2437,6 +2437,24 @@ int pic_gauss_residual_noalloc(pic_ctx* c, double* out) {
     return PIC_OK;
 }
 
+int pic_arithmetic_mismatches(int32_t device, const float* divisors, int32_t n, uint64_t* mismatches) {
+    if (n < 0 || (n > 0 && !divisors) || !mismatches) return fail(PIC_E_INVALID, "null argument");
+    for (int32_t i = 0; i < n; ++i)
+        if (!(divisors[i] > 0.0f) || !std::isfinite(divisors[i]))
+            return fail(PIC_E_INVALID, "divisors must be positive and finite");
+    PIC_HIP(hipSetDevice(device));
+    unsigned long long* bad = nullptr;
+    PIC_HIP(hipMalloc(&bad, 4 * sizeof(*bad)));
+    unsigned long long out[4] = {0, 0, 0, 0};
+    hipError_t e = hipMemcpy(bad, out, sizeof(out), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = pic::launchArithmeticCheck(divisors, n, bad, nullptr);
+    if (e == hipSuccess) e = hipMemcpy(out, bad, sizeof(out), hipMemcpyDeviceToHost);
+    (void)hipFree(bad);
+    PIC_HIP(e);
+    for (int k = 0; k < 4; ++k) mismatches[k] = out[k];
+    return PIC_OK;
+}
+
 int pic_error_flags(pic_ctx* c, uint32_t* flags) {
     if (!c || !flags) return fail(PIC_E_INVALID, "null argument");
     PIC_HIP(hipStreamSynchronize(c->stream));

@@ -50,10 +50,13 @@ __device__ __forceinline__ float esirkepovWeight(float s0i, float dsi, float s0j
 }
 
 // RN(1 / s) for the root s of a float: the hardware reciprocal (within an ulp)
-// and one Newton step in multiply-adds. The residual 1 - s r is exact; the
-// step's rounding is the correct one for every float of [1, 4), which with
-// the exact scaling by powers of 2 is every s whose reciprocal is normal
-// (a root lies in [2^-75, 2^64]); div_fixup gives 1/0, 1/inf and 1/NaN. Four
+// and one Newton step in multiply-adds, whose residual 1 - s r is exact. An
+// ulp alone is not enough: for the mantissa of all ones the quotient lies just
+// above the middle of two floats, and the step rounds to the even one, the
+// wrong one, if the reciprocal was rounded down. That the hardware's values
+// give the correct rounding for every mantissa is what
+// pic_arithmetic_mismatches counts (0 of every float of [2^-75, 2^65); a root
+// lies in [2^-75, 2^64]); div_fixup gives 1/0, 1/inf and 1/NaN. Four
 // instructions instead of the eleven of the full division, whose scaling of
 // denormal operands a root never needs.
 __device__ __forceinline__ float recipOfRoot(float s) {
@@ -62,7 +65,8 @@ __device__ __forceinline__ float recipOfRoot(float s) {
     return __builtin_amdgcn_div_fixupf(r, s, 1.0f);
 }
 
-// the same for x >= 1 (or NaN); the full division above 2^126
+// the same for x >= 1 (or NaN); the full division above 2^126, where the
+// quotient is subnormal
 __device__ __forceinline__ float recipAbove1(float x) {
     float r = __builtin_amdgcn_rcpf(x);
     r = __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
@@ -71,8 +75,8 @@ __device__ __forceinline__ float recipAbove1(float x) {
 }
 
 // RN(sqrt(x)) for x >= 1 (or NaN): the hardware root (within an ulp) and its
-// two neighbours tested by the signs of exact residuals. The general sqrtf
-// scales arguments below 2^-96 besides.
+// two neighbours tested by the signs of exact residuals (Tuckerman's test).
+// The general sqrtf scales arguments below 2^-96 besides.
 __device__ __forceinline__ float sqrtAbove1(float x) {
     float const s = __builtin_amdgcn_sqrtf(x);
     float const down = __int_as_float(__float_as_int(s) - 1);

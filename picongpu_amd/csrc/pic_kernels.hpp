@@ -20,7 +20,9 @@ constexpr int kOffStride = 28;    // per-supercell offset table entries
 // relatively, and no quotient of two floats lies closer than 2^-49 to the
 // midpoint of two neighbouring normal floats (|x - m c| is at least one unit
 // of a 49-bit product, and never 0 for a 25-bit m), so rounding the product
-// rounds the quotient. Three instructions instead of eleven.
+// rounds the quotient; of a subnormal quotient, which can lie on a midpoint,
+// it may round the last bit (2^-149) the other way. Three instructions instead
+// of eleven.
 __device__ __forceinline__ float divExact(float x, double rc) { return (float)((double)x * rc); }
 
 struct SpeciesDev {
@@ -232,6 +234,9 @@ int fieldStepTiles(int solver, const GridDev& g);
 // nblocks partial sums (6 * nblocks doubles of scratch), then out[0..5]
 hipError_t launchEnergy(const FieldArgs& a, double* partials, int nblocks, double* out, hipStream_t s);
 hipError_t launchCountSum(const uint32_t* counts, int n, unsigned long long* out, hipStream_t s);
+// bad[4] += the inputs for which recipOfRoot, recipAbove1, sqrtAbove1 and
+// divExact (by each divisor) differ from the correctly rounded value
+hipError_t launchArithmeticCheck(const float* divisors, int n, unsigned long long* bad, hipStream_t s);
 hipError_t launchGaussResidual(const FieldArgs& f, const SpeciesDev* sp, const int* supp, int nsp, double qScale,
                                double eps0, double* buf, hipStream_t s);
 // The allocation-free Gauss residual's scratch: a file-scope device array of

@@ -22,7 +22,7 @@
 
 namespace pic {
 
-// v in [-n, 2n) wrapped into [0, n)
+// v in [-n, 2n) wrapped into [0, n); n >= 4
 __device__ __forceinline__ int wrapI(int v, int n) {
     v = v < 0 ? v + n : v;
     return v >= n ? v - n : v;
@@ -31,6 +31,14 @@ __device__ __forceinline__ int wrapI(int v, int n) {
 __device__ __forceinline__ size_t gidx(const GridDev& g, int x, int y, int z) {
     return (size_t)wrapI(x, g.nx) + (size_t)g.nx * ((size_t)wrapI(y, g.ny) + (size_t)g.ny * (size_t)wrapI(z, g.nz));
 }
+
+// The first cell of a move's stencil, relative to the particle's cell: the
+// lower of its start and end, -1 .. 1 for a particle's position (in [0, 1] at
+// the end, less than a cell away at the start). A position made from
+// non-finite data may give any integer (the conversion of the floor turns NaN
+// into 0 and saturates): the bounds keep the nodes it addresses within wrapI's
+// range, and the sums with a cell from overflowing.
+__device__ __forceinline__ int stencilCell(int start, int end) { return max(-2, min(2, min(start, end))); }
 
 // Signed periodic difference in [-n/2, n/2) of two cells of [0, n).
 __device__ __forceinline__ int wrapDiff(int d, int n) {
@@ -300,7 +308,7 @@ __device__ __forceinline__ void depositCIC(const DiffArgs& a, unsigned long long
         p1[d] = np[d];
         int const iS = (int)floorf(p0[d]);
         int const iE = (int)floorf(p1[d]);
-        gs[d] = iS < iE ? iS : iE;
+        gs[d] = stencilCell(iS, iE);
         st[d] = (gs[d] == iS ? 2 : 0) | (gs[d] == iE ? 4 : 0) | (iS != iE ? 1 : 0);
         p0[d] -= (float)gs[d];
         p1[d] -= (float)gs[d];
@@ -708,7 +716,7 @@ __device__ __forceinline__ void adjointParticle(const AdjPartArgs& a, const AdjS
             R const step = divExact(v[d], a.rcell[d]);  // v dt / cell
             X1[d] = r[d] + step;
             X0[d] = X1[d] - step;
-            int const gs = (int)fmin(floor(X0[d]), floor(X1[d]));
+            int const gs = stencilCell((int)floor(X0[d]), (int)floor(X1[d]));
             X0[d] -= (R)gs;
             X1[d] -= (R)gs;
             gs3[d] = gs;

@@ -137,6 +137,39 @@ def test_hot_particles_match_fp64_tape(ppc):
     pic.close()
 
 
+@pytest.mark.parametrize("ppc", [2, 9])
+def test_non_finite_particles_stay_in_the_box(ppc):
+    """Particles with infinite and NaN momenta (their positions become NaN) in
+    sparse and dense tiles: the forward and backward passes address nodes of
+    the grid only, every particle keeps a cell of it, and in the first step,
+    before the fields carry the NaN on, the other particles move as without
+    them."""
+    grid = (16, 16, 8)
+    print(f"case adjoint non-finite particles grid={grid} ppc={ppc}", flush=True)
+    st = setups.differentiable(grid=grid, ppc=ppc, steps=6)
+    cell, pos, mom, w = adjoint.cold_plasma(st)
+    rng = np.random.default_rng(ppc)
+    bad = rng.choice(cell.shape[1], 40, replace=False)
+    sick = mom.copy()
+    sick[:, bad] = rng.choice(np.array([np.inf, -np.inf, np.nan], np.float32), (3, 40))
+    E0, B0 = adjoint.gaussian_pulse(st, torch.tensor([1.0, 0.5, 0.05], dtype=F64).cuda(), amp=pulse_amp(st))
+    moved = []
+    for p in (mom, sick):
+        pic = adjoint.DifferentiablePIC(st, cell, pos, p, w, 1, 4)
+        pic.forward_raw(E0, B0)
+        moved.append(pic.sim.adjoint_read_particles())
+        pic.close()
+    good = np.setdiff1d(np.arange(cell.shape[1]), bad)
+    for a, b in zip(*moved):
+        np.testing.assert_array_equal(np.asarray(a)[:, good], np.asarray(b)[:, good])
+    pic = adjoint.DifferentiablePIC(st, cell, pos, sick, w, 6, 4)
+    E, B = pic.forward_raw(E0, B0)
+    pic.backward_raw(torch.ones_like(E, dtype=F64), torch.ones_like(B, dtype=F64), particles=True)
+    cells = np.asarray(pic.sim.adjoint_read_particles()[0])
+    assert (cells >= 0).all() and (cells < np.array(grid)[:, None]).all()
+    pic.close()
+
+
 def test_parameter_gradient_matches_central_differences():
     """dF/dtheta through the torch.autograd.Function (pulse built in torch on
     the device, HIP forward and adjoint) against FP64 central differences of

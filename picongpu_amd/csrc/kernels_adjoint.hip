@@ -20,6 +20,8 @@
 
 #include <rocprim/device/device_radix_sort.hpp>
 
+#include <type_traits>
+
 namespace pic {
 
 // v in [-n, 2n) wrapped into [0, n); n >= 4
@@ -663,6 +665,7 @@ struct BorisFwd {
 // Boris push in the adjoint's precision (particlePusherBoris.hpp:41-90); dt = c = 1
 template <typename R>
 __device__ __forceinline__ BorisFwd<R> borisFwd(V3<R> p0, V3<R> E, V3<R> B, R m, R q) {
+    static_assert(std::is_same<R, float>::value, "sqrtAbove1 and recipAbove1 are FP32 operations");
     BorisFwd<R> b;
     b.hq = R(0.5) * q;
     b.pm = axpy(b.hq, E, p0);
@@ -680,6 +683,7 @@ template <bool LDS, typename R>
 __device__ __forceinline__ void adjointParticle(const AdjPartArgs& a, const AdjState& S, int64_t idx, const int* c,
                                                 const BlockWindow& win, const int* rel, const float* sF,
                                                 const R* sLJ, double* sL) {
+    static_assert(std::is_same<R, float>::value, "divExact is an FP32 operation");
     int64_t const n = S.n;
     R const r[3] = {(R)S.pos[idx], (R)S.pos[n + idx], (R)S.pos[2 * n + idx]};
     V3<R> const p0{(R)S.mom[idx], (R)S.mom[n + idx], (R)S.mom[2 * n + idx]};
@@ -757,7 +761,7 @@ __device__ __forceinline__ void adjointParticle(const AdjPartArgs& a, const AdjS
     }
 
     phaseBarrier();
-    // ---- reverse velocity: v = p1 / sqrt(m^2 + |p1|^2 rc2) ----
+    // ---- reverse velocity: v = p1 / sqrt(m^2 + |p1|^2) ----
     V3<R> const LV{lv[0], lv[1], lv[2]};
     R const kv = dotD(p1, LV) / (G * G * G);
     V3<R> const l1{(R)S.lP[idx] + LV.x / G - p1.x * kv, (R)S.lP[n + idx] + LV.y / G - p1.y * kv,
@@ -971,12 +975,23 @@ static inline unsigned blocksOf(size_t n) { return (unsigned)((n + 255) / 256); 
 // per tile and one more tile along x, (8 (t + 1) + 3) x 7 x 5 cells with the
 // nodes around them, and more as the particles drift (up to two cells before
 // the next sort). 512 threads share a window where a tile fills them: more
-// waves per CU for the same LDS. The windows are the largest that leave two
-// blocks of 512 per CU (48 B a cell in the forward kernel, 84 B in the
-// adjoint one). 64^3 cells, 8 particles per cell, us a launch, forward and
-// adjoint kernel: 229 and 412 with the fields gathered from memory by wrapped
-// indices and 256 threads; 88 and 287 now (129 and 447 with 768 cells, where
-// more particles lie outside the window).
+// waves per CU for the same LDS. The windows were chosen by measurement among
+// those that leave two blocks of 512 per CU (48 B a cell in the forward
+// kernel, 84 B in the adjoint one, at most about 1,680 and 960 cells). 64^3
+// cells, 8 particles per cell, us a launch, forward and adjoint kernel: 229
+// and 412 with the fields gathered from memory by wrapped indices and 256
+// threads; 88 and 287 now (129 and 447 with 768 cells, where more particles
+// lie outside the window).
+// Both forms by density, 64^3 cells, 16 steps forward + backward, ms with 256
+// and with 512 threads; cold, and hot (half a cell a step, where more
+// particles lie outside the windows):
+//   particles per cell   2            4            6            7            8             12            16
+//   cold                 4.2   6.0    5.7   5.1    7.4   6.2    8.3   6.9    8.9   7.4    12.5  10.2   16.2  12.8
+//   hot                 11.2  14.9   14.0  15.4   16.6  18.1   18.4  20.4   18.8  19.7    23.5  24.9   30.2  28.9
+// The line lies where a tile nearly fills the 512 threads: from there on cold
+// particles gain a sixth to a fifth and hot ones lose a tenth at most, below
+// it the gain shrinks and turns into a loss. (Fields from memory, 256 threads:
+// 2 particles per cell 5.7 cold and 17.7 hot, 8: 13.9 and 26.8, 16: 25.5 and 40.5.)
 constexpr int kAdjDenseTile = 448;
 static bool denseTiles(int64_t particles, const GridDev& g) {
     double const tiles = (double)(g.nx / kTileX) * (g.ny / kTileY) * (g.nz / kTileZ);

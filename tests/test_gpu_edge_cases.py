@@ -1,9 +1,10 @@
 """Edge cases of the frame layout, the push and the shift, bit-exact against
 the oracle: empty and ragged supercells (counts at and around frame
-boundaries), a supercell larger than the push kernel's leaver lists reach
-(the shift then collects its leavers itself), positions on cell borders,
-ultra-relativistic momenta for every pusher, and supercells that overflow
-their frames in the shift: they grow, and no particle is lost."""
+boundaries), supercells with more leavers than the push keeps in LDS or more
+particles than its leaver bits reach, positions on cell borders, non-finite
+field nodes beside the stencils, ultra-relativistic momenta for every pusher,
+and supercells that overflow their frames in the shift: they grow, and no
+particle is lost."""
 import copy
 
 import numpy as np
@@ -86,8 +87,8 @@ def test_empty_and_ragged_supercells(shape):
 
 
 def test_supercell_beyond_the_leaver_lists():
-    """17000 particles in one supercell (more than 512 threads x 32 iterations
-    of the push's leaver lists): the shift collects that species itself."""
+    """17000 particles in one supercell, more than 512 threads x 32 leaver
+    bits: the push lists its leavers from their multiMask, in global memory."""
     st = thermal(frames=70)  # 17920 slots
     counts = [17000, 300, 0, 17, 256, 1, 2, 3, 511, 0, 64, 5]
     print(f"case large supercell counts={counts}", flush=True)

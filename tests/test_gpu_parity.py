@@ -87,11 +87,13 @@ def test_push_fused_bit_exact(name, make):
 DEPOSIT_CASES = CASES[:3] + CASES[-3:]
 
 
+@pytest.mark.parametrize("schedule", [abi.PUSH_SCHEDULE_PHASES, abi.PUSH_SCHEDULE_SINGLE], ids=["phases", "single"])
 @pytest.mark.parametrize("name,make", DEPOSIT_CASES, ids=[c[0] for c in DEPOSIT_CASES])
-def test_deposit_unfused_bit_exact(name, make):
+def test_deposit_unfused_bit_exact(name, make, schedule):
     st = make()
-    print(f"case deposit {name} grid={st.grid}", flush=True)
+    print(f"case deposit {name} grid={st.grid} schedule={schedule}", flush=True)
     sim, ora, _ = H.make_pair(st)
+    sim.set_push_schedule(schedule)
     sim.current_reset()
     sim.deposit(-1)
     ora.current_reset()

@@ -666,8 +666,9 @@ struct YeeAfterLds {
 };
 
 // update_afterCurrent for one z-marching tile (Yee): B'' = (B - curlE(E)*0.5*dt) - curlE(Enew)*0.5*dt;
-// with TWO = false one B half step alone, B' = B - curlE(E)*0.5*dt (kBHalf's arithmetic)
-template <bool OPEN, bool TWO, bool PML = false>
+// with TWO = false one B half step alone, B' = B - curlE(E)*0.5*dt (kBHalf's arithmetic).
+// DIV = true takes the quotients by full divisions, the same values (divideInAfter).
+template <bool OPEN, bool TWO, bool PML = false, bool DIV = false>
 __device__ __forceinline__ void yeeAfterTile(const FieldArgs& a, float* const* Enew, int b, int zc, YeeAfterLds& L,
                                              const PmlArgs* p = nullptr, int updatePsi = 0) {
     ZTile const T = zTile(a.g, b, zc);
@@ -684,6 +685,7 @@ __device__ __forceinline__ void yeeAfterTile(const FieldArgs& a, float* const* E
     }
     float* const Eb = &L.E[0][0][0][0];
     float* const Nb = &L.En[0][0][0][0];
+    auto quot = [&](float x, int d) { return DIV ? x / a.cell[d] : divExact(x, a.rcell[d]); };
     // this thread's elements of planes k of E and Enew on x, y in [0, T+1)
     auto fetch = [&](int k, float (&ve)[NE], float (&vn)[NE]) {
         size_t const zoff = plane * (size_t)wrap1(k, nz);
@@ -745,9 +747,9 @@ __device__ __forceinline__ void yeeAfterTile(const FieldArgs& a, float* const* E
                             float& cz) {
                 // F: plane k, G: plane k+1 (forward differences, curl as kBHalf)
                 float const f0 = F[0][ly][lx], f1 = F[1][ly][lx], f2 = F[2][ly][lx];
-                cx = divExact(F[2][ly + 1][lx] - f2, a.rcell[1]) - divExact(G[1][ly][lx] - f1, a.rcell[2]);
-                cy = divExact(G[0][ly][lx] - f0, a.rcell[2]) - divExact(F[2][ly][lx + 1] - f2, a.rcell[0]);
-                cz = divExact(F[1][ly][lx + 1] - f1, a.rcell[0]) - divExact(F[0][ly + 1][lx] - f0, a.rcell[1]);
+                cx = quot(F[2][ly + 1][lx] - f2, 1) - quot(G[1][ly][lx] - f1, 2);
+                cy = quot(G[0][ly][lx] - f0, 2) - quot(F[2][ly][lx + 1] - f2, 0);
+                cz = quot(F[1][ly][lx + 1] - f1, 0) - quot(F[0][ly + 1][lx] - f0, 1);
             };
             size_t const i = ixy + plane * k;
             float cx, cy, cz;
@@ -970,12 +972,12 @@ __global__ __launch_bounds__(256) void kYeeBeforeAdd(FieldArgs a, float* Enew0, 
     yeeBeforeAddTile<OPEN>(a, En, blockIdx.x, zc, L);
 }
 
-template <bool OPEN>
+template <bool OPEN, bool DIV>
 __global__ __launch_bounds__(256) void kYeeAfter(FieldArgs a, float* Enew0, float* Enew1, float* Enew2, int zc) {
     if (halted(a.g)) return;
     __shared__ YeeAfterLds L;
     float* const En[3] = {Enew0, Enew1, Enew2};
-    yeeAfterTile<OPEN, true>(a, En, blockIdx.x, zc, L);
+    yeeAfterTile<OPEN, true, false, DIV>(a, En, blockIdx.x, zc, L);
 }
 
 // one B half step (the stage call kBHalf) in the z-marching form
@@ -1384,6 +1386,16 @@ int yeeChunk(const GridDev& g) {
     return zTileCount(g, zc) >= kZFill / 2 ? zc : 0;
 }
 
+// Full divisions in kYeeAfter where the E, Enew and B it streams (36 B a cell)
+// exceed the 256 MB of the Infinity Cache: the launch then waits for HBM and
+// shorter quotients gain little, and on some grids the two curls' FP64
+// products cost more than they save. A field step in ms with products and
+// with divisions: 192^3 cells 0.197 and 0.198, 192x192x160 0.170 and 0.174,
+// 96^3 0.039 and 0.041; beyond the line 256x256x128 0.230 and 0.210, 256^3
+// 0.417 and 0.404, 288^3 0.586 and 0.568, 200x200x192 0.294 and 0.296,
+// 320x256x128 0.308 and 0.314, 512x256x256 0.784 and 0.784.
+static bool divideInAfter(const GridDev& g) { return (size_t)g.nx * g.ny * g.nz * 36 > ((size_t)256 << 20); }
+
 template <bool OPEN>
 static hipError_t fieldStepT(int solver, const FieldArgs& a, float* const Enew[3], const AbsorbPlan* ab, hipStream_t s) {
     // update_afterCurrent damps E before its B half step and B after it
@@ -1427,8 +1439,10 @@ static hipError_t fieldStepT(int solver, const FieldArgs& a, float* const Enew[3
     else if (zc == 0)
         hipLaunchKernelGGL((kFieldAfter<PIC_SOLVER_YEE, OPEN>), dim3(tiles), dim3(256), 0, s, a, Enew[0], Enew[1],
                            Enew[2]);
+    else if (divideInAfter(a.g))
+        hipLaunchKernelGGL((kYeeAfter<OPEN, true>), dim3(zt), dim3(256), 0, s, a, Enew[0], Enew[1], Enew[2], zc);
     else
-        hipLaunchKernelGGL(kYeeAfter<OPEN>, dim3(zt), dim3(256), 0, s, a, Enew[0], Enew[1], Enew[2], zc);
+        hipLaunchKernelGGL((kYeeAfter<OPEN, false>), dim3(zt), dim3(256), 0, s, a, Enew[0], Enew[1], Enew[2], zc);
     if (absorb) return launchAbsorb(a.g, a.B, *ab, s);
     return hipGetLastError();
 }

@@ -165,6 +165,39 @@ def test_one_launch_with_empty_supercells(shape, open_):
 
 
 @pytest.mark.parametrize("open_", [False, True], ids=["periodic", "open"])
+@pytest.mark.parametrize("grid", [(184, 200, 200), (200, 192, 200)], ids=["in-cache", "beyond-cache"])
+def test_large_field_step_equals_its_stages(grid, open_):
+    """The fused Yee field step of a large box, on both sides of the size from
+    which its second kernel divides in full, against the stage calls' kernels
+    (compared with the oracle on small grids), bit for bit; the last tile along
+    x is ragged."""
+    st = setups.thermal(grid=grid, ppc=1)
+    st.species[0].frames_per_sc = 1
+    if open_:
+        open_box(st)
+    print(f"case large field step grid={grid} open={open_}", flush=True)
+    assert (36 * st.ncells > 256 << 20) == (grid[0] == 200)
+    E, B = H.random_fields(st, 3, 1e-2, 1e-2)
+    J = H.random_fields(st, 4, 1e-2, 1e-2)[0]
+    out = []
+    for fused in (True, False):
+        sim = abi.Simulation(st.config())
+        for which, f in ((abi.FIELD_E, E), (abi.FIELD_B, B), (abi.FIELD_J, J)):
+            sim.load_field(which, f)
+        for _ in range(2):
+            if fused:
+                sim.fdtd_step()
+            else:
+                sim.update_before_current()
+                sim.add_current()
+                sim.update_after_current()
+        out.append((sim.read_field(abi.FIELD_E), sim.read_field(abi.FIELD_B)))
+        sim.close()
+    for nm, a, b in zip("EB", *out):
+        assert np.array_equal(H.bits(a), H.bits(b)), nm
+
+
+@pytest.mark.parametrize("open_", [False, True], ids=["periodic", "open"])
 def test_shift_bit_exact(open_):
     st = small_thermal(abi.SHAPE_CIC, abi.PUSHER_BORIS, u=0.3)
     if open_:

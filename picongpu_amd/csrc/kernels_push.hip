@@ -777,6 +777,10 @@ __device__ __forceinline__ CoverAxis coverAxis(int s, int nsc, bool open, const 
     return a;
 }
 
+// pointers that come from a table in memory are generic to the compiler, and a
+// flat load waits with the scalar and LDS operations: global memory stated
+typedef const __attribute__((address_space(1))) float* GlobalFloats;
+
 // Component C of one supercell's 256 J cells, a thread each: the values of
 // the at most 2 x 2 x 3 tiles that cover a cell, all loaded before the first
 // addition, then added as the flush adds them, in ascending checkerboard
@@ -785,7 +789,7 @@ __device__ __forceinline__ CoverAxis coverAxis(int s, int nsc, bool open, const 
 // ascending colour is ascending phase (every supercell covering a cell lies
 // in another phase). Bit k of `held` is 0 for a neighbour beyond an open
 // border and for one whose tile is not written.
-template <int SUPP, int C>
+template <int SUPP, int C, bool BATCH>
 __device__ __forceinline__ void gatherFlushComponent(const GridDev& g, const float* __restrict__ tiles,
                                                      const CoverAxis& ax, const CoverAxis& ay, const CoverAxis& az,
                                                      uint32_t held, float* __restrict__ J, size_t cell, bool fresh) {
@@ -797,22 +801,29 @@ __device__ __forceinline__ void gatherFlushComponent(const GridDev& g, const flo
     int const lx = tid & 7, ly = (tid >> 3) & 7, lz = tid >> 6;
     int const lane = (lz * EY + ly) * EX + lx;
     float w[27];
+    // batched: opaque, so that the tiles' addresses are formed per component
+    // (kept for all three they spilled 40 scalar registers; the plain kernel is
+    // faster with them). 32 boxes of 32 to 96 cells an axis, five steps: 39.0
+    // ms with them, 38.5 without, 38.3 before the tiles' words were read.
+    int nscx = g.nscx;
+    if (BATCH) asm volatile("" : "+s"(nscx));
 #pragma unroll
     for (int k = 0; k < 27; ++k) {
         int const a = k / 9, b = (k / 3) % 3, d = k % 3;
         int const ox = DLO - SCX * ax.step[d], oy = DLO - SCY * ay.step[b], oz = DLO - SCZ * az.step[a];
         w[k] = 0.0f;
-        int const sc = ax.sc[d] + g.nscx * (ay.sc[b] + g.nscy * az.sc[a]);
-        const float* const t = tiles + (ptrdiff_t)sc * J_ELEMS + TG::off(C) + (oz * EY + oy) * EX + ox;
+        int const sc = ax.sc[d] + nscx * (ay.sc[b] + g.nscy * az.sc[a]);
+        GlobalFloats const t = (GlobalFloats)tiles + (ptrdiff_t)sc * J_ELEMS + TG::off(C) + (oz * EY + oy) * EX + ox;
         // one predicate per load (no branch), so that the loads stay together
         bool const covers = ((unsigned)(lx + ox) < (unsigned)EX) & ((unsigned)(ly + oy) < (unsigned)EY) &
                             ((unsigned)(lz + oz) < (unsigned)EZ) & (((held >> k) & 1u) != 0u);
         if (covers) w[k] = t[lane];
     }
-    float v = fresh ? 0.0f : J[cell];
+    auto const j = (__attribute__((address_space(1))) float*)J + cell;
+    float v = fresh ? 0.0f : *j;
 #pragma unroll
     for (int k = 0; k < 27; ++k) v += w[k];
-    J[cell] = v;
+    *j = v;
 }
 
 // J of one supercell (256 threads). fresh: J holds nothing yet (the sums
@@ -823,7 +834,7 @@ __device__ __forceinline__ void gatherFlushComponent(const GridDev& g, const flo
 // empty box of 192x128x160 cells (TSC, 15,360 supercells) took 0.40 ms a step
 // in one launch and 0.28 by phases, now 0.25; a laser box of 96x512x64 cells,
 // four fifths vacuum, 8.76 and 7.59 ms for ten steps.
-template <int SUPP>
+template <int SUPP, bool BATCH>
 __device__ __forceinline__ void gatherFlushSC(const GridDev& g, const float* __restrict__ tiles,
                                               const uint32_t* __restrict__ tileHeld,
                                               const uint8_t* __restrict__ colour, float* J0, float* J1, float* J2,
@@ -844,9 +855,11 @@ __device__ __forceinline__ void gatherFlushSC(const GridDev& g, const float* __r
     }
     size_t const cell = (size_t)(sx * SCX + (tid & 7)) +
                         (size_t)g.nx * ((size_t)(sy * SCY + ((tid >> 3) & 7)) + (size_t)g.ny * (sz * SCZ + (tid >> 6)));
-    gatherFlushComponent<SUPP, 0>(g, tiles, ax, ay, az, held, J0, cell, fresh);
-    gatherFlushComponent<SUPP, 1>(g, tiles, ax, ay, az, held, J1, cell, fresh);
-    gatherFlushComponent<SUPP, 2>(g, tiles, ax, ay, az, held, J2, cell, fresh);
+    gatherFlushComponent<SUPP, 0, BATCH>(g, tiles, ax, ay, az, held, J0, cell, fresh);
+    if (BATCH) asm volatile("" : "+s"(held) : : "memory");
+    gatherFlushComponent<SUPP, 1, BATCH>(g, tiles, ax, ay, az, held, J1, cell, fresh);
+    if (BATCH) asm volatile("" : "+s"(held) : : "memory");
+    gatherFlushComponent<SUPP, 2, BATCH>(g, tiles, ax, ay, az, held, J2, cell, fresh);
 }
 
 template <int SUPP>
@@ -855,16 +868,17 @@ __global__ __launch_bounds__(SCV) void kGatherFlush(GridDev g, const float* __re
                                                      const uint8_t* __restrict__ colour, float* J0, float* J1,
                                                      float* J2, int fresh) {
     if (halted(g)) return;
-    gatherFlushSC<SUPP>(g, tiles, held, colour, J0, J1, J2, (int)blockIdx.x, fresh != 0);
+    gatherFlushSC<SUPP, false>(g, tiles, held, colour, J0, J1, J2, (int)blockIdx.x, fresh != 0);
 }
 
 template <int SUPP>
 __global__ __launch_bounds__(SCV) void kGatherFlushBatch(const GatherEntry* __restrict__ table,
                                                           const int2* __restrict__ blocks, int fresh) {
     int2 const it = blocks[blockIdx.x];
-    const GatherEntry& e = table[it.x];
+    GatherEntry const e = table[__builtin_amdgcn_readfirstlane(it.x)];
     if (halted(e.g)) return;
-    gatherFlushSC<SUPP>(e.g, e.tiles, e.held, e.colour, e.J[0], e.J[1], e.J[2], it.y, fresh != 0);
+    gatherFlushSC<SUPP, true>(e.g, e.tiles, e.held, e.colour, e.J[0], e.J[1], e.J[2], __builtin_amdgcn_readfirstlane(it.y),
+                        fresh != 0);
 }
 
 hipError_t launchGatherFlushBatch(int supp, const GatherEntry* table, const int2* blocks, int nblocks, bool fresh,

@@ -42,12 +42,12 @@ HBM_PEAK_GBS = 8000.0
 # workload, scaled by what the counters read for a 1 GiB device copy
 # (FETCH_SIZE reads 0.5 GiB for it: factor 2.0; WRITE_SIZE 1 GiB: factor 1.0).
 # The kernel's epilogue also stages the supercell shift (leaver records to
-# the outbox, compaction of the supercell), and the TSC kernels' spilled
-# registers go to scratch, so these bytes include both.
+# the outbox, compaction of the supercell), and the queued particles' state is
+# read again when they are deposited, so these bytes include both.
 # Command: rocprofv3 --pmc FETCH_SIZE (then WRITE_SIZE) -- python3 bench.py
 # --steps 1 --warmup 1 --no-cpu-baseline --no-adjoint --no-ensemble --calibrate-copy
 MEASURED_TRAFFIC = {
-    ("kelvin_helmholtz", (256, 256, 256)): {"fetch_kib": 1094990.0, "write_kib": 1084480.0, "fetch_scale": 2.0,
+    ("kelvin_helmholtz", (256, 256, 256)): {"fetch_kib": 1096250.0, "write_kib": 1084330.0, "fetch_scale": 2.0,
                                             "write_scale": 1.0},
 }
 # Instruction counters of the fused push/deposit kernel on this workload,
@@ -60,8 +60,8 @@ MEASURED_TRAFFIC = {
 # the push kernel that also damps the weightings in the layers
 # (kPushDepositPml).
 MEASURED_INSTS = {
-    ("kelvin_helmholtz", (256, 256, 256), "none"): {"valu": 708.50e6, "lds": 98.163e6, "lds_bank_conflict": 323.53e6,
-                                                    "grbm_gui_active": 25.764e6},
+    ("kelvin_helmholtz", (256, 256, 256), "none"): {"valu": 708.94e6, "lds": 98.262e6, "lds_bank_conflict": 323.53e6,
+                                                    "grbm_gui_active": 26.000e6},
     ("laser_plasma", (192, 1536, 192), "exponential"): {"valu": 375.31e6, "lds": 52.880e6,
                                                         "lds_bank_conflict": 134.53e6, "grbm_gui_active": 14.656e6},
     ("laser_plasma", (192, 1536, 192), "pml"): {"valu": 390.52e6, "lds": 52.857e6, "lds_bank_conflict": 134.46e6,

@@ -648,7 +648,7 @@ __device__ __forceinline__ void pushDepositSC(const PushArgs& a, int sc, unsigne
 // issue, both near 80 % of the launch. Before the aligned reads of the E/B
 // tile and the one-word queue the LDS was busy 86 % of it and the vector
 // units 73 %; on the 256^3 two-species shear flow a pass of five steps went
-// from 150.1 to 125.5 ms.
+// from 150.1 to 126 ms.
 // Waves per SIMD the register budget must allow. TSC and PQS: at most 128
 // VGPRs, two workgroups per CU. TSC at 80 VGPRs has room for three, but the
 // loop then spills (126 ms a pass against 133 to 142 with 80 VGPRs), and
@@ -676,7 +676,9 @@ __global__ __launch_bounds__(kPushThreads, SUPP == 2 ? 6 : 4) void kPushDepositP
 // memory (the table does not change while the kernel runs) at a uniform
 // index, so they come by scalar loads as a kernel's own arguments do; as
 // ordinary memory that stores might change they were held in vector
-// registers (240 bytes per lane spilled, one workgroup less per CU).
+// registers (240 bytes per lane spilled, one workgroup less per CU). The loop
+// over items still leaves 152 (CIC) to 300 bytes (PQS) per lane in scratch,
+// where the plain kernel has none.
 template <int SUPP, int PUSHER, int MODE, bool EMZ = false>
 __global__ __launch_bounds__(kPushThreads, SUPP == 2 ? 6 : 4) void kPushDepositBatch(const PushArgs* __restrict__ table,
                                                                   const int2* __restrict__ work, int nwork) {
